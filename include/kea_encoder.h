@@ -44,6 +44,17 @@ int kea_relpos_attention_ws(const float *qkv_dev, int64_t ld, const float *pos_d
                             int64_t batch, int64_t t, int heads, int head_dim, float scale, void *workspace_dev,
                             int64_t workspace_bytes, void *stream);
 
+/* The same attention at any length t (up to 65535 tiles of 64 frames), for every length with a workspace of
+ * kea_relpos_attention_tiled_workspace bytes (16-byte aligned, 0 for sizes the call refuses): a first launch splits Q, K,
+ * V and the positions into pairs of FP16 values of one power-of-two scale a row (exact to 2^-22), a second walks the keys
+ * in blocks with an online softmax on the FP16 matrix cores. Equal to kea_relpos_attention up to FP32 rounding. The
+ * workspace is written before it is read, so it needs no clearing and may be reused by the next call on the stream. */
+int64_t kea_relpos_attention_tiled_workspace(int64_t batch, int64_t t, int heads);
+int kea_relpos_attention_tiled(const float *qkv_dev, int64_t ld, const float *pos_dev, int64_t ldp,
+                               const float *bias_u_dev, const float *bias_v_dev, float *out_dev, int64_t ldo,
+                               int64_t batch, int64_t t, int heads, int head_dim, float scale, void *workspace_dev,
+                               int64_t workspace_bytes, void *stream);
+
 /* The P-part int8 quantization (as kea_quantize, f32 scales, no LayerNorm) of the attention output that a
  * kea_relpos_attention_ws call with out == NULL left as two halves in `workspace_dev`: bitwise what kea_quantize
  * gives on that call's merged out, without writing it. The same batch, t and heads as that call (the split must

@@ -1,0 +1,578 @@
+// Relative-position self-attention over sequences of any length for MI355X (gfx950): key blocks with an online softmax
+// on the FP16 matrix cores at FP32 accuracy.
+//
+//   s[i][j] = ((q_i + u) . k_j + (q_i + v) . p_{T-1-i+j}) * scale,  out_i = sum_j softmax_j(s)[i][j] v_j
+//
+// Arithmetic. The FP32 matrix instruction runs at 1/16 of the FP16 rate, so every operand is split into two FP16
+// values, x * 2^a = hi + lo, and a product takes three FP16 MFMAs with FP32 accumulation (hi hi + hi lo + lo hi; the
+// dropped lo lo term is 2^-22 of the product, of random sign). The power of two a is chosen per query row, per four
+// rows of K and P and per eight keys of V so that the largest value lies in [2^14, 2^15): hi + lo then holds every
+// element to 2^-22 of itself or 2^-39 of that largest value, whatever the input's range, and the scaling is exact.
+// Against FP64 the result is closer than the FP32 forms (fewer roundings of the accumulator). An infinity in the
+// inputs has no such scale: a workgroup that meets one recomputes its rows with plain FP32 dot products (NaNs
+// propagate by themselves).
+//
+// Two launches. split_kernel writes K, V and P once as hi / lo planes in the order the LDS of the second kernel holds
+// them, 64 rows to a block; relpos_tiled_kernel then copies blocks straight to LDS (global_load_lds) and spends no
+// vector instruction on them. (Splitting inside the attention kernel, every 64-query workgroup for itself, took a third
+// of its time: T = 750, batch 2 67 us against 58 for the two launches.)
+//
+// Layout of the work. A workgroup is 4 x 2 waves on 64 queries of one (clip, head); it walks the keys in blocks of 64,
+// wave (qg, ks) taking queries 16 qg .. and keys 32 ks .. of a block with its own online softmax; the two partial
+// results of a query group are merged through LDS at the end. Scores are formed transposed (D[key][query] = K Q^T), so
+// a lane owns one query, the row maximum is two cross-lane steps, and its eight probabilities of a 32-key step are
+// already the B operand of O^T = V^T P^T: the contraction order over keys is chosen to match (group g of a wave's
+// keys: 4 g + r of both 16-key tiles), and V is stored transposed in that order. The position scores of a wave are the
+// band of 47 relative rows its 16 x 32 tile needs (three 16-row tiles), read back along the diagonal from LDS. The
+// band of a workgroup is 127 rows, two blocks of P, which are cut so that every workgroup's band starts at a block:
+// each key block needs one new block of P. Rows are unpadded with XOR-swizzled 16-byte units, so 16 rows read at one
+// unit are conflict-free. K and the new P block are copied while the softmax and the P.V products run, V while the
+// next scores do.
+//
+// Bound by LDS reads (a 64-key block: 448 KB for the eight waves, 3500 of its 7400 cycles, measured; the MFMAs of two
+// waves on a SIMD take 2700) and the phases' barriers. Measured on MI355X, graph-timed, both launches, against what
+// served these lengths before (T <= 256 an FP32 vector kernel, above it PyTorch operators on [T, 2T] score matrices):
+// T = 200 batch 8 33 / 181 us, T = 250 batch 1 25 / 30, T = 375 batch 2 35 / 146, T = 750 batch 2 58 / 291, T = 750
+// batch 8 165 / 898. Up to 128 frames the FP32 matrix-core kernels of kea_encoder.hip, one pass without a workspace,
+// are the faster ones: T = 125 batch 8 21 against 24 us, batch 1 11 against 17; at T = 129 batch 1 it is 21 against 21.
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <string>
+#include <type_traits>
+
+#include "kea_internal.h"
+#include "kea_wave.h"
+#include "../../include/kea_encoder.h"
+
+namespace {
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+constexpr int kDK = 128;
+
+using kea::dpp;
+using kea::wave_max;
+using kea::wave_sum;
+
+// The binary exponent e of a magnitude given by its bits (2^e <= m < 2^(e+1)), clamped so that 2^(14-e) and 2^(e-14)
+// are normal numbers.
+__device__ __forceinline__ int exponent_of(int bits) { return min(max((bits >> 23) - 127, -90), 127); }
+// 2^e for e in [-127, 127] (2^-127 as zero).
+__device__ __forceinline__ float pow2(int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); }
+
+// x * sf (sf a power of two) as hi + lo: one mixed-precision fma for each half.
+__device__ __forceinline__ void split8(const float *x, float sf, v8h &hi, v8h &lo) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        hi[e] = (_Float16)__builtin_fmaf(x[e], sf, 0.f);
+        lo[e] = (_Float16)__builtin_fmaf(x[e], sf, -(float)hi[e]);
+    }
+}
+
+// The largest magnitude of N values. The three-operand maximum with magnitude modifiers is written out because fmaxf
+// costs a canonicalising instruction more per value. NaNs are passed over.
+template <int N>
+__device__ __forceinline__ float max_abs(const float *x) {
+    static_assert(N % 2 == 0, "pairs");
+    float m = 0.f;
+#pragma unroll
+    for (int e = 0; e < N; e += 2) asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(m) : "v"(x[e]), "v"(x[e + 1]), "v"(m));
+    return m;
+}
+// The bits of the largest of 64 non-negative values, wave-uniform (such floats order as their bits do).
+__device__ __forceinline__ int wave_max_bits(float m) {
+    m = fmaxf(m, dpp<0xB1>(m));
+    m = fmaxf(m, dpp<0x4E>(m));
+    m = fmaxf(m, dpp<0x141>(m));
+    m = fmaxf(m, dpp<0x140>(m));
+    const int v = __builtin_bit_cast(int, m);
+    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+constexpr int kInfBits = 0x7f800000;
+
+__device__ __forceinline__ v4f mfma(v8h a, v8h b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+
+
+constexpr int kQG = 4, kKS = 2;                 // query groups and key halves: one wave each
+constexpr int kNW = kQG * kKS, kRows = 64;      // rows of a block of K, V or P; queries of a workgroup
+static_assert(16 * kQG == kRows && 32 * kKS == kRows, "queries, keys and P rows advance by the same block");
+constexpr int kPlane = kRows * kDK;             // elements of one plane of a block
+constexpr int kBlockBytes = 2 * kPlane * 2;     // hi and lo planes
+constexpr int kBandStride = 52;                 // band scores of a query in LDS (floats): 47 used
+
+// The split operands in the workspace.
+//   K, V: block (b, h, kb), keys 64 kb ..;  P: block (h, pb), relative rows T - 64 + 64 (pb + 1 - tiles) ..: the two
+//   planes, in LDS order;  Q: block (b, h, tile): for both biases (u, v) the two planes of four 16-query groups as MFMA
+//   operands [s][lane][8] (lane: query lane % 16, elements 32 s + 8 (lane / 16) .. + 7).
+//   Multipliers 2^(e - 14): km, pm one for four rows, qm [bias][query]; ve: the exponents of the eight V groups.
+//   top: the bits of the largest magnitude, kt for K and V, pt for P, qt for Q.
+struct SplitOperands {
+    char *q, *k, *v, *p;
+    float *qm, *km, *pm;
+    int32_t *ve, *qt, *kt, *pt;
+    int tiles, pblocks;  // 64-row tiles of the sequence; blocks of P per head
+};
+constexpr int kQBlockBytes = 2 * kBlockBytes;
+inline long long split_layout(SplitOperands *s, char *ws, long long batch, int heads, long long t) {
+    const long long tiles = (t + kRows - 1) / kRows, kv = batch * heads * tiles, np = 2 * tiles * heads;
+    long long off = 0;
+    auto take = [&](auto &field, long long bytes) {
+        field = (std::remove_reference_t<decltype(field)>)(ws + off);
+        off += (bytes + 15) / 16 * 16;
+    };
+    take(s->q, kv * kQBlockBytes);
+    take(s->k, kv * kBlockBytes);
+    take(s->v, kv * kBlockBytes);
+    take(s->p, np * kBlockBytes);
+    take(s->qm, kv * 2 * kRows * 4);
+    take(s->km, kv * 16 * 4);
+    take(s->pm, np * 16 * 4);
+    take(s->ve, kv * 8 * 4);
+    take(s->qt, kv * 4);
+    take(s->kt, kv * 4);
+    take(s->pt, np * 4);
+    s->tiles = (int)tiles;
+    s->pblocks = (int)(2 * tiles);
+    return off;
+}
+
+// One workgroup (256 threads) splits one block: blockIdx.x < kv a block of K and V, then kv blocks of Q, then P. Bound by
+// the bytes: 4 read and 4 (Q: 8) written an element.
+__global__ void __launch_bounds__(256)
+split_kernel(const float *qkv, long long ld, const float *pos, long long ldp, const float *bias_u, const float *bias_v,
+             int T, int H, int kv, SplitOperands so) {
+    __shared__ __attribute__((aligned(16))) _Float16 vt[2 * kPlane];
+    __shared__ int top[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4;
+    int seen = 0;
+    // 64 rows of a [rows][stride] matrix from row `first` (zeros outside [0, count)): four rows a wave and step, 16
+    // lanes a row
+    auto rows = [&](const float *src, long long stride, int first, int count, _Float16 *dst, float *mul) {
+        float x[4][8];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int row = first + 16 * u + 4 * wave + g;
+            float4 a = make_float4(0.f, 0.f, 0.f, 0.f), d = a;
+            if (row >= 0 && row < count) {
+                const float *p = src + (long long)row * stride + 8 * n;
+                a = *(const float4 *)p;
+                d = *(const float4 *)(p + 4);
+            }
+            x[u][0] = a.x; x[u][1] = a.y; x[u][2] = a.z; x[u][3] = a.w; x[u][4] = d.x; x[u][5] = d.y; x[u][6] = d.z; x[u][7] = d.w;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int row = 16 * u + 4 * wave + g;
+            const int bits = wave_max_bits(max_abs<8>(x[u])), e = exponent_of(bits);
+            seen = max(seen, bits);
+            v8h hi, lo;
+            split8(x[u], pow2(14 - e), hi, lo);
+            _Float16 *p = dst + row * kDK + ((n ^ (row & 15)) * 8);
+            *(v8h *)p = hi;
+            *(v8h *)(p + kPlane) = lo;
+            if (lane == 0) mul[4 * u + wave] = pow2(e - 14);
+        }
+    };
+    auto finish = [&](int32_t *word) {  // the block's largest magnitude
+        if (lane == 0) top[wave] = seen;
+        __syncthreads();
+        if (tid == 0) *word = max(max(top[0], top[1]), max(top[2], top[3]));
+    };
+    if ((int)blockIdx.x >= 2 * kv) {
+        const int id = blockIdx.x - 2 * kv, h = id / so.pblocks, pb = id - h * so.pblocks;
+        rows(pos + (long long)h * kDK, ldp, T - kRows + kRows * (pb + 1 - so.tiles), 2 * T - 1,
+             (_Float16 *)(so.p + (long long)id * kBlockBytes), so.pm + (long long)id * 16);
+        finish(so.pt + id);
+        return;
+    }
+    const int id = (int)blockIdx.x < kv ? (int)blockIdx.x : (int)blockIdx.x - kv;
+    const int kb = id % so.tiles, bh = id / so.tiles, h = bh % H, b = bh / H, j0 = kb * kRows;
+    const float *qbase = qkv + (long long)b * T * ld + (long long)h * kDK;
+    if ((int)blockIdx.x >= kv) {  // queries: wave = 16-query group, a lane per query and quarter of each 32-element step
+        const int i = j0 + 16 * wave + n;
+        float x[2][4][8];
+        const float *q = qbase + (long long)min(i, T - 1) * ld + 8 * g;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int c = 0; c < 8; c += 4) {
+                const int at = h * kDK + 8 * g + 32 * s + c;
+                const float4 a = *(const float4 *)(q + 32 * s + c), u = *(const float4 *)(bias_u + at),
+                             v = *(const float4 *)(bias_v + at);
+                x[0][s][c] = a.x + u.x; x[0][s][c + 1] = a.y + u.y; x[0][s][c + 2] = a.z + u.z; x[0][s][c + 3] = a.w + u.w;
+                x[1][s][c] = a.x + v.x; x[1][s][c + 1] = a.y + v.y; x[1][s][c + 2] = a.z + v.z; x[1][s][c + 3] = a.w + v.w;
+            }
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            float m = max_abs<32>(&x[w][0][0]);
+            m = fmaxf(m, __shfl_xor(m, 16, 64));
+            m = fmaxf(m, __shfl_xor(m, 32, 64));
+            seen = max(seen, wave_max_bits(m));
+            const int e = exponent_of(__builtin_bit_cast(int, m));
+            if (g == 0) so.qm[((long long)id * 2 + w) * kRows + 16 * wave + n] = pow2(e - 14);
+            char *dst = so.q + (long long)id * kQBlockBytes + w * kBlockBytes + wave * 4096 + lane * 16;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                v8h hi, lo;
+                split8(x[w][s], pow2(14 - e), hi, lo);
+                *(v8h *)(dst + s * 1024) = hi;
+                *(v8h *)(dst + s * 1024 + kPlane * 2) = lo;
+            }
+        }
+        finish(so.qt + id);
+        return;
+    }
+    const float *kbase = qbase + (long long)H * kDK, *vbase = kbase + (long long)H * kDK;
+    float v[2][8][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int grp = 4 * u + wave;  // keys 32 (grp / 4) + 16 t + 4 (grp % 4) + r, t = 0, 1, r = 0..3
+            const int j = j0 + 32 * (grp >> 2) + 16 * (e >> 2) + 4 * (grp & 3) + (e & 3);
+            float2 w = make_float2(0.f, 0.f);
+            if (j < T) w = *(const float2 *)(vbase + (long long)j * ld + 2 * lane);
+            v[u][e][0] = w.x;
+            v[u][e][1] = w.y;
+        }
+    rows(kbase, ld, j0, T, (_Float16 *)(so.k + (long long)id * kBlockBytes), so.km + (long long)id * 16);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int grp = 4 * u + wave;
+        const int bits = wave_max_bits(max_abs<16>(&v[u][0][0])), e = exponent_of(bits);
+        seen = max(seen, bits);
+        if (lane == 0) so.ve[(long long)id * 8 + grp] = e;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            float x[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) x[k] = v[u][k][c];
+            v8h hi, lo;
+            split8(x, pow2(14 - e), hi, lo);
+            _Float16 *p = vt + (2 * lane + c) * kRows + ((grp ^ (lane & 7)) * 8);  // row d = 2 lane + c, unit ^ (d / 2 % 8)
+            *(v8h *)p = hi;
+            *(v8h *)(p + kPlane) = lo;
+        }
+    }
+    finish(so.kt + id);
+    v8h *dst = (v8h *)(so.v + (long long)id * kBlockBytes);
+#pragma unroll
+    for (int u = 0; u < 2 * kPlane / 8 / 256; ++u) dst[u * 256 + tid] = ((const v8h *)vt)[u * 256 + tid];
+}
+
+typedef __attribute__((address_space(1))) const void *gptr_t;
+typedef __attribute__((address_space(3))) void *lptr_t;
+
+// A block from the workspace to LDS, by all waves of the workgroup: four 16-byte copies a lane.
+__device__ __forceinline__ void copy_block(const char *src, char *dst, int wave, int lane) {
+#pragma unroll
+    for (int u = 0; u < kBlockBytes / (kNW * 1024); ++u) {
+        const int off = (u * kNW + wave) * 1024;
+        __builtin_amdgcn_global_load_lds((gptr_t)(src + off + lane * 16), (lptr_t)(dst + off), 16, 0, 0);
+    }
+}
+// Every copy (and load) of this wave has landed; then all waves' (no fence: only LDS copies and reads are ordered here).
+// The wait is the builtin so that the compiler counts it: after an inline one it waits again at the first use of a
+// loaded value, and with that for the copies issued since.
+__device__ __forceinline__ void landed_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+constexpr int kLdsK = 0, kLdsP = kLdsK + kBlockBytes, kLdsV = kLdsP + 2 * kBlockBytes, kLdsBand = kLdsV + kBlockBytes;
+constexpr int kLdsBad = kLdsBand + kNW * 16 * kBandStride * 4, kTiledLds = kLdsBad + 16;
+
+__global__ void __launch_bounds__(kNW * 64)
+relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long ldp, const float *bias_u,
+                    const float *bias_v, float *out, long long ldo, int T, int H, float scale, SplitOperands so) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4, qg = wave / kKS, ks = wave % kKS;
+    // blockIdx.x is the head: consecutive workgroups go to different XCDs, so one XCD's L2 serves a head's K, V and P
+    const int h = blockIdx.x, iq0 = blockIdx.y, b = blockIdx.z, tiles = so.tiles;
+    const long long bh = (long long)b * H + h;
+    const char *kblk = so.k + bh * tiles * kBlockBytes, *vblk = so.v + bh * tiles * kBlockBytes;
+    // the band starts at P block tiles - iq0 - 1; key block kb uses it and the next, advanced by kb
+    const long long pfirst = (long long)h * so.pblocks + tiles - iq0 - 1;
+    const char *pblk = so.p + pfirst * kBlockBytes;
+    _Float16 *const Kh = (_Float16 *)(lds + kLdsK), *const Ph = (_Float16 *)(lds + kLdsP), *const Vh = (_Float16 *)(lds + kLdsV);
+    float *const bd = (float *)(lds + kLdsBand) + wave * 16 * kBandStride;
+    int *const bad = (int *)(lds + kLdsBad);
+    if (tid == 0) *bad = 0;
+
+    copy_block(kblk, lds + kLdsK, wave, lane);
+    copy_block(pblk, lds + kLdsP, wave, lane);
+    copy_block(pblk + kBlockBytes, lds + kLdsP + kBlockBytes, wave, lane);
+    copy_block(vblk, lds + kLdsV, wave, lane);
+    // the wave's queries as MFMA operands; their multipliers with the softmax scale and the change to base 2
+    v8h qu[2][4], qv[2][4];
+    const char *qblk = so.q + (bh * tiles + iq0) * kQBlockBytes + qg * 4096 + lane * 16;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            qu[p][s] = *(const v8h *)(qblk + p * (kPlane * 2) + s * 1024);
+            qv[p][s] = *(const v8h *)(qblk + kBlockBytes + p * (kPlane * 2) + s * 1024);
+        }
+    const int iq = iq0 * kRows + 16 * qg + n;
+    const float *qm = so.qm + (bh * tiles + iq0) * 2 * kRows + 16 * qg + n;
+    const float mqu = qm[0] * (scale * 1.4426950408889634f), mqv = qm[kRows] * (scale * 1.4426950408889634f);
+    int seen = so.qt[bh * tiles + iq0];
+    for (int i = tid; i < tiles; i += kNW * 64)
+        seen = max(max(seen, so.kt[bh * tiles + i]), max(so.pt[pfirst + i], so.pt[pfirst + i + 1]));
+    if (seen >= kInfBits) *bad = 1;
+    // multipliers of the wave's band tiles (rows 48 - 16 qg + 32 ks + 16 t of the two blocks), keys and V groups
+    const int band0 = 48 - 16 * qg + 32 * ks;
+    const float *pmp = so.pm + pfirst * 16 + band0 / 4 + g, *kmp = so.km + bh * tiles * 16 + 8 * ks + g;
+    const int32_t *vep = so.ve + bh * tiles * 8 + 4 * ks;
+    float pmul[3], kmul[2];
+    int4 ev;
+    auto load_multipliers = [&](int kb) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) pmul[t] = pmp[kb * 16 + 4 * t];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) kmul[t] = kmp[kb * 16 + 4 * t];
+        ev = *(const int4 *)(vep + kb * 8);
+    };
+    load_multipliers(0);
+    landed_barrier();
+
+    // Online softmax in base 2 with a lazy reference: probabilities are 2^(s - m_ref) with m_ref raised (and the sums
+    // rescaled) only when a score passes it by more than 8, so most blocks accumulate in the MFMA. Probabilities then
+    // reach 2^8; they are split at 2^6 times the V group's scale relative to 2^em.
+    constexpr int kLazy = 8, kProbExp = 6;
+    float m_ref = -INFINITY, l_run = 0.f;  // l_run: this lane's keys only
+    // em follows the blocks' exponents up at once and down by more than 3, but no further than 60 below the largest seen
+    // (the sums would leave FP32's range)
+    int em = -1000, etop = -1000;
+    v4f o[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) o[d] = (v4f){0.f, 0.f, 0.f, 0.f};
+
+    for (int kb = 0; kb < tiles; ++kb) {
+        const int jw = kb * kRows + 32 * ks;  // this wave's first key
+        int pbase[3];  // element offset of each band tile in the two-block ring
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const int row = band0 + 16 * t;
+            pbase[t] = ((kb + row / kRows) & 1) * 2 * kPlane + (row % kRows + n) * kDK;
+        }
+        v4f sc[2], sp[3];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) sc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 3; ++t) sp[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+        if (jw < T) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int c = ((4 * s + g) ^ n) * 8;  // tiles start at multiples of 16 rows: row & 15 = n
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {
+                    const _Float16 *p = Ph + pbase[t] + c;
+                    const v8h hi = *(const v8h *)p, lo = *(const v8h *)(p + kPlane);
+                    sp[t] = mfma(lo, qv[0][s], sp[t]);
+                    sp[t] = mfma(hi, qv[1][s], sp[t]);
+                    sp[t] = mfma(hi, qv[0][s], sp[t]);
+                }
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const _Float16 *p = Kh + (32 * ks + 16 * t + n) * kDK + c;
+                    const v8h hi = *(const v8h *)p, lo = *(const v8h *)(p + kPlane);
+                    sc[t] = mfma(lo, qu[0][s], sc[t]);
+                    sc[t] = mfma(hi, qu[1][s], sc[t]);
+                    sc[t] = mfma(hi, qu[0][s], sc[t]);
+                }
+            }
+            // the band scores of query n at relative positions 16 t + 4 g + r; key jj of the wave is position jj + 15 - n.
+            // Stored before the next copies go out: the compiler lets an LDS store wait for every copy in flight.
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                const float mul = pmul[t] * mqv;
+                *(float4 *)(bd + n * kBandStride + 16 * t + 4 * g) =
+                    make_float4(sp[t][0] * mul, sp[t][1] * mul, sp[t][2] * mul, sp[t][3] * mul);
+            }
+        }
+        landed_barrier();  // K and the older P block are free; V has landed
+        if (kb + 1 < tiles) {
+            copy_block(kblk + (long long)(kb + 1) * kBlockBytes, lds + kLdsK, wave, lane);
+            copy_block(pblk + (long long)(kb + 2) * kBlockBytes, lds + kLdsP + (kb & 1) * kBlockBytes, wave, lane);
+        }
+        if (jw < T) {
+            float p[8], mx = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const float mul = kmul[t] * mqu;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    p[4 * t + r] = __builtin_fmaf(sc[t][r], mul, bd[n * kBandStride + 15 - n + 16 * t + 4 * g + r]);
+            }
+            if (jw + 32 > T) {  // the last keys' tile
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (jw + 16 * (e >> 2) + 4 * g + (e & 3) >= T) p[e] = -INFINITY;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mx = fmaxf(mx, p[e]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const int eb = __builtin_amdgcn_readfirstlane(max(max(ev.x, ev.y), max(ev.z, ev.w)));
+            etop = max(etop, eb);
+            const int en = eb > em || eb < em - 3 ? max(eb, etop - 60) : em;
+            if (__any(mx > m_ref + kLazy) || en != em) {
+                const float m_new = fmaxf(m_ref, mx), a = __builtin_amdgcn_exp2f(m_ref - m_new);
+                const float f = a * pow2(max(min(em - en, 127), -127));
+                l_run = l_run * a;
+                m_ref = m_new;
+                em = en;
+#pragma unroll
+                for (int d = 0; d < 8; ++d)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[d][r] = o[d][r] * f;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                p[e] = __builtin_amdgcn_exp2f(p[e] - m_ref);
+                l_run = l_run + p[e];
+            }
+            const int eg = g == 0 ? ev.x : g == 1 ? ev.y : g == 2 ? ev.z : ev.w;
+            v8h ph, pl;
+            split8(p, pow2(max(eg - em + kProbExp, -127)), ph, pl);
+#pragma unroll
+            for (int d = 0; d < 8; ++d) {
+                const _Float16 *vp = Vh + (16 * d + n) * kRows + (((4 * ks + g) ^ (n >> 1)) * 8);
+                const v8h hi = *(const v8h *)vp, lo = *(const v8h *)(vp + kPlane);
+                o[d] = mfma(lo, ph, o[d]);
+                o[d] = mfma(hi, pl, o[d]);
+                o[d] = mfma(hi, ph, o[d]);
+            }
+        }
+        if (kb + 1 < tiles) load_multipliers(kb + 1);
+        landed_barrier();  // V is free; the next K and P have landed
+        if (kb + 1 < tiles) copy_block(vblk + (long long)(kb + 1) * kBlockBytes, lds + kLdsV, wave, lane);
+    }
+    l_run = l_run + __shfl_xor(l_run, 16, 64);
+    l_run = l_run + __shfl_xor(l_run, 32, 64);
+    {
+        const float f = pow2(max(em - 14 - kProbExp, -127));  // (a wave without keys: o = 0)
+#pragma unroll
+        for (int d = 0; d < 8; ++d)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[d][r] = o[d][r] * f;
+    }
+
+    // the two partial results of a query group meet in wave ks = 0
+    constexpr int kLane = 36;  // floats per lane: 32 outputs, m, l
+    float *const mb = (float *)lds + (qg * 64 + lane) * kLane;
+    if (ks > 0) {
+#pragma unroll
+        for (int d = 0; d < 8; ++d) *(float4 *)(mb + 4 * d) = make_float4(o[d][0], o[d][1], o[d][2], o[d][3]);
+        mb[32] = m_ref;
+        mb[33] = l_run;
+    }
+    __syncthreads();
+    if (*bad) {
+        // an infinity among the inputs: plain FP32, a wave per query row, keys over the lanes
+        for (int qi = wave; qi < kRows; qi += kNW) {
+            const int i = iq0 * kRows + qi;
+            if (i >= T) break;
+            const float *qbase = qkv + (long long)b * T * ld + (long long)h * kDK, *kbase = qbase + (long long)H * kDK;
+            const float *vbase = kbase + (long long)H * kDK, *pbase = pos + (long long)h * kDK;
+            const float *q = qbase + (long long)i * ld, *u = bias_u + h * kDK, *v = bias_v + h * kDK;
+            auto score = [&](int j) {
+                const float *k = kbase + (long long)j * ld, *p = pbase + (long long)(T - 1 - i + j) * ldp;
+                float c = 0.f, r = 0.f;
+                for (int d = 0; d < kDK; ++d) {
+                    c = __builtin_fmaf(q[d] + u[d], k[d], c);
+                    r = __builtin_fmaf(q[d] + v[d], p[d], r);
+                }
+                return (c + r) * scale;
+            };
+            float m = -INFINITY, l = 0.f, o0 = 0.f, o1 = 0.f;
+            for (int j = lane; j < T; j += 64) m = fmaxf(m, score(j));
+            m = wave_max(m);
+            for (int j0 = 0; j0 < T; j0 += 64) {
+                const float p = j0 + lane < T ? expf(score(j0 + lane) - m) : 0.f;
+                l = l + p;
+                for (int jj = 0; jj < min(64, T - j0); ++jj) {
+                    const float pj = __shfl(p, jj, 64);
+                    const float2 vv = *(const float2 *)(vbase + (long long)(j0 + jj) * ld + 2 * lane);
+                    o0 = __builtin_fmaf(pj, vv.x, o0);
+                    o1 = __builtin_fmaf(pj, vv.y, o1);
+                }
+            }
+            l = wave_sum(l);
+            *(float2 *)(out + ((long long)b * T + i) * ldo + (long long)h * kDK + 2 * lane) = make_float2(o0 / l, o1 / l);
+        }
+        return;
+    }
+    if (ks > 0) return;
+    const float m1 = mb[32], mm = fmaxf(m_ref, m1);
+    const float a0 = __builtin_amdgcn_exp2f(m_ref - mm), a1 = __builtin_amdgcn_exp2f(m1 - mm);
+    const float inv = 1.0f / __builtin_fmaf(mb[33], a1, l_run * a0), f0 = a0 * inv, f1 = a1 * inv;
+    if (iq < T) {
+        float *dst = out + ((long long)b * T + iq) * ldo + (long long)h * kDK + 4 * g;
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
+            const float4 w = *(const float4 *)(mb + 4 * d);
+            *(float4 *)(dst + 16 * d) =
+                make_float4(__builtin_fmaf(w.x, f1, o[d][0] * f0), __builtin_fmaf(w.y, f1, o[d][1] * f0),
+                            __builtin_fmaf(w.z, f1, o[d][2] * f0), __builtin_fmaf(w.w, f1, o[d][3] * f0));
+        }
+    }
+}
+
+int64_t tiled_workspace(int64_t batch, int64_t t, int heads) {
+    SplitOperands so;
+    return split_layout(&so, nullptr, batch, heads, t);
+}
+
+// The largest sequence: 65535 query tiles of a launch.
+constexpr int64_t kMaxRows = 65535 * kRows;
+
+}  // namespace
+
+extern "C" int64_t kea_relpos_attention_tiled_workspace(int64_t batch, int64_t t, int heads) {
+    if (batch < 1 || t < 1 || heads < 1 || t > kMaxRows) return 0;
+    return tiled_workspace(batch, t, heads);
+}
+
+extern "C" int kea_relpos_attention_tiled(const float *qkv, int64_t ld, const float *pos, int64_t ldp,
+                                          const float *bias_u, const float *bias_v, float *out, int64_t ldo,
+                                          int64_t batch, int64_t t, int heads, int head_dim, float scale,
+                                          void *workspace, int64_t workspace_bytes, void *stream) {
+    if (batch < 0 || t < 1 || heads < 1 || head_dim != kDK || batch > 65535 || heads > 65535 || t > kMaxRows)
+        return kea::fail(KEA_EINVAL, "bad sizes (head_dim must be 128)");
+    if (batch == 0) return KEA_OK;
+    if (!qkv || !pos || !bias_u || !bias_v || !out) return kea::fail(KEA_EINVAL, "null pointer");
+    if (ld < 3LL * heads * head_dim || ldp < (int64_t)heads * head_dim || ldo < (int64_t)heads * head_dim)
+        return kea::fail(KEA_EINVAL, "leading dimension too small");
+    if (((uintptr_t)qkv | (uintptr_t)pos | (uintptr_t)out | (uintptr_t)bias_u | (uintptr_t)bias_v) & 15 ||
+        (ld | ldp | ldo) & 3)
+        return kea::fail(KEA_EALIGN, "qkv, pos, out and the biases need 16-byte aligned rows");
+    const int64_t need = tiled_workspace(batch, t, heads);
+    if (!workspace || workspace_bytes < need)
+        return kea::fail(KEA_ESPACE, "attention workspace too small: need " + std::to_string(need) + " bytes");
+    if ((uintptr_t)workspace & 15) return kea::fail(KEA_EALIGN, "attention workspace must be 16-byte aligned");
+    SplitOperands so;
+    split_layout(&so, (char *)workspace, batch, heads, t);
+    const int64_t kv = batch * heads * so.tiles, blocks = 2 * kv + (int64_t)heads * so.pblocks;
+    if (!kea::fits_dispatch(blocks, 256)) return kea::fail(KEA_EINVAL, "too large for one launch: split the batch");
+    hipError_t e = hipFuncSetAttribute((const void *)relpos_tiled_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kTiledLds);
+    if (e != hipSuccess) return kea::fail((int)e, std::string("LDS attribute refused: ") + hipGetErrorString(e));
+    hipLaunchKernelGGL(split_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, qkv, (long long)ld, pos,
+                       (long long)ldp, bias_u, bias_v, (int)t, heads, (int)kv, so);
+    e = hipGetLastError();
+    if (e != hipSuccess) return kea::fail((int)e, std::string("attention split launch failed: ") + hipGetErrorString(e));
+    hipLaunchKernelGGL(relpos_tiled_kernel, dim3((unsigned)heads, (unsigned)so.tiles, (unsigned)batch), dim3(kNW * 64),
+                       kTiledLds, (hipStream_t)stream, qkv, (long long)ld, pos, (long long)ldp, bias_u, bias_v, out,
+                       (long long)ldo, (int)t, heads, scale, so);
+    e = hipGetLastError();
+    if (e != hipSuccess) return kea::fail((int)e, std::string("attention launch failed: ") + hipGetErrorString(e));
+    return KEA_OK;
+}

@@ -5,7 +5,7 @@
 // (kk/ternary/fused_kernels.py:163-240) and `_glu_pad` + the depthwise Conv1d of the patched convolution module
 // (kk/ternary/layer_fusions4.py:10-30, :62-72). Arithmetic is IEEE FP32 (fused multiply-adds in the dot products);
 // unlike the reference's online-softmax tiles, a workgroup holds whole score rows (T <= 256), so the softmax is the
-// exact two-pass form.
+// exact two-pass form. Longer sequences, and callers with a workspace above 128 frames, run kea_attention.hip.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

@@ -291,6 +291,9 @@ def relpos_attention(qkv: Tensor, pos: Tensor, bias_u: Tensor, bias_v: Tensor, h
     _f32("bias_v", bias_v, qkv.device, d)
     args = (qkv.data_ptr(), qkv.stride(1), pos.data_ptr(), pos.stride(0), bias_u.data_ptr(), bias_v.data_ptr(),
             _hip.ptr(out), d, b, t, heads, d // heads, 1.0 / math.sqrt(d // heads))
+    if workspace is None and 128 < t <= 256:
+        # the tiled kernel (batch 8, T = 200: 33 us against 181); up to 128 frames the FP32 kernels are faster
+        return _attention_tiled(args, out)
     if workspace is None:
         rc = _hip.lib().kea_relpos_attention(*args, _hip.stream_handle(qkv.device))
     else:
@@ -298,6 +301,47 @@ def relpos_attention(qkv: Tensor, pos: Tensor, bias_u: Tensor, bias_v: Tensor, h
                                                 _hip.stream_handle(qkv.device))
     _hip.check(rc, "kea_relpos_attention")
     return out
+
+
+def _attention_tiled(args: tuple, out: Tensor) -> Tensor:
+    """kea_relpos_attention_tiled of checked arguments with a workspace of its own (stream ordered: torch's allocator
+    may hand it out again once the launches are enqueued)."""
+    L = _hip.lib()
+    batch, t, heads = args[8], args[9], args[10]
+    need = L.kea_relpos_attention_tiled_workspace(batch, t, heads)
+    ws = torch.empty(need, dtype=torch.uint8, device=out.device)
+    _hip.check(L.kea_relpos_attention_tiled(*args, ws.data_ptr(), need, _hip.stream_handle(out.device)),
+               "kea_relpos_attention_tiled")
+    return out
+
+
+def _plain_f32(t: Tensor, device) -> bool:
+    """Whether a kernel may read `t` in place of PyTorch operators: an ordinary FP32 tensor on the GPU `device`, 16-byte
+    aligned, that nothing records or transforms (autograd, vmap; see _traced)."""
+    return (type(t) in (Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.device == device
+            and t.layout == torch.strided and not (t.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t) and not t.is_neg() and t.data_ptr() % 16 == 0)
+
+
+def _traced() -> bool:
+    """Whether PyTorch operators called now are recorded or differentiated forward rather than only run."""
+    return (torch.autograd.forward_ad._current_level >= 0 or torch.jit.is_tracing() or torch.compiler.is_compiling()
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0)
+
+
+def _takes_tiled(qkv: Tensor, pos: Tensor, u: Tensor, v_bias: Tensor, heads: int) -> bool:
+    """Whether attention() of these tensors, longer than the FP32 kernels take, can run on the tiled kernel: what the
+    PyTorch form accepts beyond that (other types, strides and alignments, gradients, tracing) stays on it."""
+    if _traced() or qkv.dim() != 3 or qkv.device.type != "cuda":
+        return False
+    b, t, three_d = qkv.shape
+    d = heads * 128
+    return (b > 0 and three_d == 3 * d and tuple(pos.shape) == (2 * t - 1, d) and u.shape == v_bias.shape == (heads, 128)
+            and all(_plain_f32(x, qkv.device) for x in (qkv, pos, u, v_bias))
+            and u.is_contiguous() and v_bias.is_contiguous()
+            and qkv.stride(2) == 1 and qkv.stride(0) == t * qkv.stride(1) and qkv.stride(1) >= three_d
+            and pos.stride(1) == 1 and pos.stride(0) >= d and qkv.stride(1) % 4 == 0 and pos.stride(0) % 4 == 0
+            and 0 < _hip.lib().kea_relpos_attention_tiled_workspace(b, t, heads) and b <= 65535)
 
 
 def attention_merge_quantize(workspace: Tensor, batch: int, t: int, heads: int, parts: int) -> tuple[Tensor, Tensor]:
@@ -635,6 +679,10 @@ class FastConformerEncoder:
         dk = self.cfg.d_model // h
         if self.fused and t <= 256 and dk == 128:
             return relpos_attention(qkv, pos, u, v_bias, h, workspace=self._attention_ws(b, t))
+        if self.fused and dk == 128 and _takes_tiled(qkv, pos, u, v_bias, h):
+            out = torch.empty(b, t, h * dk, device=qkv.device, dtype=torch.float32)
+            return _attention_tiled((qkv.data_ptr(), qkv.stride(1), pos.data_ptr(), pos.stride(0), u.data_ptr(),
+                                     v_bias.data_ptr(), out.data_ptr(), h * dk, b, t, h, dk, 1.0 / math.sqrt(dk)), out)
         pos_t = pos.view(2 * t - 1, h, dk).permute(1, 2, 0).contiguous()  # [H, dk, 2t-1]
         q, k, v = qkv.view(b, t, 3, h, dk).unbind(2)
         qu = (q + u).transpose(1, 2).contiguous()                                   # [B, H, T, dk]

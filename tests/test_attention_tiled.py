@@ -1,0 +1,184 @@
+"""The tiled relative-position attention (kea_relpos_attention_tiled) and the calls that reach it: relpos_attention at
+129 .. 256 frames and FastConformerEncoder.attention above 256.
+
+Tolerance: a score is two 128-term dot products in FP32 (rounding 2^-24 a step, each operand held to 2^-22 and better),
+so it is off by at most about 128 * 2^-23 of the sum of its terms' magnitudes; measured errors are 3e-7 of the output's
+largest value, and 2e-6 is the bar of the FP32 kernels."""
+from __future__ import annotations
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+from kea_kernels import _hip, encoder as E
+
+H, DK = 8, 128
+D = H * DK
+
+
+def _inputs(b, t, seed, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(b, t, 3 * D, generator=g) * scale, torch.randn(2 * t - 1, D, generator=g),
+            torch.randn(H, DK, generator=g) * 0.1, torch.randn(H, DK, generator=g) * 0.1)
+
+
+def _reference(qkv, pos, u, v):
+    """The definition in FP64: s = ((q + u) k + (q + v) p_{T-1-i+j}) / sqrt(dk), softmax, P V."""
+    b, t, _ = qkv.shape
+    q, k, vv = (x.transpose(1, 2) for x in qkv.double().view(b, t, 3, H, DK).unbind(2))
+    p = pos.double().view(2 * t - 1, H, DK).permute(1, 2, 0)
+    i = torch.arange(t)
+    band = ((q + v.double()[:, None]) @ p).gather(3, (t - 1 - i[:, None] + i[None]).expand(b, H, t, t))
+    a = torch.softmax(((q + u.double()[:, None]) @ k.transpose(2, 3) + band) / math.sqrt(DK), -1)
+    return (a @ vv).transpose(1, 2).reshape(b, t, D)
+
+
+def _tiled(qkv, pos, u, v, ld=3 * D, ldo=D):
+    """The C entry on device tensors, into a poisoned output and workspace."""
+    L, (b, t, _) = _hip.lib(), qkv.shape
+    out = torch.full((b, t, ldo), 7.0, device="cuda")
+    need = L.kea_relpos_attention_tiled_workspace(b, t, H)
+    ws = torch.full((need,), 255, dtype=torch.uint8, device="cuda")
+    _hip.check(L.kea_relpos_attention_tiled(qkv.data_ptr(), ld, pos.data_ptr(), pos.stride(0), u.data_ptr(),
+                                            v.data_ptr(), out.data_ptr(), ldo, b, t, H, DK, 1 / math.sqrt(DK),
+                                            ws.data_ptr(), need, _hip.stream_handle(out.device)), "tiled")
+    return out.cpu()
+
+
+def _close(got, ref, tol=2e-6):
+    assert torch.isfinite(got).all()
+    assert float((got.double() - ref).abs().max() / ref.abs().max()) < tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,t", [(1, 1), (2, 15), (1, 32), (2, 63), (1, 64), (3, 65), (1, 97), (1, 128), (2, 129),
+                                 (1, 191), (1, 192), (1, 193), (1, 257), (2, 300), (1, 521), (1, 1000)])
+def test_every_tile_edge_matches_fp64(b, t):
+    x = _inputs(b, t, 31 * b + t)
+    _close(_tiled(*(a.cuda() for a in x)), _reference(*x))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale_v", [1e-30, 1e-6, 1e6, 1e30])
+def test_any_magnitude_of_values(scale_v):
+    """Values far outside FP16's range, and a key whose value row is 2^20 times the others'."""
+    qkv, pos, u, v = _inputs(1, 200, 5)
+    qkv[..., 2 * D:] *= scale_v
+    qkv[0, 70, 2 * D:] *= 2.0 ** 20
+    qkv[0, 70, D:2 * D] = 0.0
+    ref = _reference(qkv, pos, u, v)
+    _close(_tiled(*(a.cuda() for a in (qkv, pos, u, v))) / scale_v, ref / scale_v)
+
+
+@pytest.mark.gpu
+def test_large_scores_and_small_queries():
+    """Scores in the hundreds (a sharp softmax) hold the FP32 error of a score, 2^-24 of its terms; tiny queries give
+    the mean of the values."""
+    qkv, pos, u, v = _inputs(1, 150, 6)
+    qkv[..., :2 * D] *= 8.0
+    got, ref = _tiled(*(a.cuda() for a in (qkv, pos, u, v))), _reference(qkv, pos, u, v)
+    assert float((got.double() - ref).norm() / ref.norm()) < 1e-4
+    qkv[..., :D] = 0.0
+    u, v = u * 1e-30, v * 1e-30
+    _close(_tiled(*(a.cuda() for a in (qkv, pos, u, v))), _reference(qkv, pos, u, v))
+
+
+@pytest.mark.gpu
+def test_row_strides():
+    """Rows of a wider matrix: qkv with ld > 3 d, pos with ldp > d, out with ldo > d (columns past d untouched)."""
+    qkv, pos, u, v = _inputs(2, 140, 8)
+    wide = torch.randn(2, 140, 3 * D + 8)
+    wide[..., :3 * D] = qkv
+    widep = torch.randn(279, D + 4)
+    widep[:, :D] = pos
+    got = _tiled(wide.cuda(), widep.cuda()[:, :D], u.cuda(), v.cuda(), ld=3 * D + 8, ldo=D + 4)
+    _close(got[..., :D], _reference(qkv, pos, u, v))
+    assert bool((got[..., D:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", ["v_inf", "v_nan", "k_inf", "k_nan", "q_inf", "p_inf"])
+def test_non_finite_inputs_as_the_formula(where):
+    """An infinity or NaN reaches exactly the outputs the FP32 formula gives it to."""
+    qkv, pos, u, v = _inputs(2, 300, 9)
+    bad = math.inf if where.endswith("inf") else math.nan
+    part = {"q": 0, "k": D, "v": 2 * D}
+    if where[0] == "p":
+        pos[310, 130] = bad
+    else:
+        qkv[1, 200, part[where[0]] + 130] = bad
+    got = _tiled(*(a.cuda() for a in (qkv, pos, u, v)))
+    ref = _reference(qkv, pos, u, v).float()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
+    fine = torch.isfinite(ref)
+    assert float((got - ref)[fine].abs().max()) < 2e-6 * float(ref[fine].abs().max())
+
+
+@pytest.mark.gpu
+def test_layer_attention_routes(monkeypatch):
+    """FastConformerEncoder.attention above 256 frames: the tiled kernel for plain FP32 tensors, the PyTorch form for
+    what only it takes, the same values either way; relpos_attention still refuses more than 256 frames."""
+    model = E.FastConformerEncoder(E.synthetic_weights(E.EncoderConfig(layers=1)), E.EncoderConfig(layers=1))
+    x = _inputs(2, 270, 10)
+    qkv, pos, u, v = (a.cuda() for a in x)
+    calls = []
+    tiled = E._attention_tiled
+    monkeypatch.setattr(E, "_attention_tiled", lambda *a: calls.append(1) or tiled(*a))
+    ref = _reference(*x)
+    _close(model.attention(qkv, pos, u, v).cpu(), ref)
+    assert calls == [1]
+    wide = torch.cat([qkv, qkv], -1)
+    _close(model.attention(wide[..., :3 * D], pos, u, v).cpu(), ref)     # a row stride of 6 d
+    assert calls == [1, 1]
+    off = torch.cat([torch.zeros(2 * D + 1, device="cuda"), qkv.flatten()])[2 * D + 1:].view_as(qkv)
+    _close(model.attention(off, pos, u, v).cpu(), ref, 1e-5)                   # misaligned
+    _close(model.attention(qkv, pos.t().contiguous().t(), u, v).cpu(), ref, 1e-5)
+    g = qkv.clone().requires_grad_()
+    out = model.attention(g, pos, u, v)                                        # recorded by autograd
+    assert out.requires_grad
+    _close(out.detach().cpu(), ref, 1e-5)
+    with torch.no_grad():
+        _close(model.attention(g, pos, u, v).cpu(), ref)
+    assert calls == [1, 1, 1]
+    batched = torch.func.vmap(lambda q: model.attention(q, pos, u, v))(torch.stack([qkv, 2 * qkv]))
+    _close(batched[0].cpu(), ref, 1e-5)
+    with pytest.raises((ValueError, RuntimeError)):
+        model.attention(qkv.double(), pos, u, v)                               # mixed types: PyTorch refuses
+    assert calls == [1, 1, 1]
+    with pytest.raises(ValueError, match="256 frames"):
+        E.relpos_attention(qkv, pos, u, v, H)
+
+
+@pytest.mark.gpu
+def test_graph_replays_equal_eager():
+    """Captured with its workspace from the graph's pool; every replay equals the eager result on new inputs."""
+    qkv, pos, u, v = (a.cuda() for a in _inputs(1, 200, 11))
+    E.relpos_attention(qkv, pos, u, v, H)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        out = E.relpos_attention(qkv, pos, u, v, H)
+    for seed in range(3):
+        qkv.copy_(_inputs(1, 200, 20 + seed)[0].cuda())
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, E.relpos_attention(qkv, pos, u, v, H))
+
+
+def test_refusals_before_any_launch():
+    L = _hip.lib()
+    need = L.kea_relpos_attention_tiled_workspace(1, 300, 8)
+    assert need > 0 and need % 16 == 0
+    assert L.kea_relpos_attention_tiled_workspace(0, 300, 8) == 0 == L.kea_relpos_attention_tiled_workspace(1, 0, 8)
+    assert L.kea_relpos_attention_tiled_workspace(1, 65535 * 64 + 1, 1) == 0
+    q = ctypes.c_void_p(0x1000)
+
+    def call(x=q, ld=3072, ldp=1024, ldo=1024, t=300, dk=128, ws=q, nbytes=need):
+        return L.kea_relpos_attention_tiled(x, ld, q, ldp, q, q, q, ldo, 1, t, 8, dk, 1.0, ws, nbytes, None)
+
+    assert call(dk=64) == -1 and call(t=0) == -1 and call(ld=3068) == -1 and call(ldp=1020) == -1 and call(x=None) == -1
+    assert call(x=ctypes.c_void_p(0x1004)) == -2 and call(ldo=1026) == -2 and call(ws=ctypes.c_void_p(0x1008)) == -2
+    assert call(nbytes=need - 1) == -4 and call(ws=None) == -4
+    assert L.kea_relpos_attention_tiled(q, 3072, q, 1024, q, q, q, 1024, 0, 300, 8, 128, 1.0, q, need, None) == 0
