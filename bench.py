@@ -583,7 +583,7 @@ def suite() -> None:
 # the chooser's shapes: BASELINE configs 1-4 and the encoder's linears (N, K) at M from single tokens to batch 8 of
 # 125 frames, the reference's tuned M points among them (kk/binary/configs.py:17-36)
 SWEEP_SHAPES = [(4096, 1024), (1024, 4096), (3072, 1024), (1024, 1024), (2048, 1024), (2560, 640), (1030, 640)]
-SWEEP_M = (1, 16, 38, 64, 126, 256, 368, 512, 1000)
+SWEEP_M = (1, 16, 38, 64, 126, 256, 368, 512, 1000, 2000, 4000, 16000)
 
 
 def sweep(parts_list=(1, 2, 3), wbits_list=(1, 2)) -> None:
@@ -619,9 +619,10 @@ def sweep(parts_list=(1, 2, 3), wbits_list=(1, 2)) -> None:
                                                    config=kernels.GemmConfig(tile, 0))
                         except ValueError:
                             continue  # the tile does not fit this part count / K
-                        graph = capture(stream, lambda i: plan(), 100)
+                        launches = 100 if m <= 1000 else 10
+                        graph = capture(stream, lambda i: plan(), launches)
                         replay_timed(stream, [graph])
-                        row[f"t{tile}"] = round(replay_timed(stream, [graph], 3) * 1000 / 300, 3)
+                        row[f"t{tile}"] = round(replay_timed(stream, [graph], 3) * 1000 / (3 * launches), 3)
                         del graph, plan
                     print(json.dumps(row), flush=True)
 

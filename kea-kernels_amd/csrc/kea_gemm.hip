@@ -185,7 +185,7 @@ int group_tile(int wbits, int parts, long long k, int gq) {
     for (const char *name : order)
         for (int i = 0; i < kNumWsplitTiles; ++i)
             if (std::string(kWsplitTiles[i].name) == name && kea::wsplit_group_steps(wbits, parts, k, kWsplitTiles[i], gq))
-                return kNumTiles + 1 + i;
+                return kLeadTiles + 1 + i;
     return parts >= 2 ? 1 : 4;
 }
 
@@ -193,8 +193,8 @@ int group_tile(int wbits, int parts, long long k, int gq) {
 // by powers of two up to 8 slices and 256 workgroups (ternary, one part, K >= 4096: up to 128 workgroups, 512 after
 // the split); the split's second launch costs more than it saves otherwise.
 int choose_split(int wbits, int parts, long long m, long long n, long long k, int id) {
-    if (id > kNumTiles) return 1;  // wave-split tiles split K inside the workgroup; more only when K needs it
-    const Tile &t = kTiles[id - 1];
+    if (!is_ring(id)) return 1;  // wave-split tiles split K inside the workgroup; more only when K needs it
+    const Tile &t = kTiles[ring_index(id)];
     const long long bm = t.wm * t.rm * 16, bn = t.wn * t.rn * 16;
     const long long wgs = cdivl(m, bm) * cdivl(n, bn);
     const long long J = wbits == 1 ? cdivl(k, 128) : cdivl(k, 64);
@@ -221,7 +221,7 @@ int kea_config_count(void) { return kNumTiles + kNumWsplitTiles; }
 
 const char *kea_config_name(int config) {
     if (config < 1 || config > kNumTiles + kNumWsplitTiles) return "";
-    return config <= kNumTiles ? kTiles[config - 1].name : kWsplitTiles[config - kNumTiles - 1].name;
+    return is_ring(config) ? kTiles[ring_index(config)].name : kWsplitTiles[config - kLeadTiles - 1].name;
 }
 
 static int resolve(int wbits, int parts, int64_t m, int64_t n, int64_t k, int split_k, int config, int *tile,
@@ -233,19 +233,19 @@ static int resolve(int wbits, int parts, int64_t m, int64_t n, int64_t k, int sp
     if (config < 0 || config > kNumTiles + kNumWsplitTiles) return kea::fail(KEA_EINVAL, "unknown config id");
     if (split_k < 0) return kea::fail(KEA_EINVAL, "split_k must be >= 0");
     int id = config ? config : choose_tile(wbits, parts, m, n, k);
-    if (!config && id > kNumTiles) {
+    if (!config && !is_ring(id)) {
         // an automatic wave-split pick must fit its registers and LDS, run unsplit when K % 16 != 0, and honour a
         // requested split exactly (the K range of one of its workgroups is at least nw * 2 k-steps)
-        const WsplitTile &wt = kWsplitTiles[id - kNumTiles - 1];
+        const WsplitTile &wt = kWsplitTiles[id - kLeadTiles - 1];
         const long long ksteps = cdivl(k, 64), want = split_k > 1 ? split_k : 1;
         const int s = kea::wsplit_steps(wbits, cdivl(ksteps, want), wt.nw);
         const bool ok = s && kea::wsplit_fits(wbits, parts, wt, s) && (!(k & 15) || s * wt.nw * 64 >= k) &&
                         (split_k <= 1 || cdivl(ksteps, (long long)wt.nw * s) == split_k);
         if (!ok) id = ring_tile(parts, m, n);
     }
-    if (id > kNumTiles) {
+    if (!is_ring(id)) {
         // wave-split tile: a workgroup covers nw waves x s k-steps; the split is raised to what the K range needs
-        const WsplitTile &wt = kWsplitTiles[id - kNumTiles - 1];
+        const WsplitTile &wt = kWsplitTiles[id - kLeadTiles - 1];
         const long long ksteps = cdivl(k, 64);
         long long want = split_k ? split_k : choose_split(wbits, parts, m, n, k, id);
         if (k & 15) want = 1;  // byte-precise K masking runs unsplit
@@ -264,9 +264,9 @@ static int resolve(int wbits, int parts, int64_t m, int64_t n, int64_t k, int sp
         *qps = (int)per;
         return KEA_OK;
     }
-    const Tile &tl = kTiles[id - 1];
-    if (!tile_fits(wbits, parts, tl.rm, tl.rn, tl.wm, tl.wn, tl.pw))
-        return kea::fail(KEA_EINVAL, std::string("tile ") + kTiles[id - 1].name + " does not fit " +
+    const Tile &tl = kTiles[ring_index(id)];
+    if (!tile_fits(wbits, parts, tl.rm, tl.rn, tl.wm, tl.wn, tl.pw, tl.deep))
+        return kea::fail(KEA_EINVAL, std::string("tile ") + tl.name + " does not fit " +
                                          std::to_string(parts) + " activation parts");
     const long long J = wbits == 1 ? cdivl(k, 128) : cdivl(k, 64);
     const long long quads = cdivl(J, 4);
@@ -333,17 +333,17 @@ int gemm_prepare(int wbits, const int8_t *q, int64_t part_stride, int64_t ldq, i
     if (ws_group != 0) {
         if (ws_group != 64 && ws_group != 128 && ws_group != 256)
             return kea::fail(KEA_EINVAL, "ws_group must be 0 (per-channel scales), 64, 128 or 256");
-        if (config != 0 && config != 1 && config != 4 && config <= kNumTiles)
+        if (config != 0 && config != 1 && config != 4 && is_ring(config) && config <= kNumTiles + kNumWsplitTiles)
             return kea::fail(KEA_EINVAL, "per-group weight scales run tile configs 1 and 4 or a wave-split tile");
         if (split_k > 1) return kea::fail(KEA_EINVAL, "per-group weight scales run unsplit (split_k 0 or 1)");
         gq = (int)(ws_group / 64);
-        if (config > kNumTiles && config <= kNumTiles + kNumWsplitTiles &&
-            !kea::wsplit_group_steps(wbits, parts, k, kWsplitTiles[config - kNumTiles - 1], gq))
+        if (config > 0 && !is_ring(config) &&
+            !kea::wsplit_group_steps(wbits, parts, k, kWsplitTiles[config - kLeadTiles - 1], gq))
             return kea::fail(KEA_EINVAL, std::string("per-group weight scales on wave-split tile ") +
-                                             kWsplitTiles[config - kNumTiles - 1].name +
+                                             kWsplitTiles[config - kLeadTiles - 1].name +
                                              " need 16-row blocks, at most 64 columns and one workgroup covering K "
                                              "exactly (K = waves x 64 x 2..16, whole groups per wave)");
-        if (!config) config = choose_tile(wbits, parts, m, n, k) > kNumTiles ? group_tile(wbits, parts, k, gq)
+        if (!config) config = !is_ring(choose_tile(wbits, parts, m, n, k)) ? group_tile(wbits, parts, k, gq)
                                                                              : parts >= 2 ? 1 : 4;
         split_k = 1;
     }
@@ -413,15 +413,15 @@ int gemm_prepare(int wbits, const int8_t *q, int64_t part_stride, int64_t ldq, i
         ls->finish_grid = dim3((unsigned)cdivl(m * cdivl(n, 4), 256));
     }
 
-    if (tile > kNumTiles) {
-        const WsplitTile &wt = kWsplitTiles[tile - kNumTiles - 1];
+    if (!is_ring(tile)) {
+        const WsplitTile &wt = kWsplitTiles[tile - kLeadTiles - 1];
         if (!kea::fits_dispatch(cdivl(n, wt.nt * 16), wt.nw * 64))
             return kea::fail(KEA_EINVAL, "too large for one launch: split the call along N or M");
         if (gq) {
             const int gs = kea::wsplit_group_steps(wbits, parts, k, wt, gq);
             p.groups = (int)cdivl(k, ws_group);
             p.steps_per_slice = wt.nw * gs;
-            const hipError_t e = gs ? kea::wsplit_group_prepare(p, wbits, parts, tile - kNumTiles - 1, gq, gs, &ls->wl)
+            const hipError_t e = gs ? kea::wsplit_group_prepare(p, wbits, parts, tile - kLeadTiles - 1, gq, gs, &ls->wl)
                                     : hipErrorInvalidDeviceFunction;
             if (e != hipSuccess)
                 return kea::fail((int)e, std::string("no per-group wave-split kernel: ") + hipGetErrorString(e));
@@ -430,17 +430,17 @@ int gemm_prepare(int wbits, const int8_t *q, int64_t part_stride, int64_t ldq, i
             return KEA_OK;
         }
         p.steps_per_slice = qps;
-        const hipError_t e = kea::wsplit_prepare(p, wbits, parts, tile - kNumTiles - 1, qps / wt.nw, s, s > 1, &ls->wl);
+        const hipError_t e = kea::wsplit_prepare(p, wbits, parts, tile - kLeadTiles - 1, qps / wt.nw, s, s > 1, &ls->wl);
         if (e != hipSuccess) return kea::fail((int)e, std::string("no wave-split kernel: ") + hipGetErrorString(e));
         ls->wsplit = true;
         return KEA_OK;
     }
-    const Tile &t = kTiles[tile - 1];
+    const Tile &t = kTiles[ring_index(tile)];
     const int bm = t.wm * t.rm * 16, bn = t.wn * t.rn * 16;
     // Ring buffers actually used: a workgroup touches buffer s % NS for its stages s < nst, so with nst < NS only
     // the first nst buffers need LDS.
     const long long words_per_wg = std::min<long long>(4LL * qps, (long long)p.J);
-    const StageShape shape = stage_shape(wbits, parts, t.rm, t.rn, t.wm, t.wn, t.pw);
+    const StageShape shape = stage_shape(wbits, parts, t.rm, t.rn, t.wm, t.wn, t.pw, t.deep);
     const int nst = (int)cdivl(words_per_wg, shape.sw);
     int lds_bytes = std::min(shape.ns, nst) * shape.stage_bytes;
     if (gq) {
@@ -786,21 +786,21 @@ int kea_lowbit_gemm_slices(int wbits, const int8_t *q, int64_t part_stride, int6
     p.quads_per_slice = qps;
     p.slices = slices;
     p.slice_vec = (n % 4 == 0);
-    if (tile > kNumTiles) {
-        const WsplitTile &wt = kWsplitTiles[tile - kNumTiles - 1];
+    if (!is_ring(tile)) {
+        const WsplitTile &wt = kWsplitTiles[tile - kLeadTiles - 1];
         if (!kea::fits_dispatch(cdivl(n, wt.nt * 16), wt.nw * 64))
             return kea::fail(KEA_EINVAL, "too large for one launch: split the call along N");
         p.steps_per_slice = qps;
         WsplitLaunch wl;
-        hipError_t e = kea::wsplit_prepare(p, wbits, parts, tile - kNumTiles - 1, qps / wt.nw, s, true, &wl);
+        hipError_t e = kea::wsplit_prepare(p, wbits, parts, tile - kLeadTiles - 1, qps / wt.nw, s, true, &wl);
         if (e == hipSuccess) e = kea::wsplit_enqueue(wl, p, (hipStream_t)stream);
         if (e != hipSuccess) return kea::fail((int)e, std::string("slice launch failed: ") + hipGetErrorString(e));
         return KEA_OK;
     }
-    const Tile &t = kTiles[tile - 1];
+    const Tile &t = kTiles[ring_index(tile)];
     const int bm = t.wm * t.rm * 16, bn = t.wn * t.rn * 16;
     const long long words_per_wg = std::min<long long>(4LL * qps, (long long)p.J);
-    const StageShape shape = stage_shape(wbits, parts, t.rm, t.rn, t.wm, t.wn, t.pw);
+    const StageShape shape = stage_shape(wbits, parts, t.rm, t.rn, t.wm, t.wn, t.pw, t.deep);
     const int nst = (int)cdivl(words_per_wg, shape.sw);
     const int lds_bytes = std::min(shape.ns, nst) * shape.stage_bytes;
     if (!kea::fits_dispatch(cdivl(n, bn), (t.wm * t.wn + t.pw) * 64))

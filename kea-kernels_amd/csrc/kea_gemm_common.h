@@ -164,6 +164,19 @@ __device__ __forceinline__ void load_row_scales(const Params &p, int m, EpiOpera
     for (int c = 0; c < 3; ++c) e.s[c] = c < P ? load_scalar(p.qs, p.qs_dtype, c * p.qs_stride + mm) : 0.f;
 }
 
+// The aligned 32-bit word holding element i of an f32 or f16 vector (f16: the half is selected at conversion time by
+// raw_to_f32 with the same v and i). The word lies inside the 4-byte block of an in-bounds element, so it never
+// reaches past a page the vector touches.
+__device__ __forceinline__ uint32_t load_raw(const void *v, bool f16, uint32_t i) {
+    const char *a = (const char *)v + (f16 ? 2u * i : 4u * i);
+    return *(const uint32_t *)__builtin_align_down(a, 4);  // keeps the pointer's (global) address space
+}
+__device__ __forceinline__ float raw_to_f32(uint32_t raw, bool f16, const void *v, uint32_t i) {
+    const uint32_t hi = (uint32_t)(((uintptr_t)v >> 1) + i) & 1u;  // f16: which half of the word
+    const float h = (float)__builtin_bit_cast(_Float16, (uint16_t)(raw >> (hi * 16)));
+    return f16 ? h : __builtin_bit_cast(float, raw);
+}
+
 // A per-column vector of f32 or f16 values (per-channel scales, bias) read through a range-checked buffer
 // descriptor: its base is the vector's start aligned down to 4 bytes (`delta` bytes before it) and its extent ends at
 // the 4-byte word holding the last element, so a load past the vector's end returns zeros instead of touching memory
@@ -260,17 +273,12 @@ __device__ __forceinline__ void epilogue4(const Params &p, int m, int nb, const 
     }
 }
 
-// epilogue4 for an output without raw accumulators, of compile-time dtype DT, whose 4 columns are all inside N with a
-// vector-aligned y: the same values, one vector store at yrow + nb (yrow: the row's first element), no per-lane
-// selection. RES: the residual is applied (Params::res is set). SILU: 1 / 0 the SiLU is / is not applied (known at
-// compile time: a run-time flag makes the compiler evaluate the SiLU for every output and select), -1: as
-// Params::flags says. GLU: the two column pairs become two outputs at yrow + nb / 2 (no residual, no SiLU).
-template <int P, int DT, bool RES, bool SMALL, int SILU = -1, bool GLU = false>
-__device__ __forceinline__ void epilogue4_full(const Params &p, void *yrow, int nb, const int (*a)[4],
-                                               const EpiOperands &e) {
-    static_assert(!GLU || (!RES && SILU == 0), "the GLU output takes neither a residual nor the SiLU");
+// The values of 4 consecutive columns from exact accumulators, with the choices known at compile time (a run-time SiLU
+// flag makes the compiler evaluate the SiLU for every output and select). RES: the residual e.res is applied. SILU:
+// 1 / 0 the SiLU is / is not applied, -1: as Params::flags says. SMALL: the residual and the bias as Params say.
+template <int P, bool RES, bool SMALL, int SILU>
+__device__ __forceinline__ void epilogue4_values(const Params &p, const int (*a)[4], const EpiOperands &e, float (&v)[4]) {
     const int flags = SILU < 0 ? p.flags : SILU ? (p.flags | KEA_FLAG_SILU) : (p.flags & ~KEA_FLAG_SILU);
-    float v[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         int ar[3] = {a[0][r], P > 1 ? a[1][r] : 0, P > 2 ? a[2][r] : 0};
@@ -282,26 +290,42 @@ __device__ __forceinline__ void epilogue4_full(const Params &p, void *yrow, int 
             if constexpr (RES) v[r] = e.res[r] + v[r] * p.res_factor;
         }
     }
+}
+// Two FP32 values rounded to FP16 / BF16 as one word (see to_f16_bits for the empty asm).
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef __bf16 v2b __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+template <int DT>
+__device__ __forceinline__ uint32_t pack2(float x, float y) {
+    asm("" : "+v"(x), "+v"(y));
+    const v2f v = {x, y};
+    if constexpr (DT == KEA_F16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2h));
+    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2b));
+}
+// Four consecutive values in the output type (GLU: the two pairs' outputs) through `put`, which takes 4 to 16 bytes.
+template <int DT, bool GLU, class Put>
+__device__ __forceinline__ void put4_as(const float (&v)[4], Put put) {
     if constexpr (GLU) {
         const float u0 = glu_pair(v[0], v[1]), u1 = glu_pair(v[2], v[3]);
-        if constexpr (DT == KEA_F32) {
-            *(float2 *)((float *)yrow + nb / 2) = make_float2(u0, u1);
-        } else {
-            const uint32_t h0 = DT == KEA_F16 ? to_f16_bits(u0) : to_bf16_bits(u0);
-            const uint32_t h1 = DT == KEA_F16 ? to_f16_bits(u1) : to_bf16_bits(u1);
-            *(uint32_t *)((uint16_t *)yrow + nb / 2) = h0 | (h1 << 16);
-        }
+        if constexpr (DT == KEA_F32) put(__builtin_bit_cast(v2u, (v2f){u0, u1}));
+        else put(pack2<DT>(u0, u1));
     } else if constexpr (DT == KEA_F32) {
-        *(float4 *)((float *)yrow + nb) = make_float4(v[0], v[1], v[2], v[3]);
+        put(__builtin_bit_cast(v4u, (v4f){v[0], v[1], v[2], v[3]}));
     } else {
-        uint16_t h[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) h[r] = DT == KEA_F16 ? to_f16_bits(v[r]) : to_bf16_bits(v[r]);
-        uint2 packed;
-        packed.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
-        packed.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
-        *(uint2 *)((uint16_t *)yrow + nb) = packed;
+        put((v2u){pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])});
     }
+}
+// epilogue4 for an output without raw accumulators, of compile-time dtype DT, whose 4 columns are all inside N with a
+// vector-aligned y: the same values, one vector store, no per-lane selection.
+template <int P, int DT, bool RES, bool SMALL, int SILU = -1, bool GLU = false>
+__device__ __forceinline__ void epilogue4_full(const Params &p, void *yrow, int nb, const int (*a)[4],
+                                               const EpiOperands &e) {
+    static_assert(!GLU || (!RES && SILU == 0), "the GLU output takes neither a residual nor the SiLU");
+    float v[4];
+    epilogue4_values<P, RES, SMALL, SILU>(p, a, e, v);
+    char *dst = (char *)yrow + (GLU ? nb / 2 : nb) * (DT == KEA_F32 ? 4 : 2);
+    put4_as<DT, GLU>(v, [&](auto bits) { *(decltype(bits) *)dst = bits; });
 }
 
 // The per-group epilogue of 4 consecutive columns: r holds sum_g fma(comb_P(acc_g), alpha[n][g], .) from the main

@@ -9,6 +9,7 @@
 #include <type_traits>
 
 #include "kea_gemm_common.h"
+#include "kea_gemm_wsplit.h"
 
 namespace kea {
 
@@ -39,16 +40,20 @@ constexpr int kMaxStages = KEA_MAX_STAGES;
 #ifndef KEA_FULL_PRM
 #define KEA_FULL_PRM 2
 #endif
-__host__ __device__ constexpr StageShape stage_shape(int wbits, int parts, int rm, int rn, int wm, int wn, int pw = 0) {
+// Deep tiles: stages of 128 k, as many (up to 4) as half the budget holds, so that two workgroups share a CU.
+constexpr int kDeepStageK = 128, kDeepStages = 4;
+__host__ __device__ constexpr int stage_k(bool deep) { return deep ? kDeepStageK : KEA_STAGE_K; }
+__host__ __device__ constexpr StageShape stage_shape(int wbits, int parts, int rm, int rn, int wm, int wn, int pw = 0,
+                                                     bool deep = false) {
     const int nw = pw > 0 ? pw : wm * wn, bm = wm * rm * 16, bn = wn * rn * 16;  // nw: the waves issuing copies
-    const int sw = KEA_STAGE_K / (wbits == 1 ? 128 : 64);
-    const int a_units = parts * bm * (KEA_STAGE_K / 16);
+    const int sw = stage_k(deep) / (wbits == 1 ? 128 : 64);
+    const int a_units = parts * bm * (stage_k(deep) / 16);
     const int b_words = (bn / 16) * sw;
     const int stage = a_units * 16 + b_words * 256;
     const int copies = a_units / 64 / nw + b_words / nw;
-    int ns = kLdsBudget / stage;
+    int ns = (deep ? kLdsBudget / 2 : kLdsBudget) / stage;
     if (ns > 63 / copies + 1) ns = 63 / copies + 1;
-    if (ns > kMaxStages) ns = kMaxStages;
+    if (ns > (deep ? kDeepStages : kMaxStages)) ns = deep ? kDeepStages : kMaxStages;
     if (ns < 2) ns = 2;
     return StageShape{sw, stage, copies, ns};
 }
@@ -59,9 +64,11 @@ struct Tile {
     int rm, rn, wm, wn;
     const char *name;
     int pw = 0;
+    bool deep = false;
 };
 
-// Tile configurations (ids are 1-based in the ABI). Results are identical for every tile.
+// Tile configurations. In the ABI the first twelve are ids 1..12; the rest follow the wave-split tiles (kWsplitTiles,
+// ids 13 on; ring_index). Results are identical for every tile.
 constexpr Tile kTiles[] = {
     {1, 1, 1, 4, "16x64 w1x4 r1x1"},   // 1
     {2, 1, 1, 4, "32x64 w1x4 r2x1"},   // 2
@@ -75,18 +82,31 @@ constexpr Tile kTiles[] = {
     {2, 4, 2, 4, "64x256 w2x4 r2x4"},  // 10
     {4, 2, 2, 4, "128x128 w2x4 r4x2"}, // 11
     {1, 2, 2, 4, "32x128 w2x4 r1x2"},  // 12
+    // Deep tiles for thousands of rows. A wave's 4 or 8 column blocks read each activation fragment from LDS once
+    // (tile 11's two make LDS the bound: 32 RM cycles of it a k-step against 32 RM of MFMA), four short stages keep
+    // three in flight (with two of 256 k a stage's copies, 4000 cycles under load, took longer than its MFMAs, 2000), and
+    // two workgroups a CU overlap one's epilogue with the other's K loop.
+    {4, 8, 2, 2, "128x256 w2x2 r4x8 deep", 0, true},
+    {4, 4, 2, 2, "128x128 w2x2 r4x4 deep", 0, true},
+    {2, 4, 2, 2, "64x128 w2x2 r2x4 deep", 0, true},
 };
+constexpr int kLeadTiles = 12;  // the ids before the wave-split tiles
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
 // Register budget of a tile: accumulators plus double-buffered activation fragments (in 32-bit registers). Up to 8
 // waves per workgroup (two per SIMD) they may take 256 of a wave's 256; with more waves a SIMD holds three or four of
 // them in its 512 registers per lane, and the arrays must leave 64 of a wave's share to the rest of the kernel. Two
 // ring buffers of the tile's stage must fit the LDS a workgroup may allocate.
-constexpr bool tile_fits(int wbits, int parts, int rm, int rn, int wm, int wn, int pw = 0) {
-    const int waves = wm * wn + pw, per_simd = (waves + 3) / 4;
-    return parts * rm * rn * 4 + 2 * parts * rm * 4 <= (waves <= 8 ? 256 : 512 / per_simd - 64) &&
-           2 * stage_shape(wbits, parts, rm, rn, wm, wn, pw).stage_bytes <= kLdsBudget;
+__host__ __device__ constexpr int wave_registers(int waves) { return waves <= 8 ? 256 : 512 / ((waves + 3) / 4); }
+constexpr bool tile_fits(int wbits, int parts, int rm, int rn, int wm, int wn, int pw = 0, bool deep = false) {
+    const int waves = wm * wn + pw;
+    return parts * rm * rn * 4 + 2 * parts * rm * 4 <= (deep ? 176 : wave_registers(waves) - (waves <= 8 ? 0 : 64)) &&
+           2 * stage_shape(wbits, parts, rm, rn, wm, wn, pw, deep).stage_bytes <= kLdsBudget;
 }
+
+// kTiles' index of a ring tile id, and whether an id is a ring tile's.
+constexpr bool is_ring(int id) { return id <= kLeadTiles || id > kLeadTiles + kNumWsplitTiles; }
+constexpr int ring_index(int id) { return id <= kLeadTiles ? id - 1 : id - 1 - kNumWsplitTiles; }
 
 using KernelFn = void (*)(Params);
 

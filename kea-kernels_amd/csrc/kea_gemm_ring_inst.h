@@ -59,12 +59,12 @@ __device__ __forceinline__ void dma4(const void *g, void *lds_wave_base) {
 //
 // PW > 0 (producer waves): waves NW .. NW + PW - 1 of the workgroup issue every copy and wait for them, and the NW
 // compute waves never wait on memory counters for the ring; the stage barriers hand the buffers between the two.
-template <int WBITS, int P, int RM, int RN, int WM, int WN, bool SLICED, bool KTAIL, int GQ = 0, int PW = 0>
-__global__ void __launch_bounds__((WM * WN + PW) * 64) gemm_kernel(Params p) {
+template <int WBITS, int P, int RM, int RN, int WM, int WN, bool SLICED, bool KTAIL, int GQ = 0, int PW = 0, bool DEEP = false>
+__global__ void __launch_bounds__((WM * WN + PW) * 64, DEEP ? 2 : 1) gemm_kernel(Params p) {
     static_assert(GQ == 0 || GQ == 1 || GQ == 2 || GQ == 4, "groups of 64, 128 or 256 k");
     static_assert(GQ == 0 || !SLICED, "per-group scales run unsplit");
     static_assert(PW == 0 || GQ == 0, "producer waves: no per-group scales");
-    constexpr StageShape SHAPE = stage_shape(WBITS, P, RM, RN, WM, WN, PW);
+    constexpr StageShape SHAPE = stage_shape(WBITS, P, RM, RN, WM, WN, PW, DEEP);
     constexpr int SW = SHAPE.sw, NS = SHAPE.ns;
     constexpr int NW = WM * WN;                 // compute wavefronts
     constexpr int NI = PW > 0 ? PW : NW;        // wavefronts issuing the copies
@@ -94,7 +94,18 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) gemm_kernel(Params p) {
     const bool producer = PW > 0 && wave >= NW;  // wave-uniform
     const int iw = PW > 0 ? (producer ? wave - NW : 0) : wave;  // index among the issuing waves
     const int wm = wave / WN, wn = wave % WN;
-    const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
+    // Long K on the deep tiles: workgroup ids go round the 8 XCDs, so ids 8 apart (one XCD) walk the column tiles of one
+    // row tile and its L2 serves the activation rows after the first (16000 x 1024 x 4096, one part 85.5 -> 80 us on
+    // 64x128; three parts at M = 5333 86 -> 73 us). Short K measured 0 to 4% slower that way.
+    int bx = blockIdx.x, by = blockIdx.y;
+    if constexpr (DEEP) {
+        const int id = by * (int)gridDim.x + bx;
+        if (p.K >= 2048 && id < (int)((gridDim.y & ~7u) * gridDim.x)) {
+            bx = (id >> 3) % (int)gridDim.x;
+            by = (id >> 3) / (int)gridDim.x * 8 + (id & 7);
+        }
+    }
+    const int n0 = bx * BN, m0 = by * BM;
     const int nquads = (p.J + 3) >> 2;
     const int qa = SLICED ? (int)blockIdx.z * p.quads_per_slice : 0;
     const int qb = SLICED ? min(nquads, qa + p.quads_per_slice) : nquads;
@@ -328,28 +339,50 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) gemm_kernel(Params p) {
     }
 
     // Epilogue operands are fetched before the ring so their latency overlaps the main loads (the copies below are
-    // issued after these loads, so the stage waits never depend on them).
-    if constexpr (!SLICED) {
+    // issued after these loads, so the stage waits never depend on them): the raw words, converted after the ring. A
+    // conversion here, with its branch on the scale's type, made each of the 4 to 12 loads a memory round trip of its own
+    // before a workgroup's first copy (3200 cycles for a 128x128 tile on 4 waves).
+    uint32_t row_raw[RM][P];
+    v4u alpha_raw[RN], bias_raw[RN];
+    const bool qs_f16 = p.qs_dtype == KEA_F16, ws_f16 = p.ws_dtype == KEA_F16, bias_f16 = p.bias_dtype == KEA_F16;
+    const ColVec alpha_vec = col_vec(p.ws, ws_f16, p.N), bias_vec = col_vec(p.bias, bias_f16, p.bias ? p.N : 0);
+    auto part_scales = [&](int c) { return (const char *)p.qs + c * p.qs_stride * (qs_f16 ? 2 : 4); };
+    auto load_scales = [&]() {
 #pragma unroll
-        for (int i = 0; i < RM; ++i) load_row_scales<P>(p, m0 + (wm * RM + i) * 16 + (lane & 15), rows[i]);
+        for (int i = 0; i < RM; ++i) {
+            const int m = min(m0 + (wm * RM + i) * 16 + (lane & 15), p.M - 1);
 #pragma unroll
-        for (int jn = 0; jn < RN; ++jn)
-            load_col_scales(p, n0 + (wn * RN + jn) * 16 + (lane >> 4) * 4, cols[jn], GQ == 0);
-    }
-    // Residual values: prefetched with the other epilogue operands on small tiles, loaded in the epilogue otherwise
-    // (keeps the register budget of the wide tiles).
-    constexpr bool RES_PREFETCH = !SLICED && RM * RN <= 2;
-    float resv[RES_PREFETCH ? RM : 1][RES_PREFETCH ? RN : 1][4];
-    if constexpr (RES_PREFETCH) {
-        if (p.res) {
-#pragma unroll
-            for (int i = 0; i < RM; ++i)
-#pragma unroll
-                for (int jn = 0; jn < RN; ++jn)
-                    load_residual(p, m0 + (wm * RM + i) * 16 + (lane & 15), n0 + (wn * RN + jn) * 16 + (lane >> 4) * 4,
-                                  resv[i][jn]);
+            for (int c = 0; c < P; ++c) row_raw[i][c] = load_raw(part_scales(c), qs_f16, (uint32_t)m);
         }
-    }
+#pragma unroll
+        for (int jn = 0; jn < RN; ++jn) {
+            const int nb = n0 + (wn * RN + jn) * 16 + (lane >> 4) * 4;
+            if constexpr (GQ == 0) alpha_raw[jn] = col_load4(alpha_vec, ws_f16, nb);
+            bias_raw[jn] = col_load4(bias_vec, bias_f16, nb);  // zeros without a bias
+        }
+    };
+    if constexpr (!SLICED && !DEEP) load_scales();  // (deep tiles: no registers to spare, another workgroup computes)
+    auto convert_rows = [&]() {
+#pragma unroll
+        for (int i = 0; i < RM; ++i) {
+            const int m = min(m0 + (wm * RM + i) * 16 + (lane & 15), p.M - 1);
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                rows[i].s[c] = c < P ? raw_to_f32(row_raw[i][c < P ? c : 0], qs_f16, part_scales(c), (uint32_t)m) : 0.f;
+        }
+    };
+    auto convert_cols = [&]() {
+#pragma unroll
+        for (int jn = 0; jn < RN; ++jn) {
+            if constexpr (GQ == 0) col_to_f32(alpha_raw[jn], ws_f16, alpha_vec.delta, cols[jn].alpha);
+            col_to_f32(bias_raw[jn], bias_f16, bias_vec.delta, cols[jn].bias);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (GQ > 0) cols[jn].alpha[r] = 0.f;
+                if (!p.bias) cols[jn].bias[r] = kNoBias;
+            }
+        }
+    };
 
     // Per-group scales: the tile's alpha rows [n0, n0 + BN) x groups [0, 2^gp_shift) go to LDS as f32 in chunks of
     // ACH values per lane (zero past the last group; rows past N clamped, never stored). The first chunk's loads are
@@ -392,6 +425,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) gemm_kernel(Params p) {
         // LDS writes complete before the first stage barrier publishes them (lgkmcnt(0); vmcnt, expcnt untouched)
         __builtin_amdgcn_s_waitcnt(0xF | (3 << 14) | (7 << 4));
     }
+    if constexpr (GQ > 0) convert_rows();  // the folds read them
     using plain_t = std::integral_constant<bool, false>;
     using masked_t = std::integral_constant<bool, true>;
     for (int s = 0; s < nst - 1; ++s) {
@@ -408,120 +442,154 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) gemm_kernel(Params p) {
     // the last stage (the host never launches an empty K range, so nst >= 1)
     if constexpr (PW == 0) wait_vmcnt<0>();
     stage_barrier();
+
+    // An output without raw accumulators, whose 4-column vectors are aligned and never cross N, takes the straight
+    // epilogue below; the rest take the general one. Where the registers hold the residual's values beside the operands,
+    // they are loaded ahead of the last stage's MFMAs, otherwise one column block ahead of the stores (the residual may
+    // be y itself: a lane reads exactly the elements it writes, before it writes them).
+    // Its addresses are 32-bit offsets from the tile's first row, range-checked against the tile's last valid row, so
+    // neither the rows nor the columns need a branch (a column past N gets an offset past every range).
+    const bool straight = !SLICED && GQ == 0 && p.y && !p.acc && p.y_vec && ((p.N & 3) == 0 || n0 + BN <= p.N) &&
+                          p.ldy < (1 << 20) && (!p.res || (p.ldr < (1 << 20) && (p.ldr & 3) == 0 && ((uintptr_t)p.res & 15) == 0));
+    constexpr uint32_t kPastRange = 0x80000000u;
+    static_assert(BM <= 512, "512 rows of 2^20 floats stay below the sentinel offset");
+    const int rows_left = min(p.M - m0, BM);
+    auto tile_view = [&](const void *base, long long stride, int width, int esz) {
+        return __builtin_amdgcn_make_buffer_rsrc((char *)base + (long long)m0 * stride * esz, (short)0,
+                                                 (int)(((uint32_t)(rows_left - 1) * (uint32_t)stride + (uint32_t)width) * (uint32_t)esz),
+                                                 0x00020000);
+    };
+    constexpr bool EARLY = !DEEP && (P + 1) * RM * RN * 4 + 2 * P * RM * 4 + 96 <= wave_registers(NW + PW);
+    float4 resv[SLICED || GQ > 0 ? 1 : EARLY ? RN : 2][SLICED || GQ > 0 ? 1 : RM];  // [column block][row block]
+    auto load_residuals = [&](int jn, float4 (&v)[SLICED || GQ > 0 ? 1 : RM]) {
+        if constexpr (!SLICED && GQ == 0) {
+            const auto view = tile_view(p.res, p.ldr, p.N, 4);
+            const int nb = n0 + (wn * RN + jn) * 16 + (lane >> 4) * 4;
+            const uint32_t col = nb < p.N ? (uint32_t)nb * 4u : kPastRange;
+#pragma unroll
+            for (int i = 0; i < RM; ++i)
+                v[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                    view, (int)(((wm * RM + i) * 16 + (lane & 15)) * (uint32_t)p.ldr * 4u + col), 0, 0));
+        }
+    };
+    if constexpr (!SLICED && GQ == 0 && EARLY) {
+        if (straight && p.res) {
+#pragma unroll
+            for (int jn = 0; jn < RN; ++jn) load_residuals(jn, resv[jn]);
+        }
+    }
     compute(nst - 1, masked_t{});
+    if constexpr (!SLICED) {
+        if constexpr (DEEP) load_scales();
+        if constexpr (GQ == 0) convert_rows();
+        convert_cols();
+    }
 
     // ---- epilogue: the MFMA result row is the weight row n, the column the activation row m ----
-    // DT >= 0: the output dtype as a compile-time constant; then 16x16 tiles wholly inside [M, N) take a path without
-    // per-lane bounds or dtype selection (the tile test is wave-uniform). DT < 0: the general epilogue.
-    constexpr bool SMALL = RM * RN <= 2;
-    auto epilogue = [&](auto dt_tag, auto res_tag, auto silu_tag, auto glu_tag) {
-        constexpr int DT = decltype(dt_tag)::value;
-        constexpr bool RES = decltype(res_tag)::value;
-        constexpr int SILU = decltype(silu_tag)::value;
-        constexpr bool GLU = decltype(glu_tag)::value;
+    // The straight epilogue: one copy per output type, residual and SiLU (or GLU), nothing but arithmetic and stores: 5
+    // instructions an output where a block that tests its own bounds and forms 64-bit addresses takes 9. The 16 blocks
+    // of a wave (128x128 tile on 4 waves) took 5800 to 7700 cycles that way, more than its K loop at K = 1024. Epilogue
+    // and deep tiles together, 16000 x 4096 x 1024 (one part, f16 out): 122 -> 88 us, 16000 x 1024 x 4096 105 -> 66,
+    // three parts 5333 x 4096 x 1024 94 -> 77; non-temporal stores made the first 138 us.
+    if constexpr (!SLICED && GQ == 0) {
+        auto write = [&](auto dt_tag, auto res_tag, auto silu_tag, auto glu_tag) {
+            constexpr int DT = decltype(dt_tag)::value;
+            constexpr bool RES = decltype(res_tag)::value, SILU = decltype(silu_tag)::value, GLU = decltype(glu_tag)::value;
+            constexpr uint32_t ESZ = DT == KEA_F32 ? 4 : 2;
+            const auto view = tile_view(p.y, p.ldy, GLU ? p.N / 2 : p.N, ESZ);
+            uint32_t row_at[RM];
 #pragma unroll
-        for (int i = 0; i < RM; ++i) {
-            const int mt = m0 + (wm * RM + i) * 16, m = mt + (lane & 15);
-            if (m >= p.M) continue;
-            void *yrow = (int8_t *)p.y + (long long)m * p.ldy * (DT == KEA_F32 ? 4 : 2);  // unused when DT < 0
+            for (int i = 0; i < RM; ++i) row_at[i] = (uint32_t)((wm * RM + i) * 16 + (lane & 15)) * (uint32_t)p.ldy * ESZ;
+            if constexpr (RES && !EARLY) load_residuals(0, resv[0]);
 #pragma unroll
             for (int jn = 0; jn < RN; ++jn) {
-                const int nt = n0 + (wn * RN + jn) * 16, nb = nt + (lane >> 4) * 4;
-                if (nb >= p.N) continue;
-                int a[P][4];
+                if constexpr (RES && !EARLY) {
+                    if (jn + 1 < RN) load_residuals(jn + 1, resv[(jn + 1) & 1]);
+                }
+                const int nb = n0 + (wn * RN + jn) * 16 + (lane >> 4) * 4;
+                const uint32_t col_at = nb < p.N ? (uint32_t)(GLU ? nb / 2 : nb) * ESZ : kPastRange;
 #pragma unroll
-                for (int c = 0; c < P; ++c)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) a[c][r] = acc[c][i][jn][r];
-                if constexpr (SLICED) {
+                for (int i = 0; i < RM; ++i) {
+                    int a[P][4];
 #pragma unroll
                     for (int c = 0; c < P; ++c)
-                        store_int4(p.slices + (((long long)blockIdx.z * P + c) * p.M + m) * p.N + nb, p.slice_vec,
-                                   nb, p.N, a[c]);
-                } else {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) a[c][r] = acc[c][i][jn][r];
                     EpiOperands e = cols[jn];
 #pragma unroll
                     for (int c = 0; c < 3; ++c) e.s[c] = rows[i].s[c];
-                    if constexpr (RES_PREFETCH) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) e.res[r] = resv[i][jn][r];
-                    } else {
-                        load_residual(p, m, nb, e.res);
+                    if constexpr (RES) {
+                        const float4 v = resv[EARLY ? jn : jn & 1][i];
+                        e.res[0] = v.x; e.res[1] = v.y; e.res[2] = v.z; e.res[3] = v.w;
                     }
-                    if constexpr (GQ > 0) {
-                        epilogue4_groups<P>(p, m, nb, a, racc[i][jn], e);
-                    } else if constexpr (DT >= 0) {
-                        if (mt + 16 <= p.M && nt + 16 <= p.N) {
-                            epilogue4_full<P, DT, RES, SMALL, SILU, GLU>(p, yrow, nb, a, e);
-                            continue;
-                        }
-                        epilogue4<P>(p, m, nb, a, e);
-                    } else {
-                        epilogue4<P>(p, m, nb, a, e);
-                    }
+                    float v[4];
+                    epilogue4_values<P, RES, false, SILU ? 1 : 0>(p, a, e, v);
+                    put4_as<DT, GLU>(v, [&](auto bits) {
+                        const int at = (int)(row_at[i] + col_at);
+                        if constexpr (sizeof(bits) == 16) __builtin_amdgcn_raw_buffer_store_b128(bits, view, at, 0, 0);
+                        else if constexpr (sizeof(bits) == 8) __builtin_amdgcn_raw_buffer_store_b64(bits, view, at, 0, 0);
+                        else __builtin_amdgcn_raw_buffer_store_b32(bits, view, at, 0, 0);
+                    });
                 }
             }
+        };
+        using yes = std::true_type;
+        using no = std::false_type;
+        auto by_flags = [&](auto dt_tag) {
+            const bool silu = (p.flags & KEA_FLAG_SILU) != 0;
+            if (p.flags & KEA_FLAG_GLU) write(dt_tag, no{}, no{}, yes{});  // (neither residual nor SiLU)
+            else if (p.res && silu) write(dt_tag, yes{}, yes{}, no{});
+            else if (p.res) write(dt_tag, yes{}, no{}, no{});
+            else if (silu) write(dt_tag, no{}, yes{}, no{});
+            else write(dt_tag, no{}, no{}, no{});
+        };
+        if (straight) {
+            if (p.y_dtype == KEA_F16) by_flags(std::integral_constant<int, KEA_F16>{});
+            else if (p.y_dtype == KEA_BF16) by_flags(std::integral_constant<int, KEA_BF16>{});
+            else by_flags(std::integral_constant<int, KEA_F32>{});
+            return;
         }
-    };
-    // Outputs without raw accumulators and with a vector-aligned y branch once on the dtype (and GLU outputs, which
-    // take neither residual nor SiLU, on the GLU); the rest take the general epilogue.
-    const bool glu = (p.flags & KEA_FLAG_GLU) != 0;
-    const bool plain = !SLICED && GQ == 0 && p.y && !p.acc && p.y_vec && !glu;
-    const bool plain_glu = !SLICED && GQ == 0 && p.y && !p.acc && p.y_vec && glu && !p.res;
-    using kRes = std::true_type;
-    using kNoRes = std::false_type;
-    using kGlu = std::true_type;
-    using kNoGlu = std::false_type;
-    using kSiluAtRunTime = std::integral_constant<int, -1>;
-    using kNoSilu = std::integral_constant<int, 0>;
-    using kGeneral = std::integral_constant<int, -1>;
-    if (plain_glu) {
-        if (p.y_dtype == KEA_F32) epilogue(std::integral_constant<int, KEA_F32>{}, kNoRes{}, kNoSilu{}, kGlu{});
-        else if (p.y_dtype == KEA_F16) epilogue(std::integral_constant<int, KEA_F16>{}, kNoRes{}, kNoSilu{}, kGlu{});
-        else epilogue(std::integral_constant<int, KEA_BF16>{}, kNoRes{}, kNoSilu{}, kGlu{});
-        return;
     }
-    // Tiles of one or two 16x16 blocks per wave (the small-M shapes) keep one epilogue copy per dtype with the
-    // residual, bias and SiLU tested at run time: separate copies measured slower there (config 1: 4.13 vs 4.27 us).
-    if constexpr (SMALL) {
-        if (plain && p.y_dtype == KEA_F16) epilogue(std::integral_constant<int, KEA_F16>{}, kNoRes{}, kSiluAtRunTime{}, kNoGlu{});
-        else if (plain && p.y_dtype == KEA_BF16) epilogue(std::integral_constant<int, KEA_BF16>{}, kNoRes{}, kSiluAtRunTime{}, kNoGlu{});
-        else if (plain && p.y_dtype == KEA_F32) epilogue(std::integral_constant<int, KEA_F32>{}, kNoRes{}, kSiluAtRunTime{}, kNoGlu{});
-        else epilogue(kGeneral{}, kNoRes{}, kSiluAtRunTime{}, kNoGlu{});
-        return;
-    }
-    // Wider tiles: one copy per dtype, residual and SiLU, so the full-block path carries neither test nor a SiLU
-    // evaluated only to be discarded.
-    auto by_flags = [&](auto dt_tag) {
-        const bool silu = (p.flags & KEA_FLAG_SILU) != 0;
-        if (p.res) {
-            if (silu) epilogue(dt_tag, kRes{}, std::integral_constant<int, 1>{}, kNoGlu{});
-            else epilogue(dt_tag, kRes{}, kNoSilu{}, kNoGlu{});
-        } else {
-            if (silu) epilogue(dt_tag, kNoRes{}, std::integral_constant<int, 1>{}, kNoGlu{});
-            else epilogue(dt_tag, kNoRes{}, kNoSilu{}, kNoGlu{});
+    // The general epilogue: split-K slices, raw accumulators, per-group scales, unaligned outputs, N % 4 != 0.
+#pragma unroll
+    for (int i = 0; i < RM; ++i) {
+        const int m = m0 + (wm * RM + i) * 16 + (lane & 15);
+        if (m >= p.M) continue;
+#pragma unroll
+        for (int jn = 0; jn < RN; ++jn) {
+            const int nb = n0 + (wn * RN + jn) * 16 + (lane >> 4) * 4;
+            if (nb >= p.N) continue;
+            int a[P][4];
+#pragma unroll
+            for (int c = 0; c < P; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) a[c][r] = acc[c][i][jn][r];
+            if constexpr (SLICED) {
+#pragma unroll
+                for (int c = 0; c < P; ++c)
+                    store_int4(p.slices + (((long long)blockIdx.z * P + c) * p.M + m) * p.N + nb, p.slice_vec, nb, p.N,
+                               a[c]);
+            } else {
+                EpiOperands e = cols[jn];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) e.s[c] = rows[i].s[c];
+                load_residual(p, m, nb, e.res);
+                if constexpr (GQ > 0) epilogue4_groups<P>(p, m, nb, a, racc[i][jn], e);
+                else epilogue4<P>(p, m, nb, a, e);
+            }
         }
-    };
-    if (plain && p.y_dtype == KEA_F16) {
-        by_flags(std::integral_constant<int, KEA_F16>{});
-    } else if (plain && p.y_dtype == KEA_BF16) {
-        by_flags(std::integral_constant<int, KEA_BF16>{});
-    } else if (plain && p.y_dtype == KEA_F32) {
-        by_flags(std::integral_constant<int, KEA_F32>{});
-    } else {
-        epilogue(kGeneral{}, kNoRes{}, kSiluAtRunTime{}, kNoGlu{});
     }
 }
 
-template <int WBITS, int P, int RM, int RN, int WM, int WN, int PW>
+template <int WBITS, int P, int RM, int RN, int WM, int WN, int PW, bool DEEP>
 KernelFn pick_sliced(bool sliced) {
-    return sliced ? gemm_kernel<WBITS, P, RM, RN, WM, WN, true, false, 0, PW>
-                  : gemm_kernel<WBITS, P, RM, RN, WM, WN, false, false, 0, PW>;
+    return sliced ? gemm_kernel<WBITS, P, RM, RN, WM, WN, true, false, 0, PW, DEEP>
+                  : gemm_kernel<WBITS, P, RM, RN, WM, WN, false, false, 0, PW, DEEP>;
 }
 
-template <int WBITS, int P, int RM, int RN, int WM, int WN, int PW>
+template <int WBITS, int P, int RM, int RN, int WM, int WN, int PW, bool DEEP>
 KernelFn pick_fit(bool sliced) {
-    if constexpr (tile_fits(WBITS, P, RM, RN, WM, WN, PW)) return pick_sliced<WBITS, P, RM, RN, WM, WN, PW>(sliced);
+    if constexpr (tile_fits(WBITS, P, RM, RN, WM, WN, PW, DEEP)) return pick_sliced<WBITS, P, RM, RN, WM, WN, PW, DEEP>(sliced);
     else return nullptr;
 }
 
@@ -529,13 +597,13 @@ KernelFn pick_fit(bool sliced) {
 template <int WBITS, int P, int I>
 KernelFn pick_index(bool sliced) {
     constexpr Tile t = kTiles[I];
-    return pick_fit<WBITS, P, t.rm, t.rn, t.wm, t.wn, t.pw>(sliced);
+    return pick_fit<WBITS, P, t.rm, t.rn, t.wm, t.wn, t.pw, t.deep>(sliced);
 }
 
 template <int WBITS, int P>
 KernelFn pick_tile(int id, bool sliced) {
-    static_assert(kNumTiles == 12, "one case per tile id");
-    switch (id) {
+    static_assert(kNumTiles == 15, "one case per tile");
+    switch (ring_index(id) + 1) {
         case 1: return pick_index<WBITS, P, 0>(sliced);
         case 2: return pick_index<WBITS, P, 1>(sliced);
         case 3: return pick_index<WBITS, P, 2>(sliced);
@@ -548,6 +616,9 @@ KernelFn pick_tile(int id, bool sliced) {
         case 10: return pick_index<WBITS, P, 9>(sliced);
         case 11: return pick_index<WBITS, P, 10>(sliced);
         case 12: return pick_index<WBITS, P, 11>(sliced);
+        case 13: return pick_index<WBITS, P, 12>(sliced);
+        case 14: return pick_index<WBITS, P, 13>(sliced);
+        case 15: return pick_index<WBITS, P, 14>(sliced);
         default: return nullptr;
     }
 }

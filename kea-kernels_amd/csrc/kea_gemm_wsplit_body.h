@@ -10,19 +10,6 @@
 
 namespace kea {
 
-// The aligned 32-bit word holding element i of an f32 or f16 vector (f16: the half is selected at conversion time by
-// raw_to_f32 with the same v and i). The word lies inside the 4-byte block of an in-bounds element, so it never
-// reaches past a page the vector touches.
-__device__ __forceinline__ uint32_t load_raw(const void *v, bool f16, uint32_t i) {
-    const char *a = (const char *)v + (f16 ? 2u * i : 4u * i);
-    return *(const uint32_t *)__builtin_align_down(a, 4);  // keeps the pointer's (global) address space
-}
-__device__ __forceinline__ float raw_to_f32(uint32_t raw, bool f16, const void *v, uint32_t i) {
-    const uint32_t hi = (uint32_t)(((uintptr_t)v >> 1) + i) & 1u;  // f16: which half of the word
-    const float h = (float)__builtin_bit_cast(_Float16, (uint16_t)(raw >> (hi * 16)));
-    return f16 ? h : __builtin_bit_cast(float, raw);
-}
-
 // The wave's weight words: WPW native words per lane for each of the NT n-tiles from the tile at column n0, starting
 // at word j0 (J words per lane per n-tile). RAGGED = false: complete quads of words (or one word per wave), loaded
 // with 64- or 128-bit vector loads; otherwise general per-word addressing (a short last quad has lane stride < 4,
