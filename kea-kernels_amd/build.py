@@ -4,7 +4,8 @@ benchmark's probe library libkea_probe.so (include/kea_probe.h) in-tree with hip
     python kea-kernels_amd/build.py [-j JOBS] [--max-stages N]
 
 Objects go to kea-kernels_amd/_build/, the product library to kea-kernels_amd/kea_kernels/lib/libkea_hip.so and the
-probe library, which nothing in the package loads, to kea-kernels_amd/kea_probes/lib/libkea_probe.so.
+probe library, which nothing in the package loads, to kea-kernels_amd/kea_probes/lib/libkea_probe.so. The host extension
+module kea_native (the operators' native call path) goes to kea-kernels_amd/kea_kernels/lib/kea_native.so.
 --max-stages N rebuilds every translation unit with another LDS-ring depth cap for the ring kernel (default 2; a
 measurement knob: the host's LDS sizing and the kernels must agree, so it is never set per file).
 Every source is compiled for gfx950 only; device FP contraction is off (the epilogue's FP32 op order is part
@@ -27,6 +28,8 @@ LIB = HERE / "kea_kernels" / "lib" / "libkea_hip.so"
 PROBE_DIR = HERE / "kea_probes"
 PROBE_LIB = PROBE_DIR / "lib" / "libkea_probe.so"
 PROBE_SOURCES = ["kea_probe.hip"]
+NATIVE_SRC = CSRC / "kea_native.cpp"
+NATIVE_LIB = HERE / "kea_kernels" / "lib" / "kea_native.so"
 SOURCES = ["kea_gemm_ring_w1.hip", "kea_gemm_ring_w2.hip", "kea_gemm_wsplit_p1.hip", "kea_gemm_wsplit_p2.hip",
            "kea_gemm_wsplit_p3.hip", "kea_gemm_wsplit_g1.hip", "kea_gemm_wsplit_g2.hip", "kea_gemm_wsplit_g3.hip",
            "kea_gemm.hip", "kea_gemm_wsplit.hip", "kea_quantize.hip", "kea_encoder.hip",
@@ -83,14 +86,35 @@ def _link(objs: list[Path], lib: Path) -> None:
     os.replace(tmp, lib)
 
 
+def _build_native() -> None:
+    """The host extension module kea_native (kea_kernels/lib/kea_native.so), against the installed PyTorch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    tmp = NATIVE_LIB.with_suffix(".so.tmp")
+    NATIVE_LIB.parent.mkdir(parents=True, exist_ok=True)
+    libs = Path(torch.__file__).parent / "lib"
+    cmd = [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-shared", "-w", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{sysconfig.get_paths()['include']}",
+           *(f"-I{p}" for p in cpp_extension.include_paths()), "-I/opt/rocm/include", str(NATIVE_SRC), "-o", str(tmp),
+           f"-L{libs}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", f"-Wl,-rpath,{libs}"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{res.stderr}")
+    os.replace(tmp, NATIVE_LIB)
+
+
 def build(jobs: int | None = None) -> Path:
-    """Compiles every translation unit of both libraries (in parallel) and links them; returns the product library."""
+    """Compiles every translation unit of both libraries and the host extension (in parallel) and links them; returns the
+    product library."""
     BUILD.mkdir(exist_ok=True)
     units = [(CSRC / s, BUILD / (Path(s).stem + ".o")) for s in SOURCES]
     probe_units = [(PROBE_DIR / s, BUILD / (Path(s).stem + ".o")) for s in PROBE_SOURCES]
     jobs = jobs or min(len(units) + len(probe_units), os.cpu_count() or 1)
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
         futures = [pool.submit(_compile, src, obj) for src, obj in units + probe_units]
+        futures.append(pool.submit(_build_native))
         for f in futures:
             f.result()
     _link([obj for _, obj in units], LIB)

@@ -12,12 +12,14 @@ a RuntimeError: there is no fallback path.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import threading
 from pathlib import Path
 
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libkea_hip.so"
+NATIVE_PATH = LIB_PATH.with_name("kea_native.so")
 
 F32, F16, BF16 = 0, 1, 2
 FLAG_SILU, FLAG_ORDER = 1, 2
@@ -105,6 +107,28 @@ def lib() -> ctypes.CDLL:
                     fn.restype, fn.argtypes = restype, argtypes
                 _lib = handle
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The host extension module (csrc/kea_native.cpp: checks, allocations and launch of an operator call in one native
+    call), bound to the library's entry points. RuntimeError if it was not built."""
+    global _native
+    if _native is None:
+        library = lib()
+        with _lock:
+            if _native is None:
+                if not NATIVE_PATH.is_file():
+                    raise RuntimeError(f"{NATIVE_PATH} is missing: build it with `python kea-kernels_amd/build.py`")
+                spec = importlib.util.spec_from_file_location("kea_native", NATIVE_PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                module.bind(*(ctypes.cast(getattr(library, name), ctypes.c_void_p).value for name in (
+                    "kea_lowbit_project_launch", "kea_lowbit_gemm", "kea_lowbit_gemm_residual", "kea_quantize")))
+                _native = module
+    return _native
 
 
 def last_error() -> str:

@@ -24,6 +24,11 @@ from kea_kernels.binary import kernels
 
 round_up = lowbit.round_up
 
+# Call tags of Launches.replay: the operator and its part count, and for the provider's fused op its options.
+_LINEAR, _CONV = 8, 16
+PROJECT_TAGS = {(conv, parts, activation, inp): 64 + 16 * parts + 4 * conv + 2 * (activation == "silu") + (inp == "silu")
+                for conv in (False, True) for parts in (1, 2, 3) for activation in ("", "silu") for inp in ("", "silu")}
+
 
 class Int8MmaLayer:
     """One layer resident as native 1-bit words plus FP32 scale / bias. Calls use three activation parts (x3), as
@@ -87,10 +92,13 @@ class Int8MmaLayer:
 
     def linear(self, x: Tensor, *, out_dtype: torch.dtype = torch.float32) -> Tensor:
         """[..., K] -> [..., N] (FP32 unless out_dtype says otherwise)."""
-        launches, key = self.launches, _call_key(x, out_dtype, "linear")
+        launches = self.launches
+        y = launches.replay(x, out_dtype, _LINEAR + self.PARTS)
+        if y is not None:  # a layout checked and resolved before: everything checked derives from it
+            return y
+        key = _call_key(x, out_dtype, "linear")
         hit = launches.recall(key)
         if hit is not None and not (x.requires_grad and torch.is_grad_enabled()):
-            # a layout checked and resolved before: everything checked derives from the key
             y = torch.empty(hit[1], device=self.device, dtype=out_dtype)
             launches.launch(hit[0], x, y)
             return y
@@ -110,11 +118,16 @@ class Int8MmaLayer:
             e = self._run(xr, rows, m, y.view(m, self.out_features))
             if e and key is not None and xr.data_ptr() == x.data_ptr():  # not where the reshape copied x
                 launches.remember(key, e, y.shape)
+                launches.keep(x, out_dtype, _LINEAR + self.PARTS, e, y.shape)
         return y
 
     def conv(self, x: Tensor, *, out_dtype: torch.dtype = torch.float32) -> Tensor:
         """Pointwise convolution [B, K, T] -> [B, N, T] (a transposed view of a [B, T, N] result)."""
-        launches, key = self.launches, _call_key(x, out_dtype, "conv")
+        launches = self.launches
+        y = launches.replay(x, out_dtype, _CONV + self.PARTS)
+        if y is not None:
+            return y
+        key = _call_key(x, out_dtype, "conv")
         hit = launches.recall(key)
         if hit is not None and not (x.requires_grad and torch.is_grad_enabled()):
             y = torch.empty(hit[1], device=self.device, dtype=out_dtype)
@@ -127,6 +140,7 @@ class Int8MmaLayer:
             e = self._run(x, (x.stride(0), x.stride(2), x.stride(1), t), b * t, y.view(b * t, self.out_features))
             if e and key is not None:
                 launches.remember(key, e, y.shape)
+                launches.keep(x, out_dtype, _CONV + self.PARTS, e, y.shape, transposed=True)
         return y.transpose(1, 2)
 
     def _run(self, x: Tensor, rows: tuple, m: int, y: Tensor):
@@ -167,6 +181,11 @@ def _project(layer: Int8MmaLayer, x: Tensor, conv: bool, parts: int, activation:
              input_activation: str) -> Tensor:
     if activation not in ("", "silu") or input_activation not in ("", "silu"):
         raise ValueError(f"unsupported activation {activation!r} / {input_activation!r}")
+    launches, tag = layer.launches, PROJECT_TAGS.get((bool(conv), parts, activation, input_activation))
+    if tag is not None:
+        y = lowbit.replay(launches, x, torch.float32, tag, norm)
+        if y is not None:
+            return y
     xx = x.transpose(1, 2) if conv else x
     layer._check(xx, "linear")
     if xx.dim() == 2:
@@ -178,10 +197,14 @@ def _project(layer: Int8MmaLayer, x: Tensor, conv: bool, parts: int, activation:
     y = torch.empty(b, t, n, device=layer.device, dtype=torch.float32)
     if m:
         rows = (xx.stride(0), xx.stride(1), xx.stride(2), t)
-        if not layer.launches.project(xx, rows, m, parts, y.view(m, n), silu=activation == "silu", norm=norm,
-                                      input_activation=input_activation):
+        e = launches.project(xx, rows, m, parts, y.view(m, n), silu=activation == "silu", norm=norm,
+                             input_activation=input_activation)
+        if not e:
             q, qs, ldq = lowbit.quantize(xx, rows, m, k, parts, norm=norm, input_activation=input_activation)
             layer.dot(q, qs, ldq, m, y.view(m, n), silu=activation == "silu")
+        elif tag is not None:
+            launches.keep(x, torch.float32, tag, e, (b, t, n) if x.dim() == 3 else (*x.shape[:-1], n),
+                          transposed=bool(conv), norm=norm)
     if conv:
         return y.transpose(1, 2)
     return y if x.dim() == 3 else y.view(*x.shape[:-1], n)

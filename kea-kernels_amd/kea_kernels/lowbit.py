@@ -103,6 +103,22 @@ def _gemm_args(wbits, q, qs, words, n, k, wscale, bias, y, acc_out, m, silu, ord
     return args, device, workspace
 
 
+def _native_gemm(wbits, q, qs, words, n, k, wscale, bias, y, acc_out, m, silu, order, config, ws_group, residual,
+                 residual_factor, glu) -> bool:
+    """gemm() in one native call (the same checks on the tensors' fields); False, having launched nothing, where an
+    argument is not what it takes: the Python path then checks again and raises or launches."""
+    try:
+        parts, rows = q.shape[0], q.shape[1]
+        tile, split = (int(config.tile), int(config.split)) if hasattr(config, "tile") else (0, 0)
+        m = rows if m is None else m
+        return _hip.native().gemm(
+            wbits, q, qs, words, _native_words(wbits, n, k), n, k, wscale, bias, y, acc_out, m,
+            int(silu) | (2 * int(order)) | (4 * int(glu)), split, tile, ws_group,
+            _workspace_bytes(wbits, parts, m, n, k, ws_group, split, tile), residual, residual_factor)
+    except (AttributeError, IndexError, TypeError, ValueError):
+        return False
+
+
 def gemm(wbits: int, q: Tensor, qs: Tensor, words: Tensor, n: int, k: int, wscale: Tensor, bias: Tensor | None,
          y: Tensor | None = None, acc_out: Tensor | None = None, *, m: int | None = None, silu: bool = False,
          order: int = 0, config=None, ws_group: int = 0, residual: Tensor | None = None,
@@ -111,6 +127,9 @@ def gemm(wbits: int, q: Tensor, qs: Tensor, words: Tensor, n: int, k: int, wscal
     qs [P, M] (f32 or f16). words: native layout of `wbits`-bit weights; wscale [N] (or [N, G] with ws_group).
     residual (FP32 [>= m, >= N] rows, may be y itself): y = residual + value * residual_factor.
     glu: y [m, N/2] = value[2j] * sigmoid(value[2j + 1]) (weight rows interleaved value, gate)."""
+    if _native_gemm(wbits, q, qs, words, n, k, wscale, bias, y, acc_out, m, silu, order, config, ws_group, residual,
+                    residual_factor, glu):
+        return
     args, device, _ = _gemm_args(wbits, q, qs, words, n, k, wscale, bias, y, acc_out, m, silu, order, config,
                                  ws_group, residual, glu)
     L = _hip.lib()
@@ -266,11 +285,27 @@ def round_up(v: int, multiple: int) -> int:
     return -(-v // multiple) * multiple
 
 
+def _native_quantize(x, rows, m, k, parts, norm, input_activation, qs_dtype, ldq) -> tuple | None:
+    """quantize() in one native call; None, having launched nothing, where an argument is not what it takes."""
+    try:
+        xb, xt, xk, t = rows
+        nw, nb, eps = (None, None, 0.0) if norm is None else (norm.weight.detach(), norm.bias.detach(), float(norm.eps))
+        ldq = round_up(k, 16) if ldq is None else ldq
+        hit = _hip.native().quantize(x, xb, xt, xk, max(t, 1), m, k, parts, nw, nb, eps, input_activation == "silu",
+                                     qs_dtype, ldq)
+        return hit and (hit[0], hit[1], ldq)
+    except (AttributeError, TypeError, ValueError):
+        return None
+
+
 def quantize(x: Tensor, rows: tuple, m: int, k: int, parts: int, *, norm=None, input_activation: str = "",
              qs_dtype: torch.dtype = torch.float32, ldq: int | None = None) -> tuple[Tensor, Tensor, int]:
     """Residual int8 parts of x: row r at x + (r // T) * XB + (r % T) * XT + kk * XK with rows = (XB, XT, XK, T).
 
     Returns q int8 [parts, m, ldq] (zero padded from k to ldq = round_up(k, 16)), qs [parts, m] and ldq."""
+    if input_activation in ("", "silu") and (hit := _native_quantize(x, rows, m, k, parts, norm, input_activation,
+                                                                     qs_dtype, ldq)):
+        return hit
     if x.dtype not in (torch.float32, torch.float16):
         raise ValueError(f"expected FP32 or FP16 input, got {x.dtype}")
     if input_activation not in ("", "silu"):
@@ -307,6 +342,16 @@ def quantize(x: Tensor, rows: tuple, m: int, k: int, parts: int, *, norm=None, i
     return q, qs, ldq
 
 
+def replay(launches: "Launches", x, out_dtype: torch.dtype, tag: int, norm) -> Tensor | None:
+    """launches.replay() with an optional LayerNorm; None where the LayerNorm has no parameters to key on."""
+    if norm is None:
+        return launches.replay(x, out_dtype, tag)
+    try:
+        return launches.replay(x, out_dtype, tag, norm.weight, norm.bias, norm.eps)
+    except AttributeError:
+        return None
+
+
 class _Entry:
     """One resolved call layout of a Launches cache: a plan (a projection plan, or a GEMM plan for dot()), the C
     function that frees it and the device workspace bytes one launch of it needs."""
@@ -337,6 +382,10 @@ class Launches:
         self.max_entries = max_entries
         self._entries: dict = {}
         self._calls: dict = {}
+        # call(x, out_dtype, tag[, norm weight, norm bias, eps]) -> the output of a kept layout, or None: the key, both
+        # allocations and the launch in one native call (see keep())
+        self._replays = _hip.native().Replays(max_entries)
+        self.replay = self._replays.call
 
     def __len__(self) -> int:
         return len(self._entries)
@@ -395,6 +444,15 @@ class Launches:
         if len(self._calls) >= self.max_entries:
             self._calls.pop(next(iter(self._calls)), None)
         self._calls[key] = (e, out_shape)
+
+    def keep(self, x: Tensor, out_dtype: torch.dtype, tag: int, e: _Entry, out_shape: tuple, *, transposed: bool = False,
+             norm=None) -> None:
+        """Keeps a projection entry for replay(): the operator's call `tag` on inputs of x's sizes, strides, dtype and
+        device (and this LayerNorm, by its parameters' addresses as in project()) launches it on a new output of
+        `out_shape`, returned with its last two dimensions exchanged if `transposed`. The layout must determine every
+        argument the operator checks and passes. Up to `max_entries` layouts (the oldest is dropped first)."""
+        nw, nb, eps = (None, None, 0.0) if norm is None else (norm.weight, norm.bias, float(norm.eps))
+        self._replays.keep(x, out_dtype, tag, nw, nb, eps, e, e.plan, e.need, tuple(out_shape), transposed)
 
     def _resolve(self, key, x, rows, m, parts, y, silu, order, norm, input_activation, config) -> _Entry:
         """The first call of a layout: the full checks of quantize() and gemm() on real buffers, then the plan."""

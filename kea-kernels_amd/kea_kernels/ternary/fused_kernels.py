@@ -14,6 +14,7 @@ import torch
 
 from kea_kernels import lowbit
 from kea_kernels.binary import configs
+from kea_kernels.binary.layer import PROJECT_TAGS
 from kea_kernels.ternary.runtime import native_words
 
 
@@ -35,6 +36,12 @@ def int8_matmul(x, mod, conv=False, components=1, activation="", norm=None, conf
         raise ValueError(f"unsupported activation {activation!r} / {input_activation!r}")
     if components not in (1, 2, 3):
         raise ValueError(f"components must be 1, 2 or 3, got {components!r}")
+    launches = None
+    if not hasattr(config, "tile") and isinstance(x, torch.Tensor) and x.is_cuda:
+        launches, tag = _launches(mod), PROJECT_TAGS[bool(conv), components, activation, input_activation]
+        y = lowbit.replay(launches, x, torch.float32, tag, norm)
+        if y is not None:
+            return y
     xx = x.transpose(1, 2) if conv else x
     if xx.ndim == 2:
         xx = xx.unsqueeze(0)
@@ -46,10 +53,16 @@ def int8_matmul(x, mod, conv=False, components=1, activation="", norm=None, conf
     m, n = b * t, mod.out_features
     y = torch.empty((b, t, n), dtype=torch.float32, device=x.device)
     if m:
-        launches = _launches(mod)
+        kept = launches is not None
+        if launches is None:
+            launches = _launches(mod)
         rows = (xx.stride(0), xx.stride(1), xx.stride(2), t)
-        if not launches.project(xx, rows, m, components, y.view(m, n), silu=activation == "silu", norm=norm,
-                                input_activation=input_activation, config=config):
+        e = launches.project(xx, rows, m, components, y.view(m, n), silu=activation == "silu", norm=norm,
+                             input_activation=input_activation, config=config)
+        if e and kept:
+            launches.keep(x, torch.float32, tag, e, (b, t, n) if conv else (*x.shape[:-1], n), transposed=bool(conv),
+                          norm=norm)
+        if not e:
             q, qs, _ = _quantize(xx, components, norm, input_activation)
             lowbit.gemm(2, q, qs, native_words(mod), n, k, mod.scale, mod.bias, y.view(m, n), None,
                         silu=activation == "silu", config=config)
