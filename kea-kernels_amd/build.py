@@ -33,7 +33,7 @@ NATIVE_LIB = HERE / "kea_kernels" / "lib" / "kea_native.so"
 SOURCES = ["kea_gemm_ring_w1.hip", "kea_gemm_ring_w2.hip", "kea_gemm_wsplit_p1.hip", "kea_gemm_wsplit_p2.hip",
            "kea_gemm_wsplit_p3.hip", "kea_gemm_wsplit_g1.hip", "kea_gemm_wsplit_g2.hip", "kea_gemm_wsplit_g3.hip",
            "kea_gemm.hip", "kea_gemm_wsplit.hip", "kea_quantize.hip", "kea_encoder.hip",
-           "kea_attention.hip", "kea_layout.cpp"]
+           "kea_attention.hip", "kea_subsample.hip", "kea_layout.cpp"]
 ARCH = "gfx950"
 # Per-source flags. The probe's loop keeps eight MFMA accumulators live across iterations; in the accumulator
 # (AGPR) form the register allocator shuffles them with accvgpr moves every iteration, which would be measured as

@@ -3,14 +3,10 @@
 //
 //   s[i][j] = ((q_i + u) . k_j + (q_i + v) . p_{T-1-i+j}) * scale,  out_i = sum_j softmax_j(s)[i][j] v_j
 //
-// Arithmetic. The FP32 matrix instruction runs at 1/16 of the FP16 rate, so every operand is split into two FP16
-// values, x * 2^a = hi + lo, and a product takes three FP16 MFMAs with FP32 accumulation (hi hi + hi lo + lo hi; the
-// dropped lo lo term is 2^-22 of the product, of random sign). The power of two a is chosen per query row, per four
-// rows of K and P and per eight keys of V so that the largest value lies in [2^14, 2^15): hi + lo then holds every
-// element to 2^-22 of itself or 2^-39 of that largest value, whatever the input's range, and the scaling is exact.
-// Against FP64 the result is closer than the FP32 forms (fewer roundings of the accumulator). An infinity in the
-// inputs has no such scale: a workgroup that meets one recomputes its rows with plain FP32 dot products (NaNs
-// propagate by themselves).
+// Arithmetic. The FP32 matrix instruction runs at 1/16 of the FP16 rate, so operands are pairs of FP16 values and a
+// product is three FP16 MFMAs (kea_split.h), with one power of two per query row, per four rows of K and P and per eight
+// keys of V. Against FP64 the result is closer than the FP32 forms (fewer roundings of the accumulator). A workgroup
+// that meets an infinity recomputes its rows with plain FP32 dot products (NaNs propagate by themselves).
 //
 // Two launches. split_kernel writes K, V and P once as hi / lo planes in the order the LDS of the second kernel holds
 // them, 64 rows to a block; relpos_tiled_kernel then copies blocks straight to LDS (global_load_lds) and spends no
@@ -42,59 +38,24 @@
 #include <type_traits>
 
 #include "kea_internal.h"
+#include "kea_split.h"
 #include "kea_wave.h"
 #include "../../include/kea_encoder.h"
 
 namespace {
 
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-
 constexpr int kDK = 128;
 
-using kea::dpp;
+using kea::exponent_of;
+using kea::kInfBits;
+using kea::max_abs;
+using kea::pow2;
+using kea::split8;
+using kea::v4f;
+using kea::v8h;
 using kea::wave_max;
+using kea::wave_max_bits;
 using kea::wave_sum;
-
-// The binary exponent e of a magnitude given by its bits (2^e <= m < 2^(e+1)), clamped so that 2^(14-e) and 2^(e-14)
-// are normal numbers.
-__device__ __forceinline__ int exponent_of(int bits) { return min(max((bits >> 23) - 127, -90), 127); }
-// 2^e for e in [-127, 127] (2^-127 as zero).
-__device__ __forceinline__ float pow2(int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); }
-
-// x * sf (sf a power of two) as hi + lo: one mixed-precision fma for each half.
-__device__ __forceinline__ void split8(const float *x, float sf, v8h &hi, v8h &lo) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        hi[e] = (_Float16)__builtin_fmaf(x[e], sf, 0.f);
-        lo[e] = (_Float16)__builtin_fmaf(x[e], sf, -(float)hi[e]);
-    }
-}
-
-// The largest magnitude of N values. The three-operand maximum with magnitude modifiers is written out because fmaxf
-// costs a canonicalising instruction more per value. NaNs are passed over.
-template <int N>
-__device__ __forceinline__ float max_abs(const float *x) {
-    static_assert(N % 2 == 0, "pairs");
-    float m = 0.f;
-#pragma unroll
-    for (int e = 0; e < N; e += 2) asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(m) : "v"(x[e]), "v"(x[e + 1]), "v"(m));
-    return m;
-}
-// The bits of the largest of 64 non-negative values, wave-uniform (such floats order as their bits do).
-__device__ __forceinline__ int wave_max_bits(float m) {
-    m = fmaxf(m, dpp<0xB1>(m));
-    m = fmaxf(m, dpp<0x4E>(m));
-    m = fmaxf(m, dpp<0x141>(m));
-    m = fmaxf(m, dpp<0x140>(m));
-    const int v = __builtin_bit_cast(int, m);
-    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
-               max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
-}
-constexpr int kInfBits = 0x7f800000;
-
-__device__ __forceinline__ v4f mfma(v8h a, v8h b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-
 
 constexpr int kQG = 4, kKS = 2;                 // query groups and key halves: one wave each
 constexpr int kNW = kQG * kKS, kRows = 64;      // rows of a block of K, V or P; queries of a workgroup
@@ -376,17 +337,13 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
                 for (int t = 0; t < 3; ++t) {
                     const _Float16 *p = Ph + pbase[t] + c;
                     const v8h hi = *(const v8h *)p, lo = *(const v8h *)(p + kPlane);
-                    sp[t] = mfma(lo, qv[0][s], sp[t]);
-                    sp[t] = mfma(hi, qv[1][s], sp[t]);
-                    sp[t] = mfma(hi, qv[0][s], sp[t]);
+                    sp[t] = kea::mfma_split(hi, lo, qv[0][s], qv[1][s], sp[t]);
                 }
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
                     const _Float16 *p = Kh + (32 * ks + 16 * t + n) * kDK + c;
                     const v8h hi = *(const v8h *)p, lo = *(const v8h *)(p + kPlane);
-                    sc[t] = mfma(lo, qu[0][s], sc[t]);
-                    sc[t] = mfma(hi, qu[1][s], sc[t]);
-                    sc[t] = mfma(hi, qu[0][s], sc[t]);
+                    sc[t] = kea::mfma_split(hi, lo, qu[0][s], qu[1][s], sc[t]);
                 }
             }
             // the band scores of query n at relative positions 16 t + 4 g + r; key jj of the wave is position jj + 15 - n.
@@ -447,9 +404,7 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
             for (int d = 0; d < 8; ++d) {
                 const _Float16 *vp = Vh + (16 * d + n) * kRows + (((4 * ks + g) ^ (n >> 1)) * 8);
                 const v8h hi = *(const v8h *)vp, lo = *(const v8h *)(vp + kPlane);
-                o[d] = mfma(lo, ph, o[d]);
-                o[d] = mfma(hi, pl, o[d]);
-                o[d] = mfma(hi, ph, o[d]);
+                o[d] = kea::mfma_split(hi, lo, ph, pl, o[d]);
             }
         }
         if (kb + 1 < tiles) load_multipliers(kb + 1);

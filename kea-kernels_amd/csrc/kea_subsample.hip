@@ -1,0 +1,466 @@
+// The dw-striding subsampling of 128 mel bins at 256 channels in two launches, channels last, with the convolutions
+// that are contractions on the FP16 matrix cores at FP32 accuracy (kea_split.h):
+//   1. conv 3x3/2 (1 -> 256) + ReLU + depthwise 3x3/2 + pointwise 256 -> 256 + ReLU      [B][128][T] -> [B][T2][32][256]
+//   2. depthwise 3x3/2 + pointwise 256 -> 256 + ReLU                          [B][T2][32][256] -> [B][T3][16][256]
+// A workgroup makes all 256 channels of its positions, so a pointwise convolution's input never leaves LDS, where the same
+// layers as separate kernels (kea_subsample_front, a library GEMM, kea_dwconv2d_s2, a library GEMM, kea_bias_relu_flatten)
+// write and read [B][256][T2][32] three times and the FP32 GEMMs run at 1/16 of the FP16 rate. The first convolution is
+// itself one matrix product: its 9 taps times the three products of a split operand are 27 of a 32-deep MFMA's terms.
+//
+// Measured on eight 10-second clips (T = 1000): 54 + 24 us, where the five launches take 53 + 90 + 25 + 27 + 25 us; one
+// clip 15 + 12 us. Launch 1 executes 1850 vector instructions and 232 MFMAs a wave, and the two hardly overlap: about 27
+// and 12 us of its 54 at the clock it runs at, the rest waits between its phases. Two rows of 32 positions to a workgroup,
+// two workgroups to a CU, is the split that measured best: four rows (one workgroup to a CU, half the weight reads)
+// take 60 and, for one clip, 25 us. Launch 2 is latency: the weights (256 KB a workgroup) and its input from L2; half the
+// rows to a workgroup take 37 us, as the weights are read twice as often.
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <string>
+
+#include "kea_internal.h"
+#include "kea_split.h"
+#include "../../include/kea_encoder.h"
+
+namespace {
+
+using kea::exponent_of;
+using kea::kInfBits;
+using kea::mfma_f16;
+using kea::mfma_split;
+using kea::pow2;
+using kea::split1;
+using kea::v4f;
+using kea::v8h;
+
+constexpr int kC = 256, kF = 128, kF1 = 64, kF2 = 32, kF3 = 16;
+constexpr int kWaves = 8, kThreads = 64 * kWaves;
+
+// max(x, 0) of an x that is not a NaN, on the bits (fmaxf would canonicalise an MFMA's result first).
+__device__ __forceinline__ float relu(float x) { return __builtin_bit_cast(float, max(__builtin_bit_cast(int, x), 0)); }
+
+// The pointwise product of a tile of positions: D[n][m] = sum_k W[n][k] x[m][k] over the LDS tile x (hi and lo planes
+// [MT * 16][256], 16-byte units XOR-swizzled by row), wave w taking output channels 32 w .. 32 w + 31. W: the fragments
+// [n-tile][k-step][plane][lane][8] of split weights, read from L2 two k-steps ahead of their products (the first two
+// before the tile is complete). acc[nt][mt]: rows n = 4 (lane / 16) + r, column m = lane % 16.
+struct Weights {
+    const _Float16 *at;
+    v8h f[3][2][2];  // [k-step % 3][n-tile][plane]
+    __device__ __forceinline__ void load(int ks) {
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+            for (int p = 0; p < 2; ++p) f[ks % 3][nt][p] = *(const v8h *)(at + ((nt * 8 + ks) * 2 + p) * 64 * 8);
+    }
+    __device__ __forceinline__ void start(const _Float16 *w, int wave, int lane) {
+        at = w + ((long long)(2 * wave) * 8 * 2 * 64 + lane) * 8;
+        load(0);
+        load(1);
+    }
+};
+template <int MT>
+__device__ __forceinline__ void pointwise(const _Float16 *tile, Weights &w, int lane, v4f (&acc)[2][MT]) {
+    const int i = lane & 15, g = lane >> 4;
+    constexpr int PLANE = MT * 16 * kC;
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+        if (ks + 2 < 8) w.load(ks + 2);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const _Float16 *p = tile + (mt * 16 + i) * kC + (((4 * ks + g) ^ i) * 8);
+            const v8h hi = *(const v8h *)p, lo = *(const v8h *)(p + PLANE);
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+                acc[nt][mt] = mfma_split(w.f[ks % 3][nt][0], w.f[ks % 3][nt][1], hi, lo, acc[nt][mt]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// 3x3/2 taps of output position (r, c) read input rows 2 r - 1 + ky and columns 2 c - 1 + kx (padding 1).
+
+// Launch 1: a workgroup = one clip's output rows t2 = 2 blockIdx.x and + 1, all 32 columns and 256 channels.
+constexpr int kMinExponent = -50;
+constexpr int kRows2 = 2, kPos1 = kRows2 * kF2;              // positions of a tile: 64, m = 32 q + f2
+constexpr int kRows1 = 2 * kRows2 + 1, kPatchR = 2 * kRows1 + 1, kPatchC = kF + 2;
+constexpr int kPatch = kPatchR * kPatchC;                    // input rows 4 t2 - 3 .., columns -1 .. 128
+constexpr int kTile1 = 2 * kPos1 * kC * 2;                   // bytes of the split tile (the first convolution's operand
+                                                             // fragments, kRows1 x 4 KB, lie there before it)
+constexpr int kLds1Patch = kTile1, kLds1Max = kLds1Patch + (2 * kPatch + 8) * 2 / 16 * 16 + 16;
+constexpr int kLds1Scale = kLds1Max + kWaves * kPos1 * 4, kLds1Bytes = kLds1Scale + kPos1 * 4 + 32;
+
+__global__ void __launch_bounds__(kThreads, 4)
+subsample1_kernel(const float *x, int T, int T1, int T2, const _Float16 *w1f, const float *w1m, const float *w1,
+                  const float *b1, const float *w2, const float *b2, const _Float16 *w3f, const float *w3m, const float *w3,
+                  const float *b3, float *y) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15, g = lane >> 4;
+    const int b = blockIdx.y, t2a = blockIdx.x * kRows2, r0 = 4 * t2a - 3;
+    const float *xb = x + (long long)b * kF * T;
+    _Float16 *const tile = (_Float16 *)lds, *const patch = (_Float16 *)(lds + kLds1Patch);
+    float *const pmax = (float *)(lds + kLds1Max), *const pscale = (float *)(lds + kLds1Scale);
+    int *const top = (int *)(lds + kLds1Scale + kPos1 * 4);
+
+    // the weights of the wave's 32 channels, two per lane (32 wave + 2 i + e)
+    const int ch2 = 32 * wave + 2 * i;
+    const v8h wf[2] = {*(const v8h *)(w1f + (2 * wave * 64 + lane) * 8), *(const v8h *)(w1f + ((2 * wave + 1) * 64 + lane) * 8)};
+    const float2 m1 = *(const float2 *)(w1m + ch2), first = *(const float2 *)(b1 + ch2), second = *(const float2 *)(b2 + ch2);
+    float2 taps[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) taps[k] = *(const float2 *)(w2 + k * kC + ch2);
+
+    // the input patch, split with one scale for the tile
+    constexpr int PN = (kPatch + kThreads - 1) / kThreads;
+    float px[PN];
+    float m = 0.f;
+    bool plain = false;
+#pragma unroll
+    for (int u = 0; u < PN; ++u) {
+        const int e = u * kThreads + tid, c = e / kPatchR, r = e - c * kPatchR, t = r0 + r;  // time runs fastest in x
+        px[u] = e < kPatch && t >= 0 && t < T && c >= 1 && c <= kF ? xb[(long long)(c - 1) * T + t] : 0.f;
+        m = kea::max_abs2(px[u], 0.f, m);
+        plain = plain || px[u] != px[u];
+    }
+    const int wtop = kea::wave_max_bits(m);
+    if (lane == 0) top[wave] = wtop;
+    __syncthreads();
+    int bits = top[0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) bits = max(bits, top[w]);
+    // a tile of zeros has the smallest scale; one of smaller values than that is summed in FP32, as NaNs and infinities are
+    const int xe = max(exponent_of(bits), kMinExponent);
+    plain = plain || bits >= kInfBits || (bits != 0 && exponent_of(bits) < kMinExponent);
+#pragma unroll
+    for (int u = 0; u < PN; ++u) {
+        const int e = u * kThreads + tid, c = e / kPatchR, r = e - c * kPatchR;
+        _Float16 hi, lo;
+        split1(px[u], pow2(14 - xe), hi, lo);
+        if (e < kPatch) {
+            patch[r * kPatchC + c] = hi;
+            patch[kPatch + r * kPatchC + c] = lo;
+        }
+    }
+    if (tid == 0) patch[2 * kPatch] = (_Float16)0.f;
+    __syncthreads();
+    // operand fragments [row t1][16 columns f1] of the first convolution: term k = 8 g + j of a lane is tap k % 9 of
+    // x hi (k < 9, against the weights' hi), x lo (< 18, hi) and x hi (< 27, against lo)
+    {
+        int at[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int k = 8 * g + j, part = k / 9, tap = k - 9 * part;
+            at[j] = k < 27 ? (part == 1 ? kPatch : 0) + tap / 3 * kPatchC + tap % 3 : -1;
+        }
+        for (int f = wave; f < kRows1 * 4; f += kWaves) {
+            const int base = 2 * (f >> 2) * kPatchC + 2 * (16 * (f & 3) + i);
+            v8h v;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = patch[at[j] < 0 ? 2 * kPatch : base + at[j]];
+            *(v8h *)(tile + (f * 64 + lane) * 8) = v;
+        }
+    }
+    __syncthreads();
+
+    // the first convolution's rows in order, each accumulated into the depthwise outputs it belongs to. o[e][q][j][s]: row t2a + q, column 8 j + 2 g + s.
+    // The first convolution stays in the units of its operands, m1 * 2^(xe - 14): its bias is divided by them, the
+    // depthwise weights multiplied.
+    float o[2][kRows2][4][2], dw[2][9], bias1[2];
+    const float mul[2] = {m1.x * pow2(xe - 14), m1.y * pow2(xe - 14)};
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        dw[0][k] = taps[k].x * mul[0];
+        dw[1][k] = taps[k].y * mul[1];
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        bias1[e] = (e ? first.y : first.x) * __builtin_amdgcn_rcpf(e ? m1.y : m1.x) * pow2(14 - xe);  // (m1: powers of two)
+#pragma unroll
+        for (int q = 0; q < kRows2; ++q)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[e][q][j][0] = o[e][q][j][1] = e ? second.y : second.x;
+    }
+#pragma unroll
+    for (int rr = 0; rr < kRows1; ++rr) {
+        const int t1 = 2 * t2a - 1 + rr;
+        v8h xf[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) xf[j] = *(const v8h *)(tile + ((rr * 4 + j) * 64 + lane) * 8);
+        if (t1 >= 0 && t1 < T1) {  // the same for the whole workgroup; a row of the padding adds nothing
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                float v[4][4], before[4], turned[4];  // columns 16 j + 4 g + r, and the column before each four
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const v4f d = mfma_f16(xf[j], wf[e], (v4f){bias1[e], bias1[e], bias1[e], bias1[e]});
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[j][r] = relu(d[r]);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) turned[j] = __shfl(v[j][3], (lane + 48) & 63, 64);  // group g - 1's last column
+#pragma unroll
+                for (int j = 0; j < 4; ++j) before[j] = g > 0 ? turned[j] : j > 0 ? turned[j - 1] : 0.f;
+#pragma unroll
+                for (int q = 0; q < kRows2; ++q) {
+                    const int dy = rr - 2 * q;
+                    if (dy < 0 || dy > 2) continue;
+                    const float a = dw[e][3 * dy], c = dw[e][3 * dy + 1], d = dw[e][3 * dy + 2];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        float u0 = o[e][q][j][0], u1 = o[e][q][j][1];
+                        u0 = __builtin_fmaf(d, v[j][1], __builtin_fmaf(c, v[j][0], __builtin_fmaf(a, before[j], u0)));
+                        u1 = __builtin_fmaf(d, v[j][3], __builtin_fmaf(c, v[j][2], __builtin_fmaf(a, v[j][1], u1)));
+                        o[e][q][j][0] = u0;
+                        o[e][q][j][1] = u1;
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // each position's largest magnitude over the channels: 16 lanes here, the waves through LDS
+#pragma unroll
+    for (int q = 0; q < kRows2; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const float top16 = kea::max16(kea::max_abs2(o[0][q][j][s], o[1][q][j][s], 0.f));
+                if (i == 0) pmax[wave * kPos1 + 32 * q + 8 * j + 2 * g + s] = top16;
+            }
+    __syncthreads();
+    int big = 0;
+    if (tid < kPos1) {
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) big = max(big, __builtin_bit_cast(int, pmax[w * kPos1 + tid]));
+        pscale[tid] = pow2(14 - exponent_of(big));
+    }
+    plain = __syncthreads_or(plain || big >= kInfBits) != 0;
+    const int rows = min(kRows2, T2 - t2a);
+    float *const yb = y + ((long long)b * T2 + t2a) * kF2 * kC;
+    if (plain) {  // the same sums in FP32, a thread per channel
+        float *const h = (float *)lds;  // [kPos1][256]
+        const int c = tid & (kC - 1);
+        for (int p = tid >> 8; p < rows * kF2; p += kThreads / kC) {
+            const int t2 = t2a + p / kF2, f2 = p % kF2;
+            float acc = b2[c];
+            for (int dy = 0; dy < 3; ++dy)
+                for (int dx = 0; dx < 3; ++dx) {
+                    const int t1 = 2 * t2 - 1 + dy, f1 = 2 * f2 - 1 + dx;
+                    float a = 0.f;
+                    if (t1 >= 0 && t1 < T1 && f1 >= 0 && f1 < kF1) {
+                        a = b1[c];
+                        for (int k = 0; k < 9; ++k) {
+                            const int t = 2 * t1 - 1 + k / 3, f = 2 * f1 - 1 + k % 3;
+                            a = __builtin_fmaf(w1[k * kC + c], t >= 0 && t < T && f >= 0 && f < kF ? xb[(long long)f * T + t] : 0.f, a);
+                        }
+                        a = fmaxf(a, 0.f);
+                    }
+                    acc = __builtin_fmaf(w2[(dy * 3 + dx) * kC + c], a, acc);
+                }
+            h[p * kC + c] = acc;
+        }
+        __syncthreads();
+        for (int p = tid >> 8; p < rows * kF2; p += kThreads / kC) {
+            float acc = 0.f;
+            for (int k = 0; k < kC; ++k) acc = __builtin_fmaf(w3[c * kC + k], h[p * kC + k], acc);
+            yb[p * kC + c] = fmaxf(acc + b3[c], 0.f);
+        }
+        return;
+    }
+    Weights weights;
+    weights.start(w3f, wave, lane);
+    // the split tile (all waves are past the fragments): two channels of a position are one word
+#pragma unroll
+    for (int q = 0; q < kRows2; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int p = 32 * q + 8 * j + 2 * g + s, ch = 32 * wave + 2 * i;
+                const float sf = pscale[p];
+                typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+                _Float16 h0, l0, h1, l1;
+                split1(o[0][q][j][s], sf, h0, l0);
+                split1(o[1][q][j][s], sf, h1, l1);
+                _Float16 *dst = tile + p * kC + (((ch >> 3) ^ (p & 15)) * 8) + (ch & 7);
+                *(v2h *)dst = (v2h){h0, h1};
+                *(v2h *)(dst + kPos1 * kC) = (v2h){l0, l1};
+            }
+    __syncthreads();
+    v4f acc[2][kPos1 / 16];
+    pointwise<kPos1 / 16>(tile, weights, lane, acc);
+    // D[n][m]: a lane holds four consecutive output channels of a position
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+        const int n = 32 * wave + 16 * nt + 4 * g;
+        const float4 wm = *(const float4 *)(w3m + n), bias = *(const float4 *)(b3 + n);
+#pragma unroll
+        for (int mt = 0; mt < kPos1 / 16; ++mt) {
+            const int p = 16 * mt + i;
+            const float pm = 1.0f / pscale[p];  // a power of two: exact
+            const v4f d = acc[nt][mt];
+            if (p < rows * kF2)
+                *(float4 *)(yb + p * kC + n) = make_float4(fmaxf(__builtin_fmaf(d[0], wm.x * pm, bias.x), 0.f),
+                                                           fmaxf(__builtin_fmaf(d[1], wm.y * pm, bias.y), 0.f),
+                                                           fmaxf(__builtin_fmaf(d[2], wm.z * pm, bias.z), 0.f),
+                                                           fmaxf(__builtin_fmaf(d[3], wm.w * pm, bias.w), 0.f));
+        }
+    }
+}
+
+// Launch 2: a workgroup = one clip's output rows t3 = 4 blockIdx.x .. + 3, all 16 columns and 256 channels; a lane
+// takes four channels.
+constexpr int kRows3 = 4, kPos2 = kRows3 * kF3, kCols3 = kPos2 / kWaves;  // 64 positions, 8 to a wave's depthwise
+constexpr int kTile2 = 2 * kPos2 * kC * 2, kLds2Bytes = kTile2 + kPos2 * 4 + 16;
+
+__global__ void __launch_bounds__(kThreads)
+subsample2_kernel(const float *x, int T2, int T3, const float *w5, const float *b5, const _Float16 *w6f, const float *w6m,
+                  const float *w6, const float *b6, float *y) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15, g = lane >> 4;
+    const int b = blockIdx.y, t3a = blockIdx.x * kRows3;
+    const float *xb = x + (long long)b * T2 * kF2 * kC;
+    _Float16 *const tile = (_Float16 *)lds;
+    float *const pscale = (float *)(lds + kTile2);
+    float4 wt[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) wt[k] = *(const float4 *)(w5 + k * kC + 4 * lane);
+    const float4 bias = *(const float4 *)(b5 + 4 * lane);
+    // depthwise: columns f0 .. f0 + kCols3 - 1 of row q; every input column is loaded once
+    const int q = wave / (kF3 / kCols3), f0 = kCols3 * (wave % (kF3 / kCols3)), t3 = t3a + q;
+    bool plain = false;
+    float o[kCols3][4];
+#pragma unroll
+    for (int c = 0; c < kCols3; ++c) {
+        o[c][0] = bias.x, o[c][1] = bias.y, o[c][2] = bias.z, o[c][3] = bias.w;
+    }
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy) {
+        const int t2 = 2 * t3 - 1 + dy;
+        const bool row = t2 >= 0 && t2 < T2;
+        const float *src = xb + ((long long)(row ? t2 : 0) * kF2) * kC + 4 * lane;
+        float4 v[2 * kCols3 + 1];
+#pragma unroll
+        for (int c = 0; c < 2 * kCols3 + 1; ++c) {  // input columns 2 f0 - 1 + c
+            const int f2 = 2 * f0 - 1 + c;
+            v[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (row && f2 >= 0) v[c] = *(const float4 *)(src + f2 * kC);
+        }
+#pragma unroll
+        for (int c = 0; c < kCols3; ++c)
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx) {
+                const float4 a = v[2 * c + dx];
+                const float4 w = wt[3 * dy + dx];
+                o[c][0] = __builtin_fmaf(w.x, a.x, o[c][0]);
+                o[c][1] = __builtin_fmaf(w.y, a.y, o[c][1]);
+                o[c][2] = __builtin_fmaf(w.z, a.z, o[c][2]);
+                o[c][3] = __builtin_fmaf(w.w, a.w, o[c][3]);
+            }
+    }
+#pragma unroll
+    for (int c = 0; c < kCols3; ++c) {
+        const int p = 16 * q + f0 + c;
+        const int bits = kea::wave_max_bits(kea::max_abs<4>(o[c]));
+        plain = plain || bits >= kInfBits;
+        const int e = exponent_of(bits);
+        typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+        v4h hi, lo;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            _Float16 h, l;
+            split1(o[c][k], pow2(14 - e), h, l);
+            hi[k] = h;
+            lo[k] = l;
+        }
+        _Float16 *dst = tile + p * kC + (((lane >> 1) ^ (p & 15)) * 8) + (lane & 1) * 4;
+        *(v4h *)dst = hi;
+        *(v4h *)(dst + kPos2 * kC) = lo;
+        if (lane == 0) pscale[p] = pow2(e - 14);
+    }
+    Weights weights;
+    weights.start(w6f, wave, lane);
+    plain = __syncthreads_or(plain) != 0;
+    const int rows = min(kRows3, T3 - t3a);
+    float *const yb = y + ((long long)b * T3 + t3a) * kF3 * kC;
+    if (plain) {  // an infinity: the same sums in FP32
+        float *const h = (float *)lds;  // [kPos2][256]
+#pragma unroll
+        for (int c = 0; c < kCols3; ++c)
+            *(float4 *)(h + (16 * q + f0 + c) * kC + 4 * lane) = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
+        __syncthreads();
+        const int c = tid & (kC - 1);
+        for (int p = tid >> 8; p < rows * kF3; p += kThreads / kC) {
+            float acc = 0.f;
+            for (int k = 0; k < kC; ++k) acc = __builtin_fmaf(w6[c * kC + k], h[p * kC + k], acc);
+            yb[p * kC + c] = fmaxf(acc + b6[c], 0.f);
+        }
+        return;
+    }
+    v4f acc[2][kPos2 / 16];
+    pointwise<kPos2 / 16>(tile, weights, lane, acc);
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+        const int n = 32 * wave + 16 * nt + 4 * g;
+        const float4 wm = *(const float4 *)(w6m + n), bs = *(const float4 *)(b6 + n);
+#pragma unroll
+        for (int mt = 0; mt < kPos2 / 16; ++mt) {
+            const int p = 16 * mt + i;
+            const float pm = pscale[p];
+            const v4f d = acc[nt][mt];
+            if (p < rows * kF3)
+                *(float4 *)(yb + p * kC + n) = make_float4(fmaxf(__builtin_fmaf(d[0], wm.x * pm, bs.x), 0.f),
+                                                           fmaxf(__builtin_fmaf(d[1], wm.y * pm, bs.y), 0.f),
+                                                           fmaxf(__builtin_fmaf(d[2], wm.z * pm, bs.z), 0.f),
+                                                           fmaxf(__builtin_fmaf(d[3], wm.w * pm, bs.w), 0.f));
+        }
+    }
+}
+
+int launched(const char *what) {
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? KEA_OK : kea::fail((int)e, std::string(what) + " launch failed: " + hipGetErrorString(e));
+}
+template <class Fn>
+int allow_lds(Fn fn, int bytes) {
+    const hipError_t e = hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    return e == hipSuccess ? KEA_OK : kea::fail((int)e, std::string("LDS attribute refused: ") + hipGetErrorString(e));
+}
+
+}  // namespace
+
+extern "C" int kea_subsample_stage1(const float *x, int64_t batch, int64_t t, const void *w1f, const float *w1m,
+                                    const float *w1, const float *b1, const float *w2, const float *b2, const void *w3f,
+                                    const float *w3m, const float *w3, const float *b3, float *y, void *stream) {
+    if (batch < 0 || batch > 65535 || t < 1 || t > INT32_MAX / 4) return kea::fail(KEA_EINVAL, "bad sizes");
+    if (batch == 0) return KEA_OK;
+    if (!x || !w1f || !w1m || !w1 || !b1 || !w2 || !b2 || !w3f || !w3m || !w3 || !b3 || !y)
+        return kea::fail(KEA_EINVAL, "null pointer");
+    if (((uintptr_t)w1f | (uintptr_t)w1m | (uintptr_t)b1 | (uintptr_t)w2 | (uintptr_t)b2 | (uintptr_t)w3f | (uintptr_t)w3m | (uintptr_t)b3 | (uintptr_t)y) & 15)
+        return kea::fail(KEA_EALIGN, "every operand but x, w1 and w3 must be 16-byte aligned");
+    const int t1 = (int)((t - 1) / 2 + 1), t2 = (t1 - 1) / 2 + 1;
+    if (const int rc = allow_lds(subsample1_kernel, kLds1Bytes)) return rc;
+    hipLaunchKernelGGL(subsample1_kernel, dim3((unsigned)((t2 + kRows2 - 1) / kRows2), (unsigned)batch), dim3(kThreads),
+                       kLds1Bytes, (hipStream_t)stream, x, (int)t, t1, t2, (const _Float16 *)w1f, w1m, w1, b1, w2, b2,
+                       (const _Float16 *)w3f, w3m, w3, b3, y);
+    return launched("subsample stage 1");
+}
+
+extern "C" int kea_subsample_stage2(const float *x, int64_t batch, int64_t t2, const float *w5, const float *b5,
+                                    const void *w6f, const float *w6m, const float *w6, const float *b6, float *y,
+                                    void *stream) {
+    if (batch < 0 || batch > 65535 || t2 < 1 || t2 > INT32_MAX / 4) return kea::fail(KEA_EINVAL, "bad sizes");
+    if (batch == 0) return KEA_OK;
+    if (!x || !w5 || !b5 || !w6f || !w6m || !w6 || !b6 || !y) return kea::fail(KEA_EINVAL, "null pointer");
+    if (((uintptr_t)x | (uintptr_t)w5 | (uintptr_t)b5 | (uintptr_t)w6f | (uintptr_t)w6m | (uintptr_t)b6 | (uintptr_t)y) & 15)
+        return kea::fail(KEA_EALIGN, "every operand but w6 must be 16-byte aligned");
+    const int t3 = (int)((t2 - 1) / 2 + 1);
+    if (const int rc = allow_lds(subsample2_kernel, kLds2Bytes)) return rc;
+    hipLaunchKernelGGL(subsample2_kernel, dim3((unsigned)((t3 + kRows3 - 1) / kRows3), (unsigned)batch), dim3(kThreads),
+                       kLds2Bytes, (hipStream_t)stream, x, (int)t2, t3, w5, b5, (const _Float16 *)w6f, w6m, w6, b6, y);
+    return launched("subsample stage 2");
+}

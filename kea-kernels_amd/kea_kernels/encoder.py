@@ -472,6 +472,63 @@ class _Norm:
         self.normalized_shape = (weight.numel(),)
 
 
+def _split_f16(w: Tensor, least: int = -90) -> tuple:
+    """FP32 rows [n, k] as two FP16 planes: w[i] = (hi[i] + lo[i]) * 2^(e[i] - 14), 2^e[i] the power of two under the
+    row's largest magnitude (clamped to [2^least, 2^127]). Returns hi, lo and 2^(e - 14), exactly."""
+    e = ((w.abs().amax(1).view(torch.int32) >> 23) - 127).clamp(least, 127)
+    z = w * ((14 - e + 127) << 23).view(torch.float32)[:, None]
+    hi = z.half()
+    return hi, (z - hi.float()).half(), ((e - 14 + 127) << 23).view(torch.float32)
+
+
+def _fragments(planes: list) -> Tensor:
+    """Matrices [n, k] of FP16 as MFMA operands [n / 16][k / 32][plane][64 lanes][8]: lane 16 g + i holds row i,
+    columns 8 g .. 8 g + 7."""
+    return torch.stack([w.view(w.shape[0] // 16, 16, w.shape[1] // 32, 4, 8).permute(0, 2, 3, 1, 4) for w in planes],
+                       2).contiguous()
+
+
+class _SplitSubsampling:
+    """The subsampling weights as kea_subsample_stage1 / stage2 read them, laid out once per encoder: the pointwise
+    convolutions as split FP16 fragments, the first convolution's nine taps as the 27 terms (hi, hi, lo against the
+    input's hi, lo, hi) of one 32-deep product with channels 32 w + 2 i + e in fragment 2 w + e, and the output
+    linear's columns in (frequency, channel) order."""
+
+    LEAST = -30  # the exponent below which a row of the first convolution is not split (unless it is zero)
+
+    def __init__(self, s: dict, gain: float):
+        c = 256
+        self.w1, self.b1 = s["conv.0.weight"].reshape(c, 9).t().contiguous(), s["conv.0.bias"].contiguous()
+        self.w2, self.b2 = s["conv.2.weight"].reshape(c, 9).t().contiguous(), s["conv.2.bias"].contiguous()
+        self.w3, self.b3 = s["conv.3.weight"].reshape(c, c).contiguous(), s["conv.3.bias"].contiguous()
+        self.w5, self.b5 = s["conv.5.weight"].reshape(c, 9).t().contiguous(), s["conv.5.bias"].contiguous()
+        self.w6, self.b6 = s["conv.6.weight"].reshape(c, c).contiguous(), s["conv.6.bias"].contiguous()
+        hi, lo, self.m1 = _split_f16(s["conv.0.weight"].reshape(c, 9), _SplitSubsampling.LEAST)
+        terms = torch.cat([hi, hi, lo, torch.zeros_like(hi[:, :5])], 1)
+        self.f1 = terms.view(8, 16, 2, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
+        hi, lo, self.m3 = _split_f16(self.w3)
+        self.f3 = _fragments([hi, lo])
+        hi, lo, self.m6 = _split_f16(self.w6)
+        self.f6 = _fragments([hi, lo])
+        d = s["out.weight"].shape[0]
+        self.out = ((s["out.weight"] * gain).view(d, c, 16).transpose(1, 2).reshape(d, 16 * c).contiguous(),
+                    (s["out.bias"] * gain).contiguous())
+
+    @staticmethod
+    def prepare(s: dict, cfg: EncoderConfig):
+        """The layout, or None where the kernels do not take the model: they are written for 128 mel bins and 256
+        channels, a weight that is not finite has no split form, and the first convolution's bias is held in units of
+        its weights (nonzero rows from 2^-30, biases to 2^15, so that it stays finite for any scale of the input)."""
+        if cfg.feat_in != 128 or cfg.sub_channels != 256 or s["out.weight"].shape[1] != 16 * 256:
+            return None
+        if not all(bool(torch.isfinite(v).all()) for v in s.values()):
+            return None
+        top = s["conv.0.weight"].reshape(256, 9).abs().amax(1)
+        if bool(((top > 0) & (top < 2.0**_SplitSubsampling.LEAST)).any()) or bool((s["conv.0.bias"].abs() > 2**15).any()):
+            return None
+        return _SplitSubsampling(s, math.sqrt(cfg.d_model) if cfg.xscaling else 1.0)
+
+
 class FastConformerEncoder:
     """audio [B, S] -> encoder output [B, T', d]. parts = int8 activation parts of every quantized linear (1 = the
     Kea-B x1 mode); dense=True swaps the quantized linears for FP32 dense matmuls (the parity reference);
@@ -490,6 +547,7 @@ class FastConformerEncoder:
         dev = lambda t: t.to(device=device, dtype=torch.float32)  # noqa: E731
         p = "encoder.pre_encode."
         self.sub = {k[len(p):]: dev(v) for k, v in weights.items() if k.startswith(p)}
+        self._sub_split = _SplitSubsampling.prepare(self.sub, cfg) if self.fused and device.type == "cuda" else None
         self.layers = []
         self._pos_cache: dict = {}
         self._att_ws: dict = {}  # (batch, t) -> key-split attention workspace (or None)
@@ -583,7 +641,9 @@ class FastConformerEncoder:
     def subsample(self, feats: Tensor) -> Tensor:
         """[B, mels, frames] -> [B, T', d] (dw-striding x8, then the output linear).
 
-        Fused (quantized) path: the first convolution + ReLU + first depthwise convolution in one kernel
+        Fused (quantized) path, 128 mel bins and 256 channels: two launches up to the flattened features
+        (kea_subsample_stage1, kea_subsample_stage2; weights laid out when the encoder is made) and the output linear as
+        one matrix product. Other sizes: the first convolution + ReLU + first depthwise convolution in one kernel
         (kea_subsample_front), the pointwise convolutions as batched matrix products whose bias + ReLU are applied
         by the next kernel on load, the second depthwise convolution (kea_dwconv2d_s2), the last bias + ReLU with the
         (channel, frequency) flatten (kea_bias_relu_flatten), and the output linear as one matrix product. Otherwise
@@ -607,6 +667,8 @@ class FastConformerEncoder:
         s, c = self.sub, self.cfg.sub_channels
         feats = feats.contiguous()
         b, f, t = feats.shape
+        if self._sub_split is not None and f == 128 and 1 <= t < 1 << 29 and b < 1 << 16 and feats.dtype == torch.float32:
+            return self._subsample_split(feats)
         t1, f1 = (t - 1) // 2 + 1, (f - 1) // 2 + 1
         t2, f2 = (t1 - 1) // 2 + 1, (f1 - 1) // 2 + 1
         t3, f3 = (t2 - 1) // 2 + 1, (f2 - 1) // 2 + 1
@@ -628,6 +690,22 @@ class FastConformerEncoder:
             g = math.sqrt(self.cfg.d_model) if self.cfg.xscaling else 1.0
             self._sub_out = ((s["out.weight"] * g).contiguous(), (s["out.bias"] * g).contiguous())
         return F.linear(flat, *self._sub_out)
+
+    def _subsample_split(self, feats: Tensor) -> Tensor:
+        w, (b, _, t) = self._sub_split, feats.shape
+        t2 = ((t - 1) // 2) // 2 + 1
+        t3 = (t2 - 1) // 2 + 1
+        L, st = _hip.lib(), _hip.stream_handle(feats.device)
+        x1 = torch.empty(b, t2, 32, 256, device=feats.device, dtype=torch.float32)
+        _hip.check(L.kea_subsample_stage1(feats.data_ptr(), b, t, w.f1.data_ptr(), w.m1.data_ptr(), w.w1.data_ptr(),
+                                          w.b1.data_ptr(), w.w2.data_ptr(), w.b2.data_ptr(), w.f3.data_ptr(),
+                                          w.m3.data_ptr(), w.w3.data_ptr(), w.b3.data_ptr(), x1.data_ptr(), st),
+                   "kea_subsample_stage1")
+        flat = torch.empty(b, t3, 16 * 256, device=feats.device, dtype=torch.float32)
+        _hip.check(L.kea_subsample_stage2(x1.data_ptr(), b, t2, w.w5.data_ptr(), w.b5.data_ptr(), w.f6.data_ptr(),
+                                          w.m6.data_ptr(), w.w6.data_ptr(), w.b6.data_ptr(), flat.data_ptr(), st),
+                   "kea_subsample_stage2")
+        return F.linear(flat, *w.out)
 
     def positions(self, t: int) -> list:
         """W_pos applied to the relative encodings, per layer, for length t: [2t-1, d] each. Frozen per length

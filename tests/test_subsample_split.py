@@ -1,0 +1,112 @@
+"""The split-FP16 subsampling (kea_subsample_stage1 / stage2) against FP64 at the edges of its tiles: single frames, output
+rows that end inside a tile of four, several clips; infinities and NaN take the plain FP32 sums of the general kernels."""
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from kea_kernels import encoder as E
+
+FRAMES = [1, 2, 3, 5, 8, 13, 16, 17, 31, 32, 33, 36, 37, 63, 65, 129, 257, 1000]
+
+
+def model():
+    cfg = E.EncoderConfig(layers=1)
+    return E.FastConformerEncoder(E.synthetic_weights(cfg, seed=4), cfg, "cuda", parts=1)
+
+
+def exact(enc, feats):
+    s, c = {k: v.double().cpu() for k, v in enc.sub.items()}, enc.cfg.sub_channels
+    x = feats.double().cpu().transpose(1, 2).unsqueeze(1)
+    x = F.relu(F.conv2d(x, s["conv.0.weight"], s["conv.0.bias"], stride=2, padding=1))
+    for i in (2, 5):
+        x = F.conv2d(x, s[f"conv.{i}.weight"], s[f"conv.{i}.bias"], stride=2, padding=1, groups=c)
+        x = F.relu(F.conv2d(x, s[f"conv.{i + 1}.weight"], s[f"conv.{i + 1}.bias"]))
+    b, _, t, f = x.shape
+    return F.linear(x.transpose(1, 2).reshape(b, t, c * f), s["out.weight"], s["out.bias"]) * math.sqrt(enc.cfg.d_model)
+
+
+def general(enc, feats):
+    split, enc._sub_split = enc._sub_split, None
+    try:
+        return enc._subsample_fused(feats)
+    finally:
+        enc._sub_split = split
+
+
+@pytest.mark.parametrize("n,k", [(16, 32), (256, 256)])
+def test_split_weights_hold_fp32(n, k):
+    """hi + lo is the weight to 2^-22 of itself or 2^-39 of its row's largest, and the fragments are a permutation."""
+    g = torch.Generator().manual_seed(n)
+    w = torch.randn(n, k, generator=g) * torch.exp(3 * torch.randn(n, k, generator=g)) * 2.0 ** torch.randint(-80, 80, (n, 1), generator=g)
+    hi, lo, m = E._split_f16(w)
+    back = (hi.double() + lo.double()) * m.double()[:, None]
+    bound = torch.maximum(w.double().abs() * 2.0**-22, w.double().abs().amax(1, keepdim=True) * 2.0**-39)
+    assert bool(((back - w.double()).abs() <= bound).all())
+    f = E._fragments([hi, lo])
+    i, ks, gq = 5, k // 32 - 1, 3
+    assert torch.equal(f[0, ks, 1, gq, i], lo[i, 32 * ks + 8 * gq:32 * ks + 8 * gq + 8])
+    assert torch.equal(f.reshape(-1).view(torch.int16).sort()[0],
+                       torch.cat([hi, lo]).reshape(-1).view(torch.int16).sort()[0])
+
+
+@pytest.mark.parametrize("change,taken", [(None, True), ("inf", False), ("nan", False), ("tiny_row", False), ("zero_row", True),
+                                          ("bias", False), ("channels", False)])
+def test_models_that_are_taken(change, taken):
+    """What has no split form, or is of another size, stays on the general kernels."""
+    cfg = E.EncoderConfig(layers=1, sub_channels=128 if change == "channels" else 256)
+    p = "encoder.pre_encode."
+    s = {k[len(p):]: v.float().clone() for k, v in E.synthetic_weights(cfg, seed=4).items() if k.startswith(p)}
+    if change in ("inf", "nan"):
+        s["conv.3.weight"].view(-1)[7] = float(change)
+    elif change in ("tiny_row", "zero_row"):
+        s["conv.0.weight"][5] = 1e-10 if change == "tiny_row" else 0.0
+    elif change == "bias":
+        s["conv.0.bias"][9] = 1e5
+    assert (E._SplitSubsampling.prepare(s, cfg) is not None) == taken
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,frames", [(1 + i % 3, t) for i, t in enumerate(FRAMES)])
+@torch.inference_mode()
+def test_matches_exact(b, frames):
+    """FP32 accuracy. Every operand is held to 2^-22 and sums are FP32: the root mean square error is the general
+    kernels' within a quarter (the output linear, an FP32 sum of 4096 terms that both share, is most of it), and no
+    element is off by more than the 1e-5 of the largest output that the general kernels are held to."""
+    enc = model()
+    assert enc._sub_split is not None
+    feats = torch.randn(b, 128, frames, generator=torch.Generator().manual_seed(frames)).cuda()
+    want, got, old = exact(enc, feats), enc.subsample(feats).double().cpu(), general(enc, feats).double().cpu()
+    assert got.shape == want.shape == old.shape
+    top = float(want.abs().max())
+    rms, rms_old = ((got - want).square().mean().sqrt() / top, (old - want).square().mean().sqrt() / top)
+    print(b, frames, float(rms), float(rms_old), float((got - want).abs().max()) / top)
+    assert float((got - want).abs().max()) < 1e-5 * top and rms <= 1.25 * rms_old
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1e-30, 1e-6, 1e6, 1e30])
+@torch.inference_mode()
+def test_any_magnitude(scale):
+    """Power-of-two scales per tile and position: accuracy does not depend on the size of the features."""
+    enc = model()
+    feats = (torch.randn(2, 128, 50, generator=torch.Generator().manual_seed(1)) * scale).cuda()
+    want, got = exact(enc, feats), enc.subsample(feats).double().cpu()
+    assert float((got - want).abs().max() / want.abs().max()) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan"), 3e38])
+@torch.inference_mode()
+def test_special_values_as_general(value):
+    """An infinite, NaN or near-overflow feature gives what the general kernels give: the same elements finite, and those
+    close; the rest the same kind."""
+    enc = model()
+    feats = torch.randn(2, 128, 200, generator=torch.Generator().manual_seed(2)).cuda()
+    feats[1, 77, 90] = value
+    got, want = enc.subsample(feats), general(enc, feats)
+    assert torch.equal(got[0], enc.subsample(feats[:1])[0])
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    ok = torch.isfinite(want)
+    assert float((got[ok] - want[ok]).abs().max()) <= 1e-5 * float(want[ok].abs().max())
