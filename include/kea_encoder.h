@@ -116,12 +116,19 @@ int kea_dwconv2d_s2(const float *x_dev, const float *in_bias_dev, const float *w
 int kea_bias_relu_flatten(const float *x_dev, const float *bias_dev, float *y_dev, int64_t batch, int64_t channels,
                           int64_t h, int64_t wd, void *stream);
 
-/* The same subsampling for 128 mel bins and 256 channels with its pointwise convolutions, in two launches, channels
- * last. t2 = ((t-1)/2)/2+1, t3 = (t2-1)/2+1.
+/* The same subsampling for 128 mel bins and 256 channels with its pointwise convolutions and the output linear,
+ * channels last. t2 = ((t-1)/2)/2+1, t3 = (t2-1)/2+1.
  *
  * kea_subsample_stage1: x [batch][128][t] -> y [batch][t2][32][256] =
  *   relu(pointwise3(depthwise2(relu(conv1(x) + b1)) + b2) + b3).
- * kea_subsample_stage2: x [batch][t2][32][256] -> y [batch][t3][16][256] = relu(pointwise6(depthwise5(x) + b5) + b6).
+ * kea_subsample_stage2: x [batch][t2][32][256] -> relu(pointwise6(depthwise5(x) + b5) + b6), [batch][t3][16 x 256]
+ *   (frequency, channel), as FP16 planes y [batch][t3][2][4096] (hi, lo) and row scales ys [batch][t3]: a value is
+ *   (hi + lo) * ys, ys a power of two that puts the row's largest hi into [2^14, 2^15). A row with an infinity has an
+ *   infinite ys, and then only which of its hi are infinite counts.
+ * kea_subsample_out: such rows x [m][2][4096], xs [m] -> y [m][n] = x w^T + bias: wf the weights in (frequency, channel)
+ *   order split like w3f ([n / 16][128][2][64][8], scales wm), w the same linear's weights [n][256 x 16] (channel,
+ *   frequency) before the factor gain > 0. n a multiple of 128. workspace: kea_subsample_out_workspace(m, n) bytes (0:
+ *   none needed).
  *
  * w1, w2, w5 [9][256], w3, w6 [256][256] (out, in): FP32, and the convolution weights split row by row into FP16 planes,
  * w[n] = (hi[n] + lo[n]) * m[n] with a power of two m[n] that puts the row's largest |hi| into [2^14, 2^15): w1f
@@ -129,14 +136,18 @@ int kea_bias_relu_flatten(const float *x_dev, const float *bias_dev, float *y_de
  * 9-17 are hi, 18-26 lo, 27-31 zero; w3f, w6f [16][8][2][64][8], n-tile, k-step, plane, lane 16 g + i, element j =
  * row 16 tile + i, column 32 step + 8 g + j. Weights are finite, nonzero rows of
  * w1 at least 2^-30, |b1| <= 2^15, and m1 no less than 2^-44; inputs may be anything (a NaN is zero after a ReLU). Every
- * pointer but w1, w3, w6 and stage 1's x is 16-byte aligned. batch <= 65535. */
+ * pointer but w1, w3, w6, w, ys, xs and stage 1's x is 16-byte aligned. batch <= 65535. */
 int kea_subsample_stage1(const float *x_dev, int64_t batch, int64_t t, const void *w1f_dev, const float *m1_dev,
                          const float *w1_dev, const float *b1_dev, const float *w2_dev, const float *b2_dev,
                          const void *w3f_dev, const float *m3_dev, const float *w3_dev, const float *b3_dev, float *y_dev,
                          void *stream);
 int kea_subsample_stage2(const float *x_dev, int64_t batch, int64_t t2, const float *w5_dev, const float *b5_dev,
-                         const void *w6f_dev, const float *m6_dev, const float *w6_dev, const float *b6_dev, float *y_dev,
-                         void *stream);
+                         const void *w6f_dev, const float *m6_dev, const float *w6_dev, const float *b6_dev, void *y_dev,
+                         float *ys_dev, void *stream);
+int64_t kea_subsample_out_workspace(int64_t m, int64_t n);
+int kea_subsample_out(const void *x_dev, const float *xs_dev, int64_t m, int64_t n, const void *wf_dev,
+                      const float *wm_dev, const float *w_dev, float gain, const float *bias_dev, float *y_dev,
+                      void *workspace_dev, int64_t workspace_bytes, void *stream);
 
 /* Normalised log-mel features from an STFT (the preprocessor of NeMo's AudioToMelSpectrogramPreprocessor, which
  * the reference's encoder runs in front of its layers): spec interleaved complex [batch][bins][ld_t] (ld_t >= frames),

@@ -1,18 +1,22 @@
-// The dw-striding subsampling of 128 mel bins at 256 channels in two launches, channels last, with the convolutions
-// that are contractions on the FP16 matrix cores at FP32 accuracy (kea_split.h):
-//   1. conv 3x3/2 (1 -> 256) + ReLU + depthwise 3x3/2 + pointwise 256 -> 256 + ReLU      [B][128][T] -> [B][T2][32][256]
-//   2. depthwise 3x3/2 + pointwise 256 -> 256 + ReLU                          [B][T2][32][256] -> [B][T3][16][256]
-// A workgroup makes all 256 channels of its positions, so a pointwise convolution's input never leaves LDS, where the same
-// layers as separate kernels (kea_subsample_front, a library GEMM, kea_dwconv2d_s2, a library GEMM, kea_bias_relu_flatten)
-// write and read [B][256][T2][32] three times and the FP32 GEMMs run at 1/16 of the FP16 rate. The first convolution is
-// itself one matrix product: its 9 taps times the three products of a split operand are 27 of a 32-deep MFMA's terms.
+// The dw-striding subsampling of 128 mel bins at 256 channels in three kernels, channels last, with everything that is a
+// contraction on the FP16 matrix cores at FP32 accuracy (kea_split.h):
+//   1. conv 3x3/2 (1 -> 256) + ReLU + depthwise 3x3/2 + pointwise 256 -> 256 + ReLU     [B][128][T] -> [B][T2][32][256]
+//   2. depthwise 3x3/2 + pointwise 256 -> 256 + ReLU, split            [B][T2][32][256] -> [B][T3][hi, lo][16 x 256]
+//   3. the output linear 4096 -> d (and a sum over its K slices)                                     -> [B][T3][d]
+// A workgroup of 1 and 2 makes all 256 channels of its positions, so a pointwise convolution's input never leaves LDS,
+// where the same layers as separate kernels (kea_subsample_front, a library GEMM, kea_dwconv2d_s2, a library GEMM,
+// kea_bias_relu_flatten) write and read [B][256][T2][32] three times and the FP32 GEMMs run at 1/16 of the FP16 rate.
+// The first convolution is itself one matrix product: its 9 taps times the three products of a split operand are 27 of a
+// 32-deep MFMA's terms. Kernel 2 makes whole rows of the output linear's input, so it can split them with a row's scale.
 //
-// Measured on eight 10-second clips (T = 1000): 54 + 24 us, where the five launches take 53 + 90 + 25 + 27 + 25 us; one
-// clip 15 + 12 us. Launch 1 executes 1850 vector instructions and 232 MFMAs a wave, and the two hardly overlap: about 27
-// and 12 us of its 54 at the clock it runs at, the rest waits between its phases. Two rows of 32 positions to a workgroup,
-// two workgroups to a CU, is the split that measured best: four rows (one workgroup to a CU, half the weight reads)
-// take 60 and, for one clip, 25 us. Launch 2 is latency: the weights (256 KB a workgroup) and its input from L2; half the
-// rows to a workgroup take 37 us, as the weights are read twice as often.
+// Measured on eight 10-second clips (T = 1000): 50 + 26 + 34 us, where five launches and a library GEMM take 53 + 90 +
+// 25 + 27 + 25 + 70 us; one clip 15 + 15 + 17 us.
+// Kernel 1 executes 1850 vector instructions and 232 MFMAs a wave, and the two hardly overlap: about 27 and 12 us of its
+// 50 at the clock it runs at, the rest waits between its phases. Two rows of 32 positions to a workgroup, two workgroups to
+// a CU, is the split that measured best: four rows (one workgroup to a CU, half the weight reads) take 60 and, for one
+// clip, 25 us. Kernel 2 is latency: the weights (256 KB a workgroup) and its input from L2; half the rows to a workgroup
+// take 37 us, as the weights are read twice as often. Kernel 3 is bound by L2: 268 MB of operands in 26 us, then 16 MB of
+// partial sums out and in again; larger tiles would halve the operands and double the partial sums.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -83,7 +87,7 @@ __device__ __forceinline__ void pointwise(const _Float16 *tile, Weights &w, int 
 
 // 3x3/2 taps of output position (r, c) read input rows 2 r - 1 + ky and columns 2 c - 1 + kx (padding 1).
 
-// Launch 1: a workgroup = one clip's output rows t2 = 2 blockIdx.x and + 1, all 32 columns and 256 channels.
+// Kernel 1: a workgroup = one clip's output rows t2 = 2 blockIdx.x and + 1, all 32 columns and 256 channels.
 constexpr int kMinExponent = -50;
 constexpr int kRows2 = 2, kPos1 = kRows2 * kF2;              // positions of a tile: 64, m = 32 q + f2
 constexpr int kRows1 = 2 * kRows2 + 1, kPatchR = 2 * kRows1 + 1, kPatchC = kF + 2;
@@ -312,20 +316,23 @@ subsample1_kernel(const float *x, int T, int T1, int T2, const _Float16 *w1f, co
     }
 }
 
-// Launch 2: a workgroup = one clip's output rows t3 = 4 blockIdx.x .. + 3, all 16 columns and 256 channels; a lane
+// Kernel 2: a workgroup = one clip's output rows t3 = 4 blockIdx.x .. + 3, all 16 columns and 256 channels; a lane
 // takes four channels.
 constexpr int kRows3 = 4, kPos2 = kRows3 * kF3, kCols3 = kPos2 / kWaves;  // 64 positions, 8 to a wave's depthwise
-constexpr int kTile2 = 2 * kPos2 * kC * 2, kLds2Bytes = kTile2 + kPos2 * 4 + 16;
+constexpr int kTile2 = 2 * kPos2 * kC * 2, kLds2Top = 2 * kTile2 + kPos2 * 4;  // (the FP32 path has its result after the tile)
+constexpr int kLds2Bytes = kLds2Top + kWaves * kRows3 * 4;
+constexpr int kOutK = kF3 * kC;  // the output linear's inputs
 
 __global__ void __launch_bounds__(kThreads)
 subsample2_kernel(const float *x, int T2, int T3, const float *w5, const float *b5, const _Float16 *w6f, const float *w6m,
-                  const float *w6, const float *b6, float *y) {
+                  const float *w6, const float *b6, _Float16 *y, float *ys) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15, g = lane >> 4;
     const int b = blockIdx.y, t3a = blockIdx.x * kRows3;
     const float *xb = x + (long long)b * T2 * kF2 * kC;
     _Float16 *const tile = (_Float16 *)lds;
-    float *const pscale = (float *)(lds + kTile2);
+    float *const pscale = (float *)(lds + 2 * kTile2);
+    int *const tops = (int *)(lds + kLds2Top);
     float4 wt[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) wt[k] = *(const float4 *)(w5 + k * kC + 4 * lane);
@@ -386,39 +393,254 @@ subsample2_kernel(const float *x, int T2, int T3, const float *w5, const float *
     weights.start(w6f, wave, lane);
     plain = __syncthreads_or(plain) != 0;
     const int rows = min(kRows3, T3 - t3a);
-    float *const yb = y + ((long long)b * T3 + t3a) * kF3 * kC;
+    const long long row0 = (long long)b * T3 + t3a;
+    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+    // four values of a row, split with its scale; of a row with an infinity only the infinities count
+    auto store = [&](int r, int k, v4f v, float sf, bool inf) {
+        v4h hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            _Float16 h, l;
+            split1(v[e], sf, h, l);
+            hi[e] = h;
+            lo[e] = inf ? (_Float16)0.f : l;
+        }
+        _Float16 *dst = y + (row0 + r) * 2 * kOutK + k;
+        *(v4h *)dst = hi;
+        *(v4h *)(dst + kOutK) = lo;
+    };
+    auto row_scale = [&](int r) {  // of row r's largest magnitude (all waves' parts are in tops)
+        int big = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) big = max(big, tops[w * kRows3 + r]);
+        return big;
+    };
     if (plain) {  // an infinity: the same sums in FP32
-        float *const h = (float *)lds;  // [kPos2][256]
+        float *const h = (float *)lds, *const out = (float *)(lds + kTile2);  // [kPos2][256]
 #pragma unroll
         for (int c = 0; c < kCols3; ++c)
             *(float4 *)(h + (16 * q + f0 + c) * kC + 4 * lane) = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
         __syncthreads();
         const int c = tid & (kC - 1);
-        for (int p = tid >> 8; p < rows * kF3; p += kThreads / kC) {
+        for (int p = tid >> 8; p < kPos2; p += kThreads / kC) {
             float acc = 0.f;
             for (int k = 0; k < kC; ++k) acc = __builtin_fmaf(w6[c * kC + k], h[p * kC + k], acc);
-            yb[p * kC + c] = fmaxf(acc + b6[c], 0.f);
+            out[p * kC + c] = fmaxf(acc + b6[c], 0.f);
+        }
+        __syncthreads();
+        for (int r = 0; r < kRows3; ++r) {
+            float m = 0.f;
+            for (int k = tid; k < kOutK; k += kThreads) m = kea::max_abs2(out[r * kOutK + k], 0.f, m);
+            const int t = kea::wave_max_bits(m);
+            if (lane == 0) tops[wave * kRows3 + r] = t;
+        }
+        __syncthreads();
+        for (int r = 0; r < rows; ++r) {
+            const int big = row_scale(r), e = exponent_of(big);
+            for (int k = 4 * tid; k < kOutK; k += 4 * kThreads)
+                store(r, k, *(const v4f *)(out + r * kOutK + k), pow2(14 - e), big >= kInfBits);
+            if (tid == 0) ys[row0 + r] = big >= kInfBits ? __builtin_inff() : pow2(e - 14);
         }
         return;
     }
     v4f acc[2][kPos2 / 16];
     pointwise<kPos2 / 16>(tile, weights, lane, acc);
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-        const int n = 32 * wave + 16 * nt + 4 * g;
-        const float4 wm = *(const float4 *)(w6m + n), bs = *(const float4 *)(b6 + n);
+    for (int mt = 0; mt < kPos2 / 16; ++mt) {  // m-tile = output row, m = its column
+        const float pm = pscale[16 * mt + i];
+        float m = 0.f;
 #pragma unroll
-        for (int mt = 0; mt < kPos2 / 16; ++mt) {
-            const int p = 16 * mt + i;
-            const float pm = pscale[p];
-            const v4f d = acc[nt][mt];
-            if (p < rows * kF3)
-                *(float4 *)(yb + p * kC + n) = make_float4(fmaxf(__builtin_fmaf(d[0], wm.x * pm, bs.x), 0.f),
-                                                           fmaxf(__builtin_fmaf(d[1], wm.y * pm, bs.y), 0.f),
-                                                           fmaxf(__builtin_fmaf(d[2], wm.z * pm, bs.z), 0.f),
-                                                           fmaxf(__builtin_fmaf(d[3], wm.w * pm, bs.w), 0.f));
+        for (int nt = 0; nt < 2; ++nt) {
+            const int n = 32 * wave + 16 * nt + 4 * g;
+            const v4f wm = *(const v4f *)(w6m + n), bs = *(const v4f *)(b6 + n);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[nt][mt][r] = fmaxf(__builtin_fmaf(acc[nt][mt][r], wm[r] * pm, bs[r]), 0.f);
+            m = kea::max_abs2(acc[nt][mt][0], acc[nt][mt][1], m);
+            m = kea::max_abs2(acc[nt][mt][2], acc[nt][mt][3], m);
+        }
+        const int t = kea::wave_max_bits(m);
+        if (lane == 0) tops[wave * kRows3 + mt] = t;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < kPos2 / 16; ++mt) {
+        if (mt >= rows) continue;
+        const int big = row_scale(mt), e = exponent_of(big);
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+            store(mt, i * kC + 32 * wave + 16 * nt + 4 * g, acc[nt][mt], pow2(14 - e), big >= kInfBits);
+        if (tid == 0) ys[row0 + mt] = big >= kInfBits ? __builtin_inff() : pow2(e - 14);
+    }
+}
+
+// Kernel 3, the output linear: y[m][n] = sum_k x[m][k] w[n][k] + bias[n] over the 4096 split inputs of a row, 128 x 128
+// tiles. Both operands come by direct copies to LDS in MFMA operand order (the weights laid out so, the inputs by
+// their rows), two k-steps of 32 a stage, two stages; waves 0 - 3 (64 x 64 each) take the stage's first
+// k-step, waves 4 - 7 the second, and their sums meet in LDS at the end. A wave holds the next stage's operands in
+// registers while it multiplies this one's, so a stage's buffer is refilled a stage and a half before it is read.
+constexpr int kBlk = 128, kStage = 2 * 2 * kBlk * 32 * 2 * 2, kLds3Bytes = 2 * kStage;  // 64 KB a stage
+
+typedef __attribute__((address_space(1))) const void *gptr_t;
+typedef __attribute__((address_space(3))) void *lptr_t;
+template <int VM, int LGKM>
+__device__ __forceinline__ void wait_counts() { __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4) | (LGKM << 8)); }
+__device__ __forceinline__ void stage_barrier() {  // without the wait for the copies in flight that __syncthreads makes
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// One output row's four columns: scaled sums, or for a row with infinities those alone (w: [n][256 x 16] FP32).
+__device__ __forceinline__ void finish(const _Float16 *x, const float *xs, const float *wm, const float *w, float gain,
+                                       const float *bias, long long m, int n, int N, v4f v, float *y) {
+    const float s = xs[m];
+    const v4f b = *(const v4f *)(bias + n), sc = *(const v4f *)(wm + n);
+    v4f r;
+    if (s == __builtin_inff()) {
+        v = (v4f){0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < kOutK; ++k)
+            if ((float)x[m * 2 * kOutK + k] == __builtin_inff())
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    v[e] += w[(long long)(n + e) * kOutK + (k % kC) * kF3 + k / kC] * gain * __builtin_inff();
+        r = v + b;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = __builtin_fmaf(v[e], sc[e] * s, b[e]);
+    }
+    *(v4f *)(y + m * N + n) = r;
+}
+
+__global__ void __launch_bounds__(kThreads)
+subsample3_kernel(const _Float16 *x, const float *xs, long long M, int N, int S, const _Float16 *wf, const float *wm,
+                  const float *w, float gain, const float *bias, float *part, float *y) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15, g = lane >> 4;
+    // an XCD (workgroups go round them) takes neighbouring tiles of one K slice
+    const int total = gridDim.x, id = blockIdx.x;
+    const int v = total % 8 == 0 ? (id & 7) * (total / 8) + (id >> 3) : id;
+    const int tiles_n = N / kBlk, nt0 = v % tiles_n, rest = v / tiles_n, tiles_m = (int)((M + kBlk - 1) / kBlk);
+    const long long m0 = (long long)(rest % tiles_m) * kBlk;
+    const int slice = rest / tiles_m, n0 = nt0 * kBlk;
+    const int steps = kOutK / 64 / S;  // stages of this slice: 4 to 64
+    // A stage: [x][16-row tile][plane][16 rows][64 inputs], 16-byte pieces XOR-swizzled by row, then [w][k-step][16-row
+    // tile][plane][64 lanes][8]; this wave copies its tile of x, whole 128-byte lines of eight rows at a time, and of w.
+    const int r8 = lane >> 3, piece = (lane & 7) ^ r8;
+    const long long row = m0 + 16 * wave + r8;
+    const _Float16 *xa = x + min(row, M - 1) * 2 * kOutK + slice * (kOutK / S) + 8 * piece;
+    const _Float16 *xb = x + min(row + 8, M - 1) * 2 * kOutK + slice * (kOutK / S) + 8 * piece;
+    const _Float16 *wa = wf + (((long long)(n0 / 16 + wave) * (kOutK / 32) + slice * (kOutK / 32 / S)) * 2 * 64 + lane) * 8;
+    auto copy = [&](int p) {
+        char *dst = lds + (p & 1) * kStage;
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl) {
+            __builtin_amdgcn_global_load_lds((gptr_t)(xa + pl * kOutK + p * 64), (lptr_t)(dst + (wave * 2 + pl) * 2048), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gptr_t)(xb + pl * kOutK + p * 64),
+                                             (lptr_t)(dst + (wave * 2 + pl) * 2048 + 1024), 16, 0, 0);
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+                __builtin_amdgcn_global_load_lds((gptr_t)(wa + ((2 * p + kk) * 2 + pl) * 512),
+                                                 (lptr_t)(dst + 32768 + kk * 16384 + (wave * 2 + pl) * 1024), 16, 0, 0);
+        }
+    };
+    const int kg = wave >> 2, wm4 = 4 * ((wave >> 1) & 1), wn4 = 4 * (wave & 1);
+    struct Operands {
+        v8h x[4][2], w[4][2];
+    };
+    auto read = [&](int p, Operands &o) {
+        const char *src = lds + (p & 1) * kStage, *sx = src + i * 128 + (((4 * kg + g) ^ (i & 7)) * 16),
+                   *sw = src + 32768 + kg * 16384 + lane * 16;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int pl = 0; pl < 2; ++pl) {
+                o.x[t][pl] = *(const v8h *)(sx + ((wm4 + t) * 2 + pl) * 2048);
+                o.w[t][pl] = *(const v8h *)(sw + ((wn4 + t) * 2 + pl) * 1024);
+            }
+    };
+    v4f acc[4][4];  // [n-tile][m-tile]
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[a][c] = (v4f){0.f, 0.f, 0.f, 0.f};
+    auto step = [&](int p, const Operands &now, Operands &next) {
+        if (p + 2 < steps)
+            wait_counts<8, 15>();  // stage p + 1 has landed, p + 2 may be in flight
+        else
+            wait_counts<0, 15>();
+        stage_barrier();
+        if (p + 1 < steps) read(p + 1, next);
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc[a][c] = mfma_split(now.w[a][0], now.w[a][1], now.x[c][0], now.x[c][1], acc[a][c]);
+        wait_counts<63, 0>();  // the reads are done: the buffer can be refilled
+        stage_barrier();
+        if (p + 3 < steps) copy(p + 3);
+    };
+    Operands even, odd;
+    copy(0);
+    copy(1);
+    wait_counts<8, 15>();
+    stage_barrier();
+    read(0, even);
+    wait_counts<63, 0>();
+    stage_barrier();
+    copy(2);
+    for (int p = 0; p < steps; p += 2) {
+        step(p, even, odd);
+        step(p + 1, odd, even);
+    }
+    // waves 4 - 7 hand their sums over
+    v4f *const hand = (v4f *)lds + (wave & 3) * 16 * 64 + lane;
+    if (kg == 1) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) hand[(a * 4 + c) * 64] = acc[a][c];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const long long m = m0 + 16 * (wm4 + c) + i;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const int n = n0 + 16 * (wn4 + a) + 4 * g;
+            const v4f sum = acc[a][c] + hand[(a * 4 + c) * 64];
+            if (m < M) {
+                if (S > 1)
+                    *(v4f *)(part + ((long long)slice * M + m) * N + n) = sum;
+                else
+                    finish(x, xs, wm, w, gain, bias, m, n, N, sum, y);
+            }
         }
     }
+}
+
+// The K slices of kernel 3 added up in order.
+template <int S>
+__global__ void __launch_bounds__(256)
+subsample_sum_kernel(const _Float16 *x, const float *xs, long long M, int N, const float *wm, const float *w,
+                     float gain, const float *bias, const float *part, float *y) {
+    const long long e = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (e >= M * N) return;
+    v4f t[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) t[s] = *(const v4f *)(part + s * M * N + e);
+    v4f sum = t[0];
+#pragma unroll
+    for (int s = 1; s < S; ++s) sum += t[s];
+    const long long m = e / N;
+    finish(x, xs, wm, w, gain, bias, m, (int)(e - m * N), N, sum, y);
+}
+
+// K slices: enough workgroups for the 256 CUs, at least four stages to a slice.
+int slices(long long M, int N) {
+    const long long tiles = (M + kBlk - 1) / kBlk * (N / kBlk);
+    int s = 1;
+    while (s < 16 && tiles * s * 2 <= 256) s *= 2;
+    return s;
 }
 
 int launched(const char *what) {
@@ -451,16 +673,49 @@ extern "C" int kea_subsample_stage1(const float *x, int64_t batch, int64_t t, co
 }
 
 extern "C" int kea_subsample_stage2(const float *x, int64_t batch, int64_t t2, const float *w5, const float *b5,
-                                    const void *w6f, const float *w6m, const float *w6, const float *b6, float *y,
-                                    void *stream) {
+                                    const void *w6f, const float *w6m, const float *w6, const float *b6, void *y,
+                                    float *ys, void *stream) {
     if (batch < 0 || batch > 65535 || t2 < 1 || t2 > INT32_MAX / 4) return kea::fail(KEA_EINVAL, "bad sizes");
     if (batch == 0) return KEA_OK;
-    if (!x || !w5 || !b5 || !w6f || !w6m || !w6 || !b6 || !y) return kea::fail(KEA_EINVAL, "null pointer");
+    if (!x || !w5 || !b5 || !w6f || !w6m || !w6 || !b6 || !y || !ys) return kea::fail(KEA_EINVAL, "null pointer");
     if (((uintptr_t)x | (uintptr_t)w5 | (uintptr_t)b5 | (uintptr_t)w6f | (uintptr_t)w6m | (uintptr_t)b6 | (uintptr_t)y) & 15)
-        return kea::fail(KEA_EALIGN, "every operand but w6 must be 16-byte aligned");
+        return kea::fail(KEA_EALIGN, "every operand but w6 and ys must be 16-byte aligned");
     const int t3 = (int)((t2 - 1) / 2 + 1);
     if (const int rc = allow_lds(subsample2_kernel, kLds2Bytes)) return rc;
     hipLaunchKernelGGL(subsample2_kernel, dim3((unsigned)((t3 + kRows3 - 1) / kRows3), (unsigned)batch), dim3(kThreads),
-                       kLds2Bytes, (hipStream_t)stream, x, (int)t2, t3, w5, b5, (const _Float16 *)w6f, w6m, w6, b6, y);
+                       kLds2Bytes, (hipStream_t)stream, x, (int)t2, t3, w5, b5, (const _Float16 *)w6f, w6m, w6, b6,
+                       (_Float16 *)y, ys);
     return launched("subsample stage 2");
+}
+
+extern "C" int64_t kea_subsample_out_workspace(int64_t m, int64_t n) {
+    if (m < 1 || n < kBlk || n % kBlk) return 0;
+    const int s = slices(m, (int)n);
+    return s > 1 ? s * m * n * (int64_t)sizeof(float) : 0;
+}
+
+extern "C" int kea_subsample_out(const void *x, const float *xs, int64_t m, int64_t n, const void *wf, const float *wm,
+                                 const float *w, float gain, const float *bias, float *y, void *workspace,
+                                 int64_t workspace_bytes, void *stream) {
+    if (m < 0 || n < kBlk || n % kBlk || n > 65536) return kea::fail(KEA_EINVAL, "bad sizes: n must be a multiple of 128");
+    if (m == 0) return KEA_OK;
+    const long long tiles = (m + kBlk - 1) / kBlk * (n / kBlk);
+    if (tiles > (1 << 20)) return kea::fail(KEA_EINVAL, "too many rows");
+    if (!x || !xs || !wf || !wm || !w || !bias || !y) return kea::fail(KEA_EINVAL, "null pointer");
+    if (((uintptr_t)x | (uintptr_t)wf | (uintptr_t)wm | (uintptr_t)bias | (uintptr_t)y | (uintptr_t)workspace) & 15)
+        return kea::fail(KEA_EALIGN, "every operand but xs and w must be 16-byte aligned");
+    const int s = slices(m, (int)n);
+    if (s > 1 && (!workspace || workspace_bytes < kea_subsample_out_workspace(m, n)))
+        return kea::fail(KEA_ESPACE, "workspace too small");
+    if (const int rc = allow_lds(subsample3_kernel, kLds3Bytes)) return rc;
+    hipLaunchKernelGGL(subsample3_kernel, dim3((unsigned)(tiles * s)), dim3(kThreads), kLds3Bytes, (hipStream_t)stream,
+                       (const _Float16 *)x, xs, (long long)m, (int)n, s, (const _Float16 *)wf, wm, w, gain, bias,
+                       (float *)workspace, y);
+    if (const int rc = launched("subsample output linear")) return rc;
+    if (s == 1) return KEA_OK;
+    const auto sum = s == 2 ? subsample_sum_kernel<2> : s == 4 ? subsample_sum_kernel<4> : s == 8 ? subsample_sum_kernel<8>
+                                                                                            : subsample_sum_kernel<16>;
+    hipLaunchKernelGGL(sum, dim3((unsigned)((m * n / 4 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                       (const _Float16 *)x, xs, (long long)m, (int)n, wm, w, gain, bias, (const float *)workspace, y);
+    return launched("subsample output sum");
 }

@@ -84,7 +84,9 @@ SIGNATURES = {
     "kea_dwconv2d_s2": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "kea_bias_relu_flatten": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "kea_subsample_stage1": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
-    "kea_subsample_stage2": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "kea_subsample_stage2": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "kea_subsample_out_workspace": (_i64, [_i64, _i64]),
+    "kea_subsample_out": (_i32, [_vp, _vp, _i64, _i64, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _i64, _vp]),
     "kea_dwconv_quantize": (_i32, [_vp, _i64, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _vp, _i64, _vp, _vp]),
     "kea_last_error": (_cp, []),
     "kea_version": (_i32, []),

@@ -511,15 +511,16 @@ class _SplitSubsampling:
         hi, lo, self.m6 = _split_f16(self.w6)
         self.f6 = _fragments([hi, lo])
         d = s["out.weight"].shape[0]
-        self.out = ((s["out.weight"] * gain).view(d, c, 16).transpose(1, 2).reshape(d, 16 * c).contiguous(),
-                    (s["out.bias"] * gain).contiguous())
+        self.out, self.gain, self.bias = s["out.weight"].contiguous(), gain, (s["out.bias"] * gain).contiguous()
+        hi, lo, self.mo = _split_f16((self.out * gain).view(d, c, 16).transpose(1, 2).reshape(d, 16 * c))
+        self.fo = _fragments([hi, lo])
 
     @staticmethod
     def prepare(s: dict, cfg: EncoderConfig):
         """The layout, or None where the kernels do not take the model: they are written for 128 mel bins and 256
-        channels, a weight that is not finite has no split form, and the first convolution's bias is held in units of
+        channels (and an output in tiles of 128), a weight that is not finite has no split form, and the first convolution's bias is held in units of
         its weights (nonzero rows from 2^-30, biases to 2^15, so that it stays finite for any scale of the input)."""
-        if cfg.feat_in != 128 or cfg.sub_channels != 256 or s["out.weight"].shape[1] != 16 * 256:
+        if cfg.feat_in != 128 or cfg.sub_channels != 256 or s["out.weight"].shape[1] != 16 * 256 or cfg.d_model % 128:
             return None
         if not all(bool(torch.isfinite(v).all()) for v in s.values()):
             return None
@@ -641,9 +642,8 @@ class FastConformerEncoder:
     def subsample(self, feats: Tensor) -> Tensor:
         """[B, mels, frames] -> [B, T', d] (dw-striding x8, then the output linear).
 
-        Fused (quantized) path, 128 mel bins and 256 channels: two launches up to the flattened features
-        (kea_subsample_stage1, kea_subsample_stage2; weights laid out when the encoder is made) and the output linear as
-        one matrix product. Other sizes: the first convolution + ReLU + first depthwise convolution in one kernel
+        Fused (quantized) path, 128 mel bins and 256 channels: three kernels (kea_subsample_stage1,
+        kea_subsample_stage2, kea_subsample_out; weights laid out when the encoder is made). Other sizes: the first convolution + ReLU + first depthwise convolution in one kernel
         (kea_subsample_front), the pointwise convolutions as batched matrix products whose bias + ReLU are applied
         by the next kernel on load, the second depthwise convolution (kea_dwconv2d_s2), the last bias + ReLU with the
         (channel, frequency) flatten (kea_bias_relu_flatten), and the output linear as one matrix product. Otherwise
@@ -701,11 +701,18 @@ class FastConformerEncoder:
                                           w.b1.data_ptr(), w.w2.data_ptr(), w.b2.data_ptr(), w.f3.data_ptr(),
                                           w.m3.data_ptr(), w.w3.data_ptr(), w.b3.data_ptr(), x1.data_ptr(), st),
                    "kea_subsample_stage1")
-        flat = torch.empty(b, t3, 16 * 256, device=feats.device, dtype=torch.float32)
+        m, n = b * t3, w.out.shape[0]
+        flat = torch.empty(m, 2, 16 * 256, device=feats.device, dtype=torch.float16)
+        scale = torch.empty(m, device=feats.device, dtype=torch.float32)
         _hip.check(L.kea_subsample_stage2(x1.data_ptr(), b, t2, w.w5.data_ptr(), w.b5.data_ptr(), w.f6.data_ptr(),
-                                          w.m6.data_ptr(), w.w6.data_ptr(), w.b6.data_ptr(), flat.data_ptr(), st),
-                   "kea_subsample_stage2")
-        return F.linear(flat, *w.out)
+                                          w.m6.data_ptr(), w.w6.data_ptr(), w.b6.data_ptr(), flat.data_ptr(),
+                                          scale.data_ptr(), st), "kea_subsample_stage2")
+        space = torch.empty(L.kea_subsample_out_workspace(m, n), device=feats.device, dtype=torch.uint8)
+        y = torch.empty(b, t3, n, device=feats.device, dtype=torch.float32)
+        _hip.check(L.kea_subsample_out(flat.data_ptr(), scale.data_ptr(), m, n, w.fo.data_ptr(), w.mo.data_ptr(),
+                                       w.out.data_ptr(), w.gain, w.bias.data_ptr(), y.data_ptr(), space.data_ptr(),
+                                       space.numel(), st), "kea_subsample_out")
+        return y
 
     def positions(self, t: int) -> list:
         """W_pos applied to the relative encodings, per layer, for length t: [2t-1, d] each. Frozen per length
