@@ -629,7 +629,8 @@ logmel_normalize_kernel(const float2 *spec, int bins, int frames, long long ld_t
 // read with consecutive bins on consecutive lanes; each thread then sums its frames' powers in the order of
 // logmel_normalize_kernel (increasing k, one fma per bin) and the normalisation is the same code, so both layouts give
 // the same bits. Bands wider than kBand bins are staged kBand bins at a time.
-constexpr int kChunk = 512, kBand = 16;
+// A thread loads kLoads bins before it stores their powers: one by one, each load waited for the last.
+constexpr int kChunk = 512, kBand = 16, kLoads = 8;
 __global__ void __launch_bounds__(256)
 logmel_normalize_frames_kernel(const float2 *spec, int bins, int frames, long long ld_f, const float *fb,
                                const int *lo, const int *hi, int mels, float log_eps, float std_eps, float *y) {
@@ -648,10 +649,25 @@ logmel_normalize_frames_kernel(const float2 *spec, int bins, int frames, long lo
         for (int kc = k0; kc < k1; kc += kBand) {
             const int w = min(kBand, k1 - kc);
             __syncthreads();  // the previous band's readers are done
-            for (int e = th; e < nf * w; e += 256) {
-                const int f = e / w, kk = e - f * w;
-                const float2 c = sb[(long long)(t0 + f) * bins + kc + kk];
-                pw[kk * (kChunk + 1) + f] = c.x * c.x + c.y * c.y;
+            const int df = 256 / w, dk = 256 - df * w;
+            int f = th / w, kk = th - f * w;  // element th + 256 j of the band, row by row
+            while (f < nf) {
+                float2 c[kLoads];
+                int at[kLoads];
+#pragma unroll
+                for (int u = 0; u < kLoads; ++u) {
+                    at[u] = f < nf ? kk * (kChunk + 1) + f : -1;
+                    if (f < nf) c[u] = sb[(long long)(t0 + f) * bins + kc + kk];
+                    f += df;
+                    kk += dk;
+                    if (kk >= w) {
+                        kk -= w;
+                        ++f;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kLoads; ++u)
+                    if (at[u] >= 0) pw[at[u]] = c[u].x * c[u].x + c[u].y * c[u].y;
             }
             __syncthreads();
             for (int kk = 0; kk < w; ++kk) {
