@@ -629,9 +629,11 @@ logmel_normalize_kernel(const float2 *spec, int bins, int frames, long long ld_t
 // read with consecutive bins on consecutive lanes; each thread then sums its frames' powers in the order of
 // logmel_normalize_kernel (increasing k, one fma per bin) and the normalisation is the same code, so both layouts give
 // the same bits. Bands wider than kBand bins are staged kBand bins at a time.
-// A thread loads kLoads bins before it stores their powers: one by one, each load waited for the last.
-constexpr int kChunk = 512, kBand = 16, kLoads = 8;
-__global__ void __launch_bounds__(256)
+// Bound by latency: the widest bands (some 8000 bins of 1000 frames) finish last while the rest of the chip waits. A
+// thread loads kLoads bins before it stores their powers (one by one, each load waited for the last), and 512 threads
+// share a band: eight 10-second clips 29.1 -> 27 -> 24.7 us.
+constexpr int kChunk = 512, kBand = 16, kLoads = 8, kFrameThreads = 512;
+__global__ void __launch_bounds__(kFrameThreads)
 logmel_normalize_frames_kernel(const float2 *spec, int bins, int frames, long long ld_f, const float *fb,
                                const int *lo, const int *hi, int mels, float log_eps, float std_eps, float *y) {
     __shared__ float pw[kBand * (kChunk + 1)];  // [bin of the band][frame], rows padded against bank conflicts
@@ -640,17 +642,14 @@ logmel_normalize_frames_kernel(const float2 *spec, int bins, int frames, long lo
     const float2 *sb = spec + (long long)b * ld_f * bins;
     float *yr = y + ((long long)b * mels + m) * frames;
     const int k0 = lo[m], k1 = hi[m];
-    float sum = 0.f;
     for (int t0 = 0; t0 < frames; t0 += kChunk) {
         const int nf = min(kChunk, frames - t0);
-        float acc[kChunk / 256];
-#pragma unroll
-        for (int i = 0; i < kChunk / 256; ++i) acc[i] = 0.f;
+        float acc = 0.f;
         for (int kc = k0; kc < k1; kc += kBand) {
             const int w = min(kBand, k1 - kc);
             __syncthreads();  // the previous band's readers are done
-            const int df = 256 / w, dk = 256 - df * w;
-            int f = th / w, kk = th - f * w;  // element th + 256 j of the band, row by row
+            const int df = kFrameThreads / w, dk = kFrameThreads - df * w;
+            int f = th / w, kk = th - f * w;  // element th + 512 j of the band, row by row
             while (f < nf) {
                 float2 c[kLoads];
                 int at[kLoads];
@@ -670,38 +669,33 @@ logmel_normalize_frames_kernel(const float2 *spec, int bins, int frames, long lo
                     if (at[u] >= 0) pw[at[u]] = c[u].x * c[u].x + c[u].y * c[u].y;
             }
             __syncthreads();
-            for (int kk = 0; kk < w; ++kk) {
-                const float wt = fb[m * bins + kc + kk];
-#pragma unroll
-                for (int i = 0; i < kChunk / 256; ++i)
-                    acc[i] = __builtin_fmaf(wt, pw[kk * (kChunk + 1) + th + 256 * i], acc[i]);
-            }
+            for (int kk = 0; kk < w; ++kk) acc = __builtin_fmaf(fb[m * bins + kc + kk], pw[kk * (kChunk + 1) + th], acc);
         }
-#pragma unroll
-        for (int i = 0; i < kChunk / 256; ++i) {
-            const int t = t0 + th + 256 * i;
-            if (t < frames) {
-                const float v = logf(acc[i] + log_eps);
-                yr[t] = v;
-                sum = sum + v;
-            }
-        }
+        if (th < nf) yr[t0 + th] = logf(acc + log_eps);
     }
+    __syncthreads();
+    // the sums of logmel_normalize_kernel's 256 threads, in its order
+    float sum = 0.f;
+    if (th < 256)
+#pragma unroll 4
+        for (int t = th; t < frames; t += 256) sum = sum + yr[t];
     sum = wave_sum(sum);
-    if ((th & 63) == 0) red[0][wave] = sum;
+    if (th < 256 && (th & 63) == 0) red[0][wave] = sum;
     __syncthreads();
     const float mean = ((red[0][0] + red[0][1]) + (red[0][2] + red[0][3])) / (float)frames;
     float sq = 0.f;
-    for (int t = th; t < frames; t += 256) {
-        const float d = yr[t] - mean;
-        sq = __builtin_fmaf(d, d, sq);
-    }
+    if (th < 256)
+#pragma unroll 4
+        for (int t = th; t < frames; t += 256) {
+            const float d = yr[t] - mean;
+            sq = __builtin_fmaf(d, d, sq);
+        }
     sq = wave_sum(sq);
-    if ((th & 63) == 0) red[1][wave] = sq;
+    if (th < 256 && (th & 63) == 0) red[1][wave] = sq;
     __syncthreads();
     const float var = ((red[1][0] + red[1][1]) + (red[1][2] + red[1][3])) / (float)(frames > 1 ? frames - 1 : 1);
     const float inv = 1.0f / (sqrtf(var) + std_eps);
-    for (int t = th; t < frames; t += 256) yr[t] = (yr[t] - mean) * inv;
+    for (int t = th; t < frames; t += kFrameThreads) yr[t] = (yr[t] - mean) * inv;
 }
 
 using kea::attention_splits;
@@ -915,7 +909,7 @@ int kea_logmel_normalize_frames(const float *spec, int64_t batch, int64_t bins, 
     if (batch == 0) return KEA_OK;
     if (!spec || !fb || !lo || !hi || !y) return kea::fail(KEA_EINVAL, "null pointer");
     if ((uintptr_t)spec & 7) return kea::fail(KEA_EALIGN, "spec must be 8-byte aligned (interleaved complex)");
-    hipLaunchKernelGGL(logmel_normalize_frames_kernel, dim3((unsigned)mels, (unsigned)batch), dim3(256), 0,
+    hipLaunchKernelGGL(logmel_normalize_frames_kernel, dim3((unsigned)mels, (unsigned)batch), dim3(kFrameThreads), 0,
                        (hipStream_t)stream, (const float2 *)spec, (int)bins, (int)frames, (long long)ld_f, fb, lo, hi,
                        (int)mels, log_eps, std_eps, y);
     hipError_t e = hipGetLastError();
