@@ -4,8 +4,8 @@
 //   s[i][j] = ((q_i + u) . k_j + (q_i + v) . p_{T-1-i+j}) * scale,  out_i = sum_j softmax_j(s)[i][j] v_j
 //
 // Arithmetic. The FP32 matrix instruction runs at 1/16 of the FP16 rate, so operands are pairs of FP16 values and a
-// product is three FP16 MFMAs (kea_split.h), with one power of two per query row, per four rows of K and P and per eight
-// keys of V. Against FP64 the result is closer than the FP32 forms (fewer roundings of the accumulator). A workgroup
+// product is three FP16 MFMAs (kea_split.h), with one power of two per query row, per four rows of K and P and per value
+// row. Against FP64 the result is closer than the FP32 forms (fewer roundings of the accumulator). A workgroup
 // that meets an infinity recomputes its rows with plain FP32 dot products (NaNs propagate by themselves).
 //
 // Two launches. split_kernel writes K, V and P once as hi / lo planes in the order the LDS of the second kernel holds
@@ -50,6 +50,7 @@ using kea::exponent_of;
 using kea::kInfBits;
 using kea::max_abs;
 using kea::pow2;
+using kea::split1;
 using kea::split8;
 using kea::v4f;
 using kea::v8h;
@@ -68,7 +69,7 @@ constexpr int kBandStride = 52;                 // band scores of a query in LDS
 //   K, V: block (b, h, kb), keys 64 kb ..;  P: block (h, pb), relative rows T - 64 + 64 (pb + 1 - tiles) ..: the two
 //   planes, in LDS order;  Q: block (b, h, tile): for both biases (u, v) the two planes of four 16-query groups as MFMA
 //   operands [s][lane][8] (lane: query lane % 16, elements 32 s + 8 (lane / 16) .. + 7).
-//   Multipliers 2^(e - 14): km, pm one for four rows, qm [bias][query]; ve: the exponents of the eight V groups.
+//   Multipliers 2^(e - 14): km, pm one for four rows, qm [bias][query]; ve: the exponent e of each of the 64 value rows.
 //   top: the bits of the largest magnitude, kt for K and V, pt for P, qt for Q.
 struct SplitOperands {
     char *q, *k, *v, *p;
@@ -91,7 +92,7 @@ inline long long split_layout(SplitOperands *s, char *ws, long long batch, int h
     take(s->qm, kv * 2 * kRows * 4);
     take(s->km, kv * 16 * 4);
     take(s->pm, np * 16 * 4);
-    take(s->ve, kv * 8 * 4);
+    take(s->ve, kv * kRows * 4);
     take(s->qt, kv * 4);
     take(s->kt, kv * 4);
     take(s->pt, np * 4);
@@ -204,16 +205,28 @@ split_kernel(const float *qkv, long long ld, const float *pos, long long ldp, co
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const int grp = 4 * u + wave;
-        const int bits = wave_max_bits(max_abs<16>(&v[u][0][0])), e = exponent_of(bits);
-        seen = max(seen, bits);
-        if (lane == 0) so.ve[(long long)id * 8 + grp] = e;
+        int e[8];  // a scale per key: its row may be any size beside the others'
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int bits = wave_max_bits(max_abs<2>(v[u][k]));
+            e[k] = exponent_of(bits);
+            seen = max(seen, bits);
+        }
+        if (lane == 0)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                *(int4 *)(so.ve + (long long)id * kRows + 32 * u + 16 * t + 4 * wave) =
+                    make_int4(e[4 * t], e[4 * t + 1], e[4 * t + 2], e[4 * t + 3]);
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-            float x[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) x[k] = v[u][k][c];
             v8h hi, lo;
-            split8(x, pow2(14 - e), hi, lo);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                _Float16 h, l;
+                split1(v[u][k][c], pow2(14 - e[k]), h, l);
+                hi[k] = h;
+                lo[k] = l;
+            }
             _Float16 *p = vt + (2 * lane + c) * kRows + ((grp ^ (lane & 7)) * 8);  // row d = 2 lane + c, unit ^ (d / 2 % 8)
             *(v8h *)p = hi;
             *(v8h *)(p + kPlane) = lo;
@@ -291,27 +304,30 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
     // multipliers of the wave's band tiles (rows 48 - 16 qg + 32 ks + 16 t of the two blocks), keys and V groups
     const int band0 = 48 - 16 * qg + 32 * ks;
     const float *pmp = so.pm + pfirst * 16 + band0 / 4 + g, *kmp = so.km + bh * tiles * 16 + 8 * ks + g;
-    const int32_t *vep = so.ve + bh * tiles * 8 + 4 * ks;
+    const int32_t *vep = so.ve + bh * tiles * kRows + 32 * ks + 4 * g;
     float pmul[3], kmul[2];
-    int4 ev;
+    int4 ev[2];  // exponents of the lane's eight value rows
     auto load_multipliers = [&](int kb) {
 #pragma unroll
         for (int t = 0; t < 3; ++t) pmul[t] = pmp[kb * 16 + 4 * t];
 #pragma unroll
         for (int t = 0; t < 2; ++t) kmul[t] = kmp[kb * 16 + 4 * t];
-        ev = *(const int4 *)(vep + kb * 8);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) ev[t] = *(const int4 *)(vep + kb * kRows + 16 * t);
     };
     load_multipliers(0);
     landed_barrier();
 
-    // Online softmax in base 2 with a lazy reference: probabilities are 2^(s - m_ref) with m_ref raised (and the sums
-    // rescaled) only when a score passes it by more than 8, so most blocks accumulate in the MFMA. Probabilities then
-    // reach 2^8; they are split at 2^6 times the V group's scale relative to 2^em.
+    // Online softmax in base 2 with lazy references: probabilities are 2^(s - m_ref) with the integer m_ref raised only when
+    // a score passes it by more than 8. A key's contribution to its query is its probability times 2^(exponent of its value
+    // row); 2^em is their size for this lane's query, raised (and the sums rescaled) only when one passes it by a factor of
+    // 2^8, so most blocks accumulate in the MFMA. The probabilities are split at 2^6 of that: what a query's output is
+    // made of holds its 22 bits whatever the value rows of other keys are, and a contribution is held to 2^-31 of the
+    // query's largest. (em of a step's largest value row instead, whatever its probability, lost the rest of the row to a
+    // large value under a suppressed key: 4e-5 of it at 2^16, 1e-2 at 2^24.)
     constexpr int kLazy = 8, kProbExp = 6;
     float m_ref = -INFINITY, l_run = 0.f;  // l_run: this lane's keys only
-    // em follows the blocks' exponents up at once and down by more than 3, but no further than 60 below the largest seen
-    // (the sums would leave FP32's range)
-    int em = -1000, etop = -1000;
+    int em = -1000;
     v4f o[8];
 #pragma unroll
     for (int d = 0; d < 8; ++d) o[d] = (v4f){0.f, 0.f, 0.f, 0.f};
@@ -376,30 +392,41 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) mx = fmaxf(mx, p[e]);
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const int eb = __builtin_amdgcn_readfirstlane(max(max(ev.x, ev.y), max(ev.z, ev.w)));
-            etop = max(etop, eb);
-            const int en = eb > em || eb < em - 3 ? max(eb, etop - 60) : em;
-            if (__any(mx > m_ref + kLazy) || en != em) {
-                const float m_new = fmaxf(m_ref, mx), a = __builtin_amdgcn_exp2f(m_ref - m_new);
-                const float f = a * pow2(max(min(em - en, 127), -127));
-                l_run = l_run * a;
+            if (__any(mx > m_ref + kLazy)) {  // the sums keep their values: 2^em falls by what the reference rises
+                mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                const bool above = mx > m_ref + kLazy;
+                const float m_new = above ? ceilf(mx) : m_ref, rise = above ? m_new - m_ref : 0.f;
+                l_run = l_run * __builtin_amdgcn_exp2f(-rise);
+                em -= (int)fminf(rise, 1e6f);
                 m_ref = m_new;
+            }
+            const int ek[8] = {ev[0].x, ev[0].y, ev[0].z, ev[0].w, ev[1].x, ev[1].y, ev[1].z, ev[1].w};
+            float w[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                p[e] = __builtin_amdgcn_exp2f(p[e] - m_ref);
+                l_run = l_run + p[e];
+                w[e] = __builtin_amdgcn_ldexpf(p[e], ek[e] - em + kProbExp);
+            }
+            if (__any(max_abs<8>(w) >= (float)(2 << (kLazy + kProbExp)))) {
+                int size = INT32_MIN;  // the largest contribution's exponent
+#pragma unroll
+                for (int e = 0; e < 8; ++e) size = max(size, (int)(__builtin_bit_cast(uint32_t, p[e]) >> 23) + ek[e]);
+                size = max(size, __shfl_xor(size, 16, 64));
+                size = max(size, __shfl_xor(size, 32, 64)) - 127;
+                const int en = size > em + kLazy ? size : em;
+                const float f = pow2(max(em - en, -127));
                 em = en;
 #pragma unroll
                 for (int d = 0; d < 8; ++d)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) o[d][r] = o[d][r] * f;
-            }
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                p[e] = __builtin_amdgcn_exp2f(p[e] - m_ref);
-                l_run = l_run + p[e];
+                for (int e = 0; e < 8; ++e) w[e] = __builtin_amdgcn_ldexpf(p[e], ek[e] - em + kProbExp);
             }
-            const int eg = g == 0 ? ev.x : g == 1 ? ev.y : g == 2 ? ev.z : ev.w;
             v8h ph, pl;
-            split8(p, pow2(max(eg - em + kProbExp, -127)), ph, pl);
+            split8(w, 1.f, ph, pl);
 #pragma unroll
             for (int d = 0; d < 8; ++d) {
                 const _Float16 *vp = Vh + (16 * d + n) * kRows + (((4 * ks + g) ^ (n >> 1)) * 8);
@@ -413,22 +440,17 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
     }
     l_run = l_run + __shfl_xor(l_run, 16, 64);
     l_run = l_run + __shfl_xor(l_run, 32, 64);
-    {
-        const float f = pow2(max(em - 14 - kProbExp, -127));  // (a wave without keys: o = 0)
-#pragma unroll
-        for (int d = 0; d < 8; ++d)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[d][r] = o[d][r] * f;
-    }
+    em -= 14 + kProbExp;  // the sums are in units of 2^em now
 
     // the two partial results of a query group meet in wave ks = 0
-    constexpr int kLane = 36;  // floats per lane: 32 outputs, m, l
+    constexpr int kLane = 36;  // floats per lane: 32 outputs, m, l, em
     float *const mb = (float *)lds + (qg * 64 + lane) * kLane;
     if (ks > 0) {
 #pragma unroll
         for (int d = 0; d < 8; ++d) *(float4 *)(mb + 4 * d) = make_float4(o[d][0], o[d][1], o[d][2], o[d][3]);
         mb[32] = m_ref;
         mb[33] = l_run;
+        mb[34] = __builtin_bit_cast(float, em);
     }
     __syncthreads();
     if (*bad) {
@@ -469,15 +491,19 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
     if (ks > 0) return;
     const float m1 = mb[32], mm = fmaxf(m_ref, m1);
     const float a0 = __builtin_amdgcn_exp2f(m_ref - mm), a1 = __builtin_amdgcn_exp2f(m1 - mm);
-    const float inv = 1.0f / __builtin_fmaf(mb[33], a1, l_run * a0), f0 = a0 * inv, f1 = a1 * inv;
+    const float inv = 1.0f / __builtin_fmaf(mb[33], a1, l_run * a0);
+    // each half times 2^(em + m - mm) / l, the exponent last: neither leaves FP32's range before the result does
+    const int e0 = em + (int)fmaxf(m_ref - mm, -1e6f);
+    const int e1 = __builtin_bit_cast(int, mb[34]) + (int)fmaxf(m1 - mm, -1e6f);
     if (iq < T) {
         float *dst = out + ((long long)b * T + iq) * ldo + (long long)h * kDK + 4 * g;
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
             const float4 w = *(const float4 *)(mb + 4 * d);
-            *(float4 *)(dst + 16 * d) =
-                make_float4(__builtin_fmaf(w.x, f1, o[d][0] * f0), __builtin_fmaf(w.y, f1, o[d][1] * f0),
-                            __builtin_fmaf(w.z, f1, o[d][2] * f0), __builtin_fmaf(w.w, f1, o[d][3] * f0));
+            auto sum = [&](float x0, float x1) {
+                return __builtin_amdgcn_ldexpf(x0 * inv, e0) + __builtin_amdgcn_ldexpf(x1 * inv, e1);
+            };
+            *(float4 *)(dst + 16 * d) = make_float4(sum(o[d][0], w.x), sum(o[d][1], w.y), sum(o[d][2], w.z), sum(o[d][3], w.w));
         }
     }
 }

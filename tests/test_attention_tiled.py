@@ -72,6 +72,27 @@ def test_any_magnitude_of_values(scale_v):
     _close(_tiled(*(a.cuda() for a in (qkv, pos, u, v))) / scale_v, ref / scale_v)
 
 
+def _row_error(got, ref):
+    """The largest error of an output row (one query and head) over that row's own largest element."""
+    got, ref = (x.double().view(*x.shape[:2], H, DK) for x in (got, ref))
+    return float(((got - ref).abs().amax(-1) / ref.abs().amax(-1)).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("key", [0, 69, 199])
+@pytest.mark.parametrize("power,score", [(12, -60), (20, -60), (40, -60), (100, -200)])
+def test_large_values_under_a_suppressed_key(key, power, score):
+    """One key of next to no probability whose value row is 2^power times the others': every output row is as accurate,
+    for its own size, as FP32 is. (FP32: 200 roundings of 2^-24, of random sign, and scores of size 4 off by 2^-22.)"""
+    qkv, pos, u, v = _inputs(1, 200, 7)
+    q, k = qkv[..., :D].view(1, 200, H, DK), qkv[..., D:2 * D].view(1, 200, H, DK)
+    q[..., 0], k[..., 0], u[:, 0] = 4.0, 0.0, 0.0
+    k[:, key] = 0.0
+    k[:, key, :, 0] = score * math.sqrt(DK) / 4.0
+    qkv[:, key, 2 * D:] *= 2.0 ** power
+    assert _row_error(_tiled(*(a.cuda() for a in (qkv, pos, u, v))), _reference(qkv, pos, u, v)) < 2e-6
+
+
 @pytest.mark.gpu
 def test_large_scores_and_small_queries():
     """Scores in the hundreds (a sharp softmax) hold the FP32 error of a score, 2^-24 of its terms; tiny queries give
