@@ -260,7 +260,7 @@ __device__ __forceinline__ void landed_barrier() {
 }
 
 constexpr int kLdsK = 0, kLdsP = kLdsK + kBlockBytes, kLdsV = kLdsP + 2 * kBlockBytes, kLdsBand = kLdsV + kBlockBytes;
-constexpr int kLdsBad = kLdsBand + kNW * 16 * kBandStride * 4, kTiledLds = kLdsBad + 16;
+constexpr int kLdsBad = kLdsBand + kNW * 16 * kBandStride * 4, kTiledLds = kLdsBad + kNW * 4;
 
 __global__ void __launch_bounds__(kNW * 64)
 relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long ldp, const float *bias_u,
@@ -277,8 +277,7 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
     const char *pblk = so.p + pfirst * kBlockBytes;
     _Float16 *const Kh = (_Float16 *)(lds + kLdsK), *const Ph = (_Float16 *)(lds + kLdsP), *const Vh = (_Float16 *)(lds + kLdsV);
     float *const bd = (float *)(lds + kLdsBand) + wave * 16 * kBandStride;
-    int *const bad = (int *)(lds + kLdsBad);
-    if (tid == 0) *bad = 0;
+    int *const bad = (int *)(lds + kLdsBad);  // a word per wave, written by every wave before the first barrier
 
     copy_block(kblk, lds + kLdsK, wave, lane);
     copy_block(pblk, lds + kLdsP, wave, lane);
@@ -300,7 +299,8 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
     int seen = so.qt[bh * tiles + iq0];
     for (int i = tid; i < tiles; i += kNW * 64)
         seen = max(max(seen, so.kt[bh * tiles + i]), max(so.pt[pfirst + i], so.pt[pfirst + i + 1]));
-    if (seen >= kInfBits) *bad = 1;
+    const bool wave_bad = __any(seen >= kInfBits) != 0;
+    if (lane == 0) bad[wave] = wave_bad;
     // multipliers of the wave's band tiles (rows 48 - 16 qg + 32 ks + 16 t of the two blocks), keys and V groups
     const int band0 = 48 - 16 * qg + 32 * ks;
     const float *pmp = so.pm + pfirst * 16 + band0 / 4 + g, *kmp = so.km + bh * tiles * 16 + 8 * ks + g;
@@ -453,7 +453,10 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
         mb[34] = __builtin_bit_cast(float, em);
     }
     __syncthreads();
-    if (*bad) {
+    int any_bad = 0;
+#pragma unroll
+    for (int w = 0; w < kNW; ++w) any_bad |= bad[w];
+    if (any_bad) {
         // an infinity among the inputs: plain FP32, a wave per query row, keys over the lanes
         for (int qi = wave; qi < kRows; qi += kNW) {
             const int i = iq0 * kRows + qi;

@@ -138,6 +138,33 @@ def test_non_finite_inputs_as_the_formula(where):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("where,row", [("v", 4290), ("k", 4170), ("v", 4230)])
+def test_infinities_past_the_64th_key_block(where, row):
+    """More key blocks than a wave looks over: the block that holds the infinity is seen by one wave other than the first."""
+    t, L = 4300, _hip.lib()
+    g = torch.Generator().manual_seed(12)
+    qkv, pos = torch.randn(1, t, 3 * DK, generator=g), torch.randn(2 * t - 1, DK, generator=g)
+    u, v = torch.randn(1, DK, generator=g) * 0.1, torch.randn(1, DK, generator=g) * 0.1
+    qkv[0, row, {"k": DK, "v": 2 * DK}[where] + 3] = math.inf
+    dev = [a.cuda() for a in (qkv, pos, u, v)]
+    out = torch.full((1, t, DK), 7.0, device="cuda")
+    ws = torch.empty(L.kea_relpos_attention_tiled_workspace(1, t, 1), dtype=torch.uint8, device="cuda")
+    _hip.check(L.kea_relpos_attention_tiled(dev[0].data_ptr(), 3 * DK, dev[1].data_ptr(), DK, dev[2].data_ptr(),
+                                            dev[3].data_ptr(), out.data_ptr(), DK, 1, t, 1, DK, 1 / math.sqrt(DK),
+                                            ws.data_ptr(), ws.numel(), _hip.stream_handle(out.device)), "tiled")
+    got, rows = out[0].cpu(), torch.tensor([0, 63, 64, 2000, 4299])      # (the reference: a few queries of each kind)
+    q, k, vv = qkv[0].double().split(DK, 1)
+    j = torch.arange(t)
+    for i in rows.tolist():
+        s = ((q[i] + u[0].double()) * k).sum(1) + ((q[i] + v[0].double()) * pos[t - 1 - i + j].double()).sum(1)
+        p = torch.softmax(s / math.sqrt(DK), 0)
+        ref = (p[:, None] * vv).sum(0).float()
+        fine = torch.isfinite(ref)
+        assert torch.equal(torch.isnan(got[i]), torch.isnan(ref)) and torch.equal(torch.isinf(got[i]), torch.isinf(ref))
+        assert not fine.any() or float((got[i] - ref)[fine].abs().max()) < 1e-5 * float(ref[fine].abs().max())
+
+
+@pytest.mark.gpu
 def test_layer_attention_routes(monkeypatch):
     """FastConformerEncoder.attention above 256 frames: the tiled kernel for plain FP32 tensors, the PyTorch form for
     what only it takes, the same values either way; relpos_attention still refuses more than 256 frames."""
