@@ -46,8 +46,11 @@ int kea_relpos_attention_ws(const float *qkv_dev, int64_t ld, const float *pos_d
 
 /* The same attention at any length t (up to 65535 tiles of 64 frames), for every length with a workspace of
  * kea_relpos_attention_tiled_workspace bytes (16-byte aligned, 0 for sizes the call refuses): a first launch splits Q, K,
- * V and the positions into pairs of FP16 values of one power-of-two scale a row (exact to 2^-22), a second walks the keys
- * in blocks with an online softmax on the FP16 matrix cores. Equal to kea_relpos_attention up to FP32 rounding. The
+ * V and the positions into pairs of FP16 values with a power-of-two scale per query, per value row and per four rows of K
+ * and of the positions (an element is held to 2^-22 of itself or 2^-39 of the largest under its scale), a second walks the
+ * keys in blocks with an online softmax on the FP16 matrix cores. Inputs that such pairs do not hold as well as FP32 does
+ * (infinities; elements of very different size within the rows) are computed in FP32 instead, per 64 queries of a head. An
+ * output row (a query of a head) is as accurate for its own largest element as kea_relpos_attention's. The
  * workspace is written before it is read, so it needs no clearing and may be reused by the next call on the stream. */
 int64_t kea_relpos_attention_tiled_workspace(int64_t batch, int64_t t, int heads);
 int kea_relpos_attention_tiled(const float *qkv_dev, int64_t ld, const float *pos_dev, int64_t ldp,

@@ -5,8 +5,10 @@
 //
 // Arithmetic. The FP32 matrix instruction runs at 1/16 of the FP16 rate, so operands are pairs of FP16 values and a
 // product is three FP16 MFMAs (kea_split.h), with one power of two per query row, per four rows of K and P and per value
-// row. Against FP64 the result is closer than the FP32 forms (fewer roundings of the accumulator). A workgroup
-// that meets an infinity recomputes its rows with plain FP32 dot products (NaNs propagate by themselves).
+// row. Against FP64 the result is closer than the FP32 forms (fewer roundings of the accumulator). Where the inputs hold an
+// infinity, or rows whose elements differ so much in size that the pairs would lose what FP32 keeps (kScores, kLowPairs), a
+// workgroup takes an FP32 form on the FP32 matrix instruction instead (NaNs propagate by themselves). That form reads its
+// operands from global memory and computes the scores twice: T = 200 batch 8 131 us, T = 750 batch 2 364.
 //
 // Two launches. split_kernel writes K, V and P once as hi / lo planes in the order the LDS of the second kernel holds
 // them, 64 rows to a block; relpos_tiled_kernel then copies blocks straight to LDS (global_load_lds) and spends no
@@ -45,6 +47,7 @@
 namespace {
 
 constexpr int kDK = 128;
+constexpr float kLog2e = 1.4426950408889634f;
 
 using kea::exponent_of;
 using kea::kInfBits;
@@ -54,15 +57,21 @@ using kea::split1;
 using kea::split8;
 using kea::v4f;
 using kea::v8h;
-using kea::wave_max;
 using kea::wave_max_bits;
-using kea::wave_sum;
 
 constexpr int kQG = 4, kKS = 2;                 // query groups and key halves: one wave each
 constexpr int kNW = kQG * kKS, kRows = 64;      // rows of a block of K, V or P; queries of a workgroup
-static_assert(16 * kQG == kRows && 32 * kKS == kRows, "queries, keys and P rows advance by the same block");
+static_assert(kKS == 2 && 16 * kQG == kRows && 32 * kKS == kRows, "queries, keys and P rows advance by the same block");
 constexpr int kPlane = kRows * kDK;             // elements of one plane of a block
 constexpr int kBlockBytes = 2 * kPlane * 2;     // hi and lo planes
+// Rows that the split form would not hold to FP32's accuracy go to the FP32 form. A value row's elements are held to 2^-31 of
+// the row's largest (with their probabilities): a row with kLowPairs or more nonzero pairs of elements 2^10 below it is not
+// split (a normal row's pair is that small once in 10^5, four of 64 at once in 10^14). An element of Q, K or P is held to 2^-39
+// of its row's largest (K and P: of four rows'), which costs a score at most 2^-31 of the largest query element times the
+// largest of K and P times the scale, and that if every element of the rows is so small: up to kScores, 2^-25 measured,
+// what FP32 rounds off a score of ordinary rows.
+constexpr int kLowPairs = 4;
+constexpr float kScores = 4096.f;
 constexpr int kBandStride = 52;                 // band scores of a query in LDS (floats): 47 used
 
 // The split operands in the workspace.
@@ -70,7 +79,8 @@ constexpr int kBandStride = 52;                 // band scores of a query in LDS
 //   planes, in LDS order;  Q: block (b, h, tile): for both biases (u, v) the two planes of four 16-query groups as MFMA
 //   operands [s][lane][8] (lane: query lane % 16, elements 32 s + 8 (lane / 16) .. + 7).
 //   Multipliers 2^(e - 14): km, pm one for four rows, qm [bias][query]; ve: the exponent e of each of the 64 value rows.
-//   top: the bits of the largest magnitude, kt for K and V, pt for P, qt for Q.
+//   top: the bits of the largest magnitude, kt for K, pt for P, qt for Q; kt is an infinity's where the block's value rows
+//   are not to be split.
 struct SplitOperands {
     char *q, *k, *v, *p;
     float *qm, *km, *pm;
@@ -208,9 +218,11 @@ split_kernel(const float *qkv, long long ld, const float *pos, long long ldp, co
         int e[8];  // a scale per key: its row may be any size beside the others'
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const int bits = wave_max_bits(max_abs<2>(v[u][k]));
+            const float pair = max_abs<2>(v[u][k]);
+            const int bits = wave_max_bits(pair);
             e[k] = exponent_of(bits);
-            seen = max(seen, bits);
+            const bool low = pair > 0.f && pair < __builtin_bit_cast(float, bits) * 0x1p-10f;
+            if (bits >= kInfBits || __popcll(__ballot(low)) >= kLowPairs) seen = kInfBits;
         }
         if (lane == 0)
 #pragma unroll
@@ -260,7 +272,7 @@ __device__ __forceinline__ void landed_barrier() {
 }
 
 constexpr int kLdsK = 0, kLdsP = kLdsK + kBlockBytes, kLdsV = kLdsP + 2 * kBlockBytes, kLdsBand = kLdsV + kBlockBytes;
-constexpr int kLdsBad = kLdsBand + kNW * 16 * kBandStride * 4, kTiledLds = kLdsBad + kNW * 4;
+constexpr int kLdsPlain = kLdsBand + kNW * 16 * kBandStride * 4, kTiledLds = kLdsPlain + kNW * 4;
 
 __global__ void __launch_bounds__(kNW * 64)
 relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long ldp, const float *bias_u,
@@ -277,7 +289,7 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
     const char *pblk = so.p + pfirst * kBlockBytes;
     _Float16 *const Kh = (_Float16 *)(lds + kLdsK), *const Ph = (_Float16 *)(lds + kLdsP), *const Vh = (_Float16 *)(lds + kLdsV);
     float *const bd = (float *)(lds + kLdsBand) + wave * 16 * kBandStride;
-    int *const bad = (int *)(lds + kLdsBad);  // a word per wave, written by every wave before the first barrier
+    int *const plain = (int *)(lds + kLdsPlain);  // a word per wave, written by every wave before the first barrier
 
     copy_block(kblk, lds + kLdsK, wave, lane);
     copy_block(pblk, lds + kLdsP, wave, lane);
@@ -295,12 +307,14 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
         }
     const int iq = iq0 * kRows + 16 * qg + n;
     const float *qm = so.qm + (bh * tiles + iq0) * 2 * kRows + 16 * qg + n;
-    const float mqu = qm[0] * (scale * 1.4426950408889634f), mqv = qm[kRows] * (scale * 1.4426950408889634f);
-    int seen = so.qt[bh * tiles + iq0];
+    const float mqu = qm[0] * (scale * kLog2e), mqv = qm[kRows] * (scale * kLog2e);
+    const int qtop = so.qt[bh * tiles + iq0];
+    int top = 0;
     for (int i = tid; i < tiles; i += kNW * 64)
-        seen = max(max(seen, so.kt[bh * tiles + i]), max(so.pt[pfirst + i], so.pt[pfirst + i + 1]));
-    const bool wave_bad = __any(seen >= kInfBits) != 0;
-    if (lane == 0) bad[wave] = wave_bad;
+        top = max(max(top, so.kt[bh * tiles + i]), max(so.pt[pfirst + i], so.pt[pfirst + i + 1]));
+    const float most = __builtin_bit_cast(float, qtop) * __builtin_bit_cast(float, top) * fabsf(scale * kLog2e);
+    const bool wave_plain = __any(max(qtop, top) >= kInfBits || most > kScores) != 0;
+    if (lane == 0) plain[wave] = wave_plain;
     // multipliers of the wave's band tiles (rows 48 - 16 qg + 32 ks + 16 t of the two blocks), keys and V groups
     const int band0 = 48 - 16 * qg + 32 * ks;
     const float *pmp = so.pm + pfirst * 16 + band0 / 4 + g, *kmp = so.km + bh * tiles * 16 + 8 * ks + g;
@@ -332,7 +346,81 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
 #pragma unroll
     for (int d = 0; d < 8; ++d) o[d] = (v4f){0.f, 0.f, 0.f, 0.f};
 
-    for (int kb = 0; kb < tiles; ++kb) {
+    int any_plain = 0;
+#pragma unroll
+    for (int w = 0; w < kNW; ++w) any_plain |= plain[w];
+    any_plain = __builtin_amdgcn_readfirstlane(any_plain);
+    if (any_plain) {
+        // The FP32 form, on the FP32 matrix instruction: the same tiles and lanes, operands straight from global memory, the
+        // exact two-pass softmax. Element 16 s + 4 g + e of a row is step (s, e) of the contraction.
+        const float *qp = qkv + ((long long)b * T + min(iq, T - 1)) * ld + (long long)h * kDK + 4 * g;
+        const float *kbase = qkv + (long long)b * T * ld + (long long)(H + h) * kDK + 4 * g, *pbase = pos + (long long)h * kDK + 4 * g;
+        const float *vbase = qkv + (long long)b * T * ld + (long long)(2 * H + h) * kDK + n;
+        v4f fu[8], fv[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const v4f q = *(const v4f *)(qp + 16 * s);
+            fu[s] = q + *(const v4f *)(bias_u + h * kDK + 4 * g + 16 * s);
+            fv[s] = q + *(const v4f *)(bias_v + h * kDK + 4 * g + 16 * s);
+        }
+        auto product = [&](const float *row, const v4f (&q)[8]) {
+            v4f c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const v4f x = *(const v4f *)(row + 16 * s);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], q[s][e], c, 0, 0, 0);
+            }
+            return c;
+        };
+        auto scores = [&](int jw, float (&p)[8]) {
+            const int first = T - 16 - (iq0 * kRows + 16 * qg) + jw;  // the band's first relative row
+            v4f c[2], r[3];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) r[t] = product(pbase + (long long)min(max(first + 16 * t + n, 0), 2 * T - 2) * ldp, fv);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) c[t] = product(kbase + (long long)min(jw + 16 * t + n, T - 1) * ld, fu);
+            asm volatile("" ::: "memory");  // (a wave's LDS accesses stay in order)
+#pragma unroll
+            for (int t = 0; t < 3; ++t) *(v4f *)(bd + n * kBandStride + 16 * t + 4 * g) = r[t];
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int jj = 16 * t + 4 * g + e;
+                    p[4 * t + e] = jw + jj < T ? (c[t][e] + bd[n * kBandStride + 15 - n + jj]) * scale : -INFINITY;
+                }
+            asm volatile("" ::: "memory");
+        };
+        float p[8];
+        for (int jw = 32 * ks; jw < T; jw += kRows) {
+            scores(jw, p);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) m_ref = fmaxf(m_ref, p[e]);
+        }
+        m_ref = fmaxf(m_ref, __shfl_xor(m_ref, 16, 64));
+        m_ref = fmaxf(m_ref, __shfl_xor(m_ref, 32, 64));
+        float *const maxima = (float *)(lds + kLdsV);  // (nothing else lies there from here on)
+        if (g == 0) maxima[wave * 16 + n] = m_ref;
+        __syncthreads();
+        m_ref = fmaxf(m_ref, maxima[(wave ^ 1) * 16 + n]);
+        for (int jw = 32 * ks; jw < T; jw += kRows) {
+            scores(jw, p);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int j = jw + 16 * (e >> 2) + 4 * g + (e & 3);
+                p[e] = j < T ? expf(p[e] - m_ref) : 0.f;
+                l_run = l_run + p[e];
+                const float *v = vbase + (long long)min(j, T - 1) * ld;
+#pragma unroll
+                for (int d = 0; d < 8; ++d)
+                    o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(j < T ? v[16 * d] : 0.f, p[e], o[d], 0, 0, 0);
+            }
+        }
+        em = 14 + kProbExp;
+    }
+    for (int kb = 0; kb < tiles && !any_plain; ++kb) {
         const int jw = kb * kRows + 32 * ks;  // this wave's first key
         int pbase[3];  // element offset of each band tile in the two-block ring
 #pragma unroll
@@ -453,44 +541,6 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
         mb[34] = __builtin_bit_cast(float, em);
     }
     __syncthreads();
-    int any_bad = 0;
-#pragma unroll
-    for (int w = 0; w < kNW; ++w) any_bad |= bad[w];
-    if (any_bad) {
-        // an infinity among the inputs: plain FP32, a wave per query row, keys over the lanes
-        for (int qi = wave; qi < kRows; qi += kNW) {
-            const int i = iq0 * kRows + qi;
-            if (i >= T) break;
-            const float *qbase = qkv + (long long)b * T * ld + (long long)h * kDK, *kbase = qbase + (long long)H * kDK;
-            const float *vbase = kbase + (long long)H * kDK, *pbase = pos + (long long)h * kDK;
-            const float *q = qbase + (long long)i * ld, *u = bias_u + h * kDK, *v = bias_v + h * kDK;
-            auto score = [&](int j) {
-                const float *k = kbase + (long long)j * ld, *p = pbase + (long long)(T - 1 - i + j) * ldp;
-                float c = 0.f, r = 0.f;
-                for (int d = 0; d < kDK; ++d) {
-                    c = __builtin_fmaf(q[d] + u[d], k[d], c);
-                    r = __builtin_fmaf(q[d] + v[d], p[d], r);
-                }
-                return (c + r) * scale;
-            };
-            float m = -INFINITY, l = 0.f, o0 = 0.f, o1 = 0.f;
-            for (int j = lane; j < T; j += 64) m = fmaxf(m, score(j));
-            m = wave_max(m);
-            for (int j0 = 0; j0 < T; j0 += 64) {
-                const float p = j0 + lane < T ? expf(score(j0 + lane) - m) : 0.f;
-                l = l + p;
-                for (int jj = 0; jj < min(64, T - j0); ++jj) {
-                    const float pj = __shfl(p, jj, 64);
-                    const float2 vv = *(const float2 *)(vbase + (long long)(j0 + jj) * ld + 2 * lane);
-                    o0 = __builtin_fmaf(pj, vv.x, o0);
-                    o1 = __builtin_fmaf(pj, vv.y, o1);
-                }
-            }
-            l = wave_sum(l);
-            *(float2 *)(out + ((long long)b * T + i) * ldo + (long long)h * kDK + 2 * lane) = make_float2(o0 / l, o1 / l);
-        }
-        return;
-    }
     if (ks > 0) return;
     const float m1 = mb[32], mm = fmaxf(m_ref, m1);
     const float a0 = __builtin_amdgcn_exp2f(m_ref - mm), a1 = __builtin_amdgcn_exp2f(m1 - mm);

@@ -18,7 +18,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 // The binary exponent e of a magnitude given by its bits (2^e <= m < 2^(e+1)), clamped so that 2^(14-e) and 2^(e-14)
 // are normal numbers.
-__device__ __forceinline__ int exponent_of(int bits) { return min(max((bits >> 23) - 127, -90), 127); }
+__device__ __forceinline__ int exponent_of(int bits) { return min(max((bits >> 23) - 127, -112), 127); }
 // 2^e for e in [-127, 127] (2^-127 as zero).
 __device__ __forceinline__ float pow2(int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); }
 

@@ -94,6 +94,66 @@ def test_large_values_under_a_suppressed_key(key, power, score):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("power", [9, 11, 13, 15, 20, 60])
+@pytest.mark.parametrize("operand", ["k_row", "k_dim", "q_row", "q_dim", "p_row", "p_dim", "v_element", "v_half"])
+def test_rows_and_elements_of_any_size(operand, power):
+    """A row 2^power times its neighbours, or a few elements that much larger than the rest of their rows, where the other
+    operand is zero: the scores they leave ordinary, and every other element of the output, are as accurate as in FP32
+    (the bar of the kernels that serve up to 128 frames, here for each row's own size)."""
+    b, t = 1, 150
+    qkv, pos, u, v = _inputs(b, t, 14)
+    x = {"q": qkv[..., :D], "k": qkv[..., D:2 * D], "v": qkv[..., 2 * D:], "p": pos[None]}
+    heads = {name: y.unflatten(-1, (H, DK)) for name, y in x.items()}
+    big, want = 2.0 ** power, slice(None)
+    if operand in ("k_row", "p_row", "q_row"):      # the row's product: one score far below the others, or an unused row
+        heads[operand[0]][:, 70, :, 1:] = 0.0
+        heads[operand[0]][:, 70, :, 0] = -big if operand != "q_row" else big
+        heads["q"][..., 0] = u[:, 0] = v[:, 0] = 0.0
+        if operand == "q_row":
+            heads["q"][:, 70, :, 0], heads["k"][..., 0], heads["p"][..., 0] = big, 0.0, 0.0
+        else:
+            heads["q"][:, :, :, 0] = 1.0
+    elif operand in ("k_dim", "p_dim", "q_dim"):    # elements that the other operand has no use for
+        heads[operand[0]][..., 5] *= big
+        for other in "kp" if operand == "q_dim" else "q":
+            heads[other][..., 5] = 0.0
+        if operand != "q_dim":
+            u[:, 5] = v[:, 5] = 0.0
+    elif operand == "v_element":
+        heads["v"][:, 70, :, 3] *= big
+        want = [d for d in range(DK) if d != 3]
+    else:
+        heads["v"][:, :, :, 64:] *= big
+        want = slice(0, 64)
+    got, ref = _tiled(*(a.cuda() for a in (qkv, pos, u, v))), _reference(qkv, pos, u, v)
+    assert torch.isfinite(got).all()
+    got, ref = (y.double().view(b, t, H, DK)[..., want] for y in (got, ref))
+    worst = float(((got - ref).abs().amax(-1) / ref.abs().amax(-1)).max())
+    print(operand, power, worst)
+    assert worst < 4e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale_v", [1e-37, 1e-34, 1e36])
+def test_values_near_the_ends_of_the_range(scale_v):
+    qkv, pos, u, v = _inputs(1, 140, 15)
+    qkv[..., 2 * D:] *= scale_v
+    assert _row_error(_tiled(*(a.cuda() for a in (qkv, pos, u, v))), _reference(qkv, pos, u, v)) < 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,t", [(1, 1), (2, 15), (1, 33), (3, 65), (2, 129), (1, 193), (2, 300), (1, 521)])
+def test_the_fp32_form_at_every_tile_edge(b, t):
+    """Half of the heads have keys with an element past the split form's bound that no query uses, so their workgroups run
+    the FP32 form."""
+    qkv, pos, u, v = _inputs(b, t, 16 + t)
+    q, k, _ = (x.view(b, t, H, DK) for x in qkv.split(D, 2))
+    k[:, :, ::2, 9] *= 2.0 ** 30
+    q[:, :, ::2, 9] = u[::2, 9] = v[::2, 9] = 0.0
+    _close(_tiled(*(a.cuda() for a in (qkv, pos, u, v))), _reference(qkv, pos, u, v))
+
+
+@pytest.mark.gpu
 def test_large_scores_and_small_queries():
     """Scores in the hundreds (a sharp softmax) hold the FP32 error of a score, 2^-24 of its terms; tiny queries give
     the mean of the values."""
