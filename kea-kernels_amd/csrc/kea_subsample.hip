@@ -88,7 +88,7 @@ __device__ __forceinline__ void pointwise(const _Float16 *tile, Weights &w, int 
 // 3x3/2 taps of output position (r, c) read input rows 2 r - 1 + ky and columns 2 c - 1 + kx (padding 1).
 
 // Kernel 1: a workgroup = one clip's output rows t2 = 2 blockIdx.x and + 1, all 32 columns and 256 channels.
-constexpr int kMinExponent = -50;
+constexpr int kMinExponent = -50, kHalfOne = 0x3c00;  // (FP16 bits of 1, 2^-14 of the scale's lower end)
 constexpr int kRows2 = 2, kPos1 = kRows2 * kF2;              // positions of a tile: 64, m = 32 q + f2
 constexpr int kRows1 = 2 * kRows2 + 1, kPatchR = 2 * kRows1 + 1, kPatchC = kF + 2;
 constexpr int kPatch = kPatchR * kPatchC;                    // input rows 4 t2 - 3 .., columns -1 .. 128
@@ -135,7 +135,10 @@ subsample1_kernel(const float *x, int T, int T1, int T2, const _Float16 *w1f, co
     int bits = top[0];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) bits = max(bits, top[w]);
-    // a tile of zeros has the smallest scale; one of smaller values than that is summed in FP32, as NaNs and infinities are
+    // a tile of zeros has the smallest scale; one of smaller values than that is summed in FP32, as NaNs and infinities are,
+    // and as one is where the scale of its largest value costs others their accuracy: a value that both planes lose (below
+    // 2^-39 of it), or a window of 3x3 inputs without one above 2^-14 of it (held to 2^-25 of the window's largest from there
+    // on). The output rows of a tile do not all see that largest value.
     const int xe = max(exponent_of(bits), kMinExponent);
     plain = plain || bits >= kInfBits || (bits != 0 && exponent_of(bits) < kMinExponent);
 #pragma unroll
@@ -143,6 +146,7 @@ subsample1_kernel(const float *x, int T, int T1, int T2, const _Float16 *w1f, co
         const int e = u * kThreads + tid, c = e / kPatchR, r = e - c * kPatchR;
         _Float16 hi, lo;
         split1(px[u], pow2(14 - xe), hi, lo);
+        plain = plain || (px[u] != 0.f && hi == (_Float16)0.f);
         if (e < kPatch) {
             patch[r * kPatchC + c] = hi;
             patch[kPatch + r * kPatchC + c] = lo;
@@ -165,6 +169,12 @@ subsample1_kernel(const float *x, int T, int T1, int T2, const _Float16 *w1f, co
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = patch[at[j] < 0 ? 2 * kPatch : base + at[j]];
             *(v8h *)(tile + (f * 64 + lane) * 8) = v;
+            // the window's largest: its nine hi values are terms 0 .. 7 of group 0 and term 0 of group 1
+            typedef uint16_t v8u __attribute__((ext_vector_type(8)));
+            const v8u size = __builtin_bit_cast(v8u, v) & (uint16_t)0x7fff;
+            int top9 = g == 0 ? __builtin_reduce_max(size) : g == 1 ? size[0] : 0;
+            top9 = max(top9, __shfl_xor(top9, 16, 64));
+            plain = plain || (g == 0 && top9 > 0 && top9 < kHalfOne);
         }
     }
     __syncthreads();

@@ -111,6 +111,46 @@ def test_special_values_as_general(value):
     assert float((got[ok] - want[ok]).abs().max()) <= 1e-5 * float(want[ok].abs().max())
 
 
+def _row_error(got, want):
+    """The largest error of an output row (one frame of one clip) over that row's own largest element."""
+    return float(((got - want).abs().amax(-1) / want.abs().amax(-1)).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mel,frame", [(0, 86), (77, 88), (127, 90)])
+@pytest.mark.parametrize("power", [10, 16, 24, 40, 100])
+@torch.inference_mode()
+def test_a_large_feature_is_seen_by_its_own_rows_only(mel, frame, power):
+    """One feature 2^power times the others: every output row is as accurate, for its own size, as the general kernels'
+    (the rows of the same tile that do not see it among them), and those rows hold the bits of a clip without it up to FP32
+    rounding."""
+    enc = model()
+    feats = torch.randn(2, 128, 200, generator=torch.Generator().manual_seed(3)).cuda()
+    plain = enc.subsample(feats).double().cpu()
+    feats[1, mel, frame] *= 2.0**power
+    want, got, old = exact(enc, feats), enc.subsample(feats).double().cpu(), general(enc, feats).double().cpu()
+    print(mel, frame, power, _row_error(got, want), _row_error(old, want))
+    assert _row_error(got, want) <= 2 * _row_error(old, want)
+    away = (8 * torch.arange(25) - frame).abs() > 7           # an output frame t sees 8 t - 7 .. 8 t + 7
+    assert _row_error(got[1, away], plain[1, away]) < 4e-6
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_features_of_mixed_sizes():
+    """Frames and mel bands whose sizes differ by up to 2^40, zeros between them."""
+    enc = model()
+    g = torch.Generator().manual_seed(4)
+    feats = torch.randn(2, 128, 130, generator=g) * 2.0 ** torch.randint(-20, 20, (2, 128, 130), generator=g)
+    feats[0, :, :31] *= 2.0**40
+    feats[0, 40:90] *= 2.0**-30
+    feats[1] *= (torch.rand(128, 130, generator=g) < 0.1)
+    feats = feats.cuda()
+    want, got, old = exact(enc, feats), enc.subsample(feats).double().cpu(), general(enc, feats).double().cpu()
+    print(_row_error(got, want), _row_error(old, want))
+    assert _row_error(got, want) <= 2 * _row_error(old, want)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n", [(1, 128), (127, 256), (128, 1024), (129, 128), (1000, 1024), (2100, 1024), (4000, 1024),
                                  (17000, 256)])
