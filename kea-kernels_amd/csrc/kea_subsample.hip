@@ -8,6 +8,9 @@
 // kea_bias_relu_flatten) write and read [B][256][T2][32] three times and the FP32 GEMMs run at 1/16 of the FP16 rate.
 // The first convolution is itself one matrix product: its 9 taps times the three products of a split operand are 27 of a
 // 32-deep MFMA's terms. Kernel 2 makes whole rows of the output linear's input, so it can split them with a row's scale.
+// Tiles whose inputs have no such form (infinities, sizes too far apart) take the same sums in FP32, the first convolutions
+// on the vector unit with a thread per channel, the pointwise product on the FP32 matrix instruction: eight 10-second clips
+// with a large value in every tile 191 us against 113 (one thread per channel throughout took 2180).
 //
 // Measured on eight 10-second clips (T = 1000): 50 + 26 + 34 us, where five launches and a library GEMM take 53 + 90 +
 // 25 + 27 + 25 + 70 us; one clip 15 + 15 + 17 us.
@@ -37,7 +40,7 @@ using kea::split1;
 using kea::v4f;
 using kea::v8h;
 
-constexpr int kC = 256, kF = 128, kF1 = 64, kF2 = 32, kF3 = 16;
+constexpr int kC = 256, kF = 128, kF2 = 32, kF3 = 16;
 constexpr int kWaves = 8, kThreads = 64 * kWaves;
 
 // max(x, 0) of an x that is not a NaN, on the bits (fmaxf would canonicalise an MFMA's result first).
@@ -82,6 +85,32 @@ __device__ __forceinline__ void pointwise(const _Float16 *tile, Weights &w, int 
                 acc[nt][mt] = mfma_split(w.f[ks % 3][nt][0], w.f[ks % 3][nt][1], hi, lo, acc[nt][mt]);
         }
         __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// The same product of FP32 operands on the FP32 matrix instruction, for tiles that are not split: x in LDS ([MT * 16][256],
+// 16-byte units XOR-swizzled by row), W [256][256] from L2. Element 16 s + 4 g + e of a row is step (s, e).
+__device__ __forceinline__ int fp32_at(int row, int k) { return row * kC + (((k >> 2) ^ (row & 15)) << 2) + (k & 3); }
+template <int MT>
+__device__ __forceinline__ void pointwise_fp32(const float *tile, const float *w, int wave, int lane, v4f (&acc)[2][MT]) {
+    typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+    const int i = lane & 15, g = lane >> 4;
+    const float *const row = w + (long long)(32 * wave + i) * kC + 4 * g;
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < kC / 16; ++s) {
+        const v4f a0 = *(const v4f_any *)(row + 16 * s), a1 = *(const v4f_any *)(row + 16 * kC + 16 * s);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const v4f x = *(const v4f *)(tile + fp32_at(16 * mt + i, 16 * s + 4 * g));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc[0][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[e], x[e], acc[0][mt], 0, 0, 0);
+                acc[1][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[e], x[e], acc[1][mt], 0, 0, 0);
+            }
+        }
     }
 }
 
@@ -255,67 +284,78 @@ subsample1_kernel(const float *x, int T, int T1, int T2, const _Float16 *w1f, co
     plain = __syncthreads_or(plain || big >= kInfBits) != 0;
     const int rows = min(kRows2, T2 - t2a);
     float *const yb = y + ((long long)b * T2 + t2a) * kF2 * kC;
-    if (plain) {  // the same sums in FP32, a thread per channel
-        float *const h = (float *)lds;  // [kPos1][256]
-        const int c = tid & (kC - 1);
-        for (int p = tid >> 8; p < rows * kF2; p += kThreads / kC) {
-            const int t2 = t2a + p / kF2, f2 = p % kF2;
-            float acc = b2[c];
-            for (int dy = 0; dy < 3; ++dy)
-                for (int dx = 0; dx < 3; ++dx) {
-                    const int t1 = 2 * t2 - 1 + dy, f1 = 2 * f2 - 1 + dx;
-                    float a = 0.f;
-                    if (t1 >= 0 && t1 < T1 && f1 >= 0 && f1 < kF1) {
-                        a = b1[c];
-                        for (int k = 0; k < 9; ++k) {
-                            const int t = 2 * t1 - 1 + k / 3, f = 2 * f1 - 1 + k % 3;
-                            a = __builtin_fmaf(w1[k * kC + c], t >= 0 && t < T && f >= 0 && f < kF ? xb[(long long)f * T + t] : 0.f, a);
-                        }
-                        a = fmaxf(a, 0.f);
-                    }
-                    acc = __builtin_fmaf(w2[(dy * 3 + dx) * kC + c], a, acc);
-                }
-            h[p * kC + c] = acc;
+    v4f acc[2][kPos1 / 16];
+    if (plain) {  // the same sums in FP32: a thread takes a channel of one output row
+        float *const xs = (float *)patch, *const h = (float *)lds;  // the patch (all waves are past the split one), [kPos1][256]
+        static_assert(kThreads == kRows2 * kC, "a thread per channel and row");
+#pragma unroll
+        for (int u = 0; u < PN; ++u) {
+            const int e = u * kThreads + tid, c = e / kPatchR, r = e - c * kPatchR;
+            if (e < kPatch) xs[r * kPatchC + c] = px[u];
         }
         __syncthreads();
-        for (int p = tid >> 8; p < rows * kF2; p += kThreads / kC) {
-            float acc = 0.f;
-            for (int k = 0; k < kC; ++k) acc = __builtin_fmaf(w3[c * kC + k], h[p * kC + k], acc);
-            yb[p * kC + c] = fmaxf(acc + b3[c], 0.f);
+        const int c = tid & (kC - 1), q = tid / kC, t1 = 2 * (t2a + q) - 1;
+        float wa[9], wb[9], before[3] = {0.f, 0.f, 0.f};  // before: the first convolution's column 2 f2 - 1
+        const float ba = b1[c], bb = b2[c];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            wa[k] = w1[k * kC + c];
+            wb[k] = w2[k * kC + c];
         }
-        return;
-    }
-    Weights weights;
-    weights.start(w3f, wave, lane);
-    // the split tile (all waves are past the fragments): two channels of a position are one word
+        for (int f2 = 0; f2 < kF2; ++f2) {
+            const float *const x0 = xs + 4 * q * kPatchC + 4 * f2;
+            float sum = bb;
 #pragma unroll
-    for (int q = 0; q < kRows2; ++q)
+            for (int dy = 0; dy < 3; ++dy) {
+                float v[2];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+                for (int s = 0; s < 2; ++s) {
+                    float a = ba;
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const int p = 32 * q + 8 * j + 2 * g + s, ch = 32 * wave + 2 * i;
-                const float sf = pscale[p];
-                typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-                _Float16 h0, l0, h1, l1;
-                split1(o[0][q][j][s], sf, h0, l0);
-                split1(o[1][q][j][s], sf, h1, l1);
-                _Float16 *dst = tile + p * kC + (((ch >> 3) ^ (p & 15)) * 8) + (ch & 7);
-                *(v2h *)dst = (v2h){h0, h1};
-                *(v2h *)(dst + kPos1 * kC) = (v2h){l0, l1};
+                    for (int k = 0; k < 9; ++k) a = __builtin_fmaf(wa[k], x0[(2 * dy + k / 3) * kPatchC + 2 * s + k % 3], a);
+                    v[s] = t1 + dy >= 0 && t1 + dy < T1 ? fmaxf(a, 0.f) : 0.f;
+                }
+                sum = __builtin_fmaf(wb[3 * dy], before[dy], sum);
+                sum = __builtin_fmaf(wb[3 * dy + 1], v[0], sum);
+                sum = __builtin_fmaf(wb[3 * dy + 2], v[1], sum);
+                before[dy] = v[1];
             }
-    __syncthreads();
-    v4f acc[2][kPos1 / 16];
-    pointwise<kPos1 / 16>(tile, weights, lane, acc);
+            h[fp32_at(32 * q + f2, c)] = sum;
+        }
+        __syncthreads();
+        pointwise_fp32<kPos1 / 16>(h, w3, wave, lane, acc);
+    } else {
+        Weights weights;
+        weights.start(w3f, wave, lane);
+        // the split tile (all waves are past the fragments): two channels of a position are one word
+#pragma unroll
+        for (int q = 0; q < kRows2; ++q)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const int p = 32 * q + 8 * j + 2 * g + s, ch = 32 * wave + 2 * i;
+                    const float sf = pscale[p];
+                    typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+                    _Float16 h0, l0, h1, l1;
+                    split1(o[0][q][j][s], sf, h0, l0);
+                    split1(o[1][q][j][s], sf, h1, l1);
+                    _Float16 *dst = tile + p * kC + (((ch >> 3) ^ (p & 15)) * 8) + (ch & 7);
+                    *(v2h *)dst = (v2h){h0, h1};
+                    *(v2h *)(dst + kPos1 * kC) = (v2h){l0, l1};
+                }
+        __syncthreads();
+        pointwise<kPos1 / 16>(tile, weights, lane, acc);
+    }
     // D[n][m]: a lane holds four consecutive output channels of a position
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
         const int n = 32 * wave + 16 * nt + 4 * g;
-        const float4 wm = *(const float4 *)(w3m + n), bias = *(const float4 *)(b3 + n);
+        const float4 bias = *(const float4 *)(b3 + n), wm = plain ? make_float4(1.f, 1.f, 1.f, 1.f) : *(const float4 *)(w3m + n);
 #pragma unroll
         for (int mt = 0; mt < kPos1 / 16; ++mt) {
             const int p = 16 * mt + i;
-            const float pm = 1.0f / pscale[p];  // a power of two: exact
+            const float pm = plain ? 1.f : 1.0f / pscale[p];  // (powers of two: exact)
             const v4f d = acc[nt][mt];
             if (p < rows * kF2)
                 *(float4 *)(yb + p * kC + n) = make_float4(fmaxf(__builtin_fmaf(d[0], wm.x * pm, bias.x), 0.f),
@@ -329,7 +369,7 @@ subsample1_kernel(const float *x, int T, int T1, int T2, const _Float16 *w1f, co
 // Kernel 2: a workgroup = one clip's output rows t3 = 4 blockIdx.x .. + 3, all 16 columns and 256 channels; a lane
 // takes four channels.
 constexpr int kRows3 = 4, kPos2 = kRows3 * kF3, kCols3 = kPos2 / kWaves;  // 64 positions, 8 to a wave's depthwise
-constexpr int kTile2 = 2 * kPos2 * kC * 2, kLds2Top = 2 * kTile2 + kPos2 * 4;  // (the FP32 path has its result after the tile)
+constexpr int kTile2 = 2 * kPos2 * kC * 2, kLds2Top = kTile2 + kPos2 * 4;
 constexpr int kLds2Bytes = kLds2Top + kWaves * kRows3 * 4;
 constexpr int kOutK = kF3 * kC;  // the output linear's inputs
 
@@ -341,7 +381,7 @@ subsample2_kernel(const float *x, int T2, int T3, const float *w5, const float *
     const int b = blockIdx.y, t3a = blockIdx.x * kRows3;
     const float *xb = x + (long long)b * T2 * kF2 * kC;
     _Float16 *const tile = (_Float16 *)lds;
-    float *const pscale = (float *)(lds + 2 * kTile2);
+    float *const pscale = (float *)(lds + kTile2);
     int *const tops = (int *)(lds + kLds2Top);
     float4 wt[9];
 #pragma unroll
@@ -425,44 +465,25 @@ subsample2_kernel(const float *x, int T2, int T3, const float *w5, const float *
         for (int w = 0; w < kWaves; ++w) big = max(big, tops[w * kRows3 + r]);
         return big;
     };
+    v4f acc[2][kPos2 / 16];
     if (plain) {  // an infinity: the same sums in FP32
-        float *const h = (float *)lds, *const out = (float *)(lds + kTile2);  // [kPos2][256]
+        float *const h = (float *)lds;  // [kPos2][256]
 #pragma unroll
         for (int c = 0; c < kCols3; ++c)
-            *(float4 *)(h + (16 * q + f0 + c) * kC + 4 * lane) = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
+            *(float4 *)(h + fp32_at(16 * q + f0 + c, 4 * lane)) = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
         __syncthreads();
-        const int c = tid & (kC - 1);
-        for (int p = tid >> 8; p < kPos2; p += kThreads / kC) {
-            float acc = 0.f;
-            for (int k = 0; k < kC; ++k) acc = __builtin_fmaf(w6[c * kC + k], h[p * kC + k], acc);
-            out[p * kC + c] = fmaxf(acc + b6[c], 0.f);
-        }
-        __syncthreads();
-        for (int r = 0; r < kRows3; ++r) {
-            float m = 0.f;
-            for (int k = tid; k < kOutK; k += kThreads) m = kea::max_abs2(out[r * kOutK + k], 0.f, m);
-            const int t = kea::wave_max_bits(m);
-            if (lane == 0) tops[wave * kRows3 + r] = t;
-        }
-        __syncthreads();
-        for (int r = 0; r < rows; ++r) {
-            const int big = row_scale(r), e = exponent_of(big);
-            for (int k = 4 * tid; k < kOutK; k += 4 * kThreads)
-                store(r, k, *(const v4f *)(out + r * kOutK + k), pow2(14 - e), big >= kInfBits);
-            if (tid == 0) ys[row0 + r] = big >= kInfBits ? __builtin_inff() : pow2(e - 14);
-        }
-        return;
+        pointwise_fp32<kPos2 / 16>(h, w6, wave, lane, acc);
+    } else {
+        pointwise<kPos2 / 16>(tile, weights, lane, acc);
     }
-    v4f acc[2][kPos2 / 16];
-    pointwise<kPos2 / 16>(tile, weights, lane, acc);
 #pragma unroll
     for (int mt = 0; mt < kPos2 / 16; ++mt) {  // m-tile = output row, m = its column
-        const float pm = pscale[16 * mt + i];
+        const float pm = plain ? 1.f : pscale[16 * mt + i];
         float m = 0.f;
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
             const int n = 32 * wave + 16 * nt + 4 * g;
-            const v4f wm = *(const v4f *)(w6m + n), bs = *(const v4f *)(b6 + n);
+            const v4f bs = *(const v4f *)(b6 + n), wm = plain ? (v4f){1.f, 1.f, 1.f, 1.f} : *(const v4f *)(w6m + n);
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[nt][mt][r] = fmaxf(__builtin_fmaf(acc[nt][mt][r], wm[r] * pm, bs[r]), 0.f);
             m = kea::max_abs2(acc[nt][mt][0], acc[nt][mt][1], m);
