@@ -68,11 +68,13 @@ struct Key {
     int64_t tag;                // what the operator does with the input (its own numbering)
     int64_t sizes[kMaxDim], strides[kMaxDim];
     const void *norm_w, *norm_b;
+    int64_t norm_size[2];       // elements of each; -1: a call without a LayerNorm
     float eps;
     int8_t dim, dtype, out_dtype, device;
     bool operator==(const Key &o) const {
         if (tag != o.tag || dim != o.dim || dtype != o.dtype || out_dtype != o.out_dtype || device != o.device ||
-            norm_w != o.norm_w || norm_b != o.norm_b || eps != o.eps)
+            norm_w != o.norm_w || norm_b != o.norm_b || norm_size[0] != o.norm_size[0] || norm_size[1] != o.norm_size[1] ||
+            eps != o.eps)
             return false;
         for (int i = 0; i < dim; ++i)
             if (sizes[i] != o.sizes[i] || strides[i] != o.strides[i]) return false;
@@ -106,8 +108,10 @@ struct Replays {
     Py_ssize_t limit;
 };
 
-// The key of input x; false where the call cannot be kept or replayed.
-bool make_key(const at::Tensor &x, PyObject *out_dtype, int64_t tag, PyObject *norm_w, PyObject *norm_b, double eps, Key *k) {
+// The key of input x; false where the call cannot be kept or replayed. norm: the call has a LayerNorm, whose parameters
+// must be there.
+bool make_key(const at::Tensor &x, PyObject *out_dtype, int64_t tag, bool norm, PyObject *norm_w, PyObject *norm_b, double eps,
+              Key *k) {
     if (x.dim() > kMaxDim || !THPDtype_Check(out_dtype)) return false;
     *k = Key{};
     k->tag = tag;
@@ -119,7 +123,8 @@ bool make_key(const at::Tensor &x, PyObject *out_dtype, int64_t tag, PyObject *n
     k->dtype = (int8_t)x.scalar_type();
     k->out_dtype = (int8_t)((THPDtype *)out_dtype)->scalar_type;
     k->device = x.device().index();
-    if (norm_w != Py_None) {  // LayerNorm parameters are read in place, where the plan was made for
+    k->norm_size[0] = k->norm_size[1] = -1;
+    if (norm) {  // LayerNorm parameters are read in place, where the plan was made for
         const at::Tensor *w[2];
         PyObject *const o[2] = {norm_w, norm_b};
         for (int i = 0; i < 2; ++i) {
@@ -131,6 +136,8 @@ bool make_key(const at::Tensor &x, PyObject *out_dtype, int64_t tag, PyObject *n
         }
         k->norm_w = w[0]->const_data_ptr();
         k->norm_b = w[1]->const_data_ptr();
+        k->norm_size[0] = w[0]->numel();
+        k->norm_size[1] = w[1]->numel();
         k->eps = (float)eps;
     }
     return true;
@@ -173,7 +180,7 @@ PyObject *replays_call(PyObject *o, PyObject *const *args, Py_ssize_t n) {
         Py_RETURN_NONE;
     }
     Key k;
-    if (!make_key(*x, args[1], tag, n == 6 ? args[3] : Py_None, n == 6 ? args[4] : Py_None, eps, &k)) Py_RETURN_NONE;
+    if (!make_key(*x, args[1], tag, n == 6, n == 6 ? args[3] : nullptr, n == 6 ? args[4] : nullptr, eps, &k)) Py_RETURN_NONE;
     const auto it = self->entries->find(k);
     if (it == self->entries->end()) Py_RETURN_NONE;
     try {
@@ -208,7 +215,7 @@ PyObject *replays_keep(PyObject *o, PyObject *args) {
         return nullptr;
     const at::Tensor *x = plain(xo);
     Key k;
-    if (!x || !make_key(*x, dtype, tag, nw, nb, eps, &k)) Py_RETURN_NONE;
+    if (!x || !make_key(*x, dtype, tag, nw != Py_None || nb != Py_None, nw, nb, eps, &k)) Py_RETURN_NONE;
     Entry e{owner, (const kea_project_plan *)plan, need, {}, transposed != 0, {}};
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(shape); ++i) {
         e.shape.push_back(PyLong_AsLongLong(PyTuple_GET_ITEM(shape, i)));

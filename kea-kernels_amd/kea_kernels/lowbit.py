@@ -392,7 +392,7 @@ class Launches:
 
     @staticmethod
     def _norm_key(norm, device):
-        """(weight pointer, bias pointer, eps) of a LayerNorm whose parameters the kernel can read in place (f32,
+        """(weight and bias pointers and lengths, eps) of a LayerNorm whose parameters the kernel can read in place (f32,
         contiguous, on the device), None without one, False where they would need a copy (the uncached path)."""
         if norm is None:
             return None
@@ -400,7 +400,7 @@ class Launches:
         for t in (w, b):
             if t is None or t.dtype != torch.float32 or t.device != device or not t.is_contiguous():
                 return False
-        return (w.data_ptr(), b.data_ptr(), float(norm.eps))
+        return (w.data_ptr(), b.data_ptr(), w.numel(), b.numel(), float(norm.eps))
 
     def project(self, x: Tensor, rows: tuple, m: int, parts: int, y: Tensor, *, silu: bool = False,
                 order: int = 0, norm=None, input_activation: str = "", config=None) -> bool:

@@ -200,6 +200,27 @@ def test_refused_arguments_raise_as_before():
             lowbit.quantize(torch.randn(8, 272, device=DEV), rows, m, 272, 2)
 
 
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_a_norm_without_parameters_or_of_another_length_is_refused_whatever_was_kept():
+    layer = _layer()
+    x = torch.randn(4, 272, device=DEV)
+    w = torch.ones(272, device=DEV)
+    norm = torch.nn.LayerNorm(272, device=DEV)
+    norm.weight, norm.bias = torch.nn.Parameter(w), torch.nn.Parameter(w)
+    short = torch.nn.LayerNorm(272, device=DEV)
+    short.weight, short.bias = torch.nn.Parameter(w[:100]), torch.nn.Parameter(w[:100])
+    assert short.weight.data_ptr() == norm.weight.data_ptr()
+    mod = runtime.PackedLinear(formats.pack_ternary(torch.ones(96, 272, dtype=torch.int8)), torch.ones(96), 272, mode="x1").to(DEV)
+    for call in (lambda norm: layer.project(x, components=1, norm=norm), lambda norm: fused_kernels.int8_matmul(x, mod, norm=norm)):
+        for _ in range(2):
+            assert not torch.equal(call(None), call(norm))
+        with pytest.raises(AttributeError):
+            call(torch.nn.LayerNorm(272, elementwise_affine=False))
+        with pytest.raises(ValueError, match="LayerNorm shape"):
+            call(short)
+
+
 def test_the_module_is_bound_and_declines_cpu_tensors():
     native = _hip.native()
     x = torch.randn(2, 16)
