@@ -15,6 +15,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <cstdint>
 #include <list>
@@ -184,8 +185,8 @@ PyObject *replays_call(PyObject *o, PyObject *const *args, Py_ssize_t n) {
     const auto it = self->entries->find(k);
     if (it == self->entries->end()) Py_RETURN_NONE;
     try {
-        PyObject *owner = it->second.owner;
-        Py_INCREF(owner);  // the plan outlives this call whatever runs meanwhile
+        // the plan outlives this call whatever runs meanwhile, and its owner is released however the call ends
+        const THPObjectPtr owner(Py_NewRef(it->second.owner));
         const kea_project_plan *plan = it->second.plan;
         const int64_t need = it->second.need;
         const bool transposed = it->second.transposed;
@@ -194,7 +195,6 @@ PyObject *replays_call(PyObject *o, PyObject *const *args, Py_ssize_t n) {
         at::Tensor ws = at::empty({need}, at::TensorOptions().device(device).dtype(at::kByte));
         const int rc = lib.project_launch(plan, x->const_data_ptr(), y.mutable_data_ptr(), ws.mutable_data_ptr(), need,
                                           stream_of(device));
-        Py_DECREF(owner);
         if (rc != 0) Py_RETURN_NONE;  // the Python path reports it
         return THPVariable_Wrap(transposed ? y.transpose(1, 2) : std::move(y));
     } catch (const std::exception &) {

@@ -2,6 +2,7 @@
 everything it does not take left to that path."""
 from __future__ import annotations
 
+import sys
 import threading
 
 import pytest
@@ -219,6 +220,31 @@ def test_a_norm_without_parameters_or_of_another_length_is_refused_whatever_was_
             call(torch.nn.LayerNorm(272, elementwise_affine=False))
         with pytest.raises(ValueError, match="LayerNorm shape"):
             call(short)
+
+
+class _Owner:
+    """A stand-in for a plan's owner that keeps another one when it is dropped."""
+
+    def __init__(self, dropped=None):
+        self.dropped = dropped
+
+    def __del__(self):
+        if self.dropped:
+            self.dropped()
+
+
+def _keep(replays, x, owner, need=0):
+    replays.keep(x, torch.float32, 1, None, None, 0.0, owner, 0, need, (4, 16), False)
+
+
+@pytest.mark.gpu
+def test_a_failed_allocation_releases_the_owner():
+    replays, x, owner = _hip.native().Replays(4), torch.randn(4, 16, device=DEV), _Owner()
+    _keep(replays, x, owner, 1 << 60)
+    count = sys.getrefcount(owner)
+    assert replays.call(x, torch.float32, 1) is None and sys.getrefcount(owner) == count
+    del replays
+    assert sys.getrefcount(owner) == count - 1
 
 
 def test_the_module_is_bound_and_declines_cpu_tensors():
