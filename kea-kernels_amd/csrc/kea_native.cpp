@@ -221,14 +221,14 @@ PyObject *replays_keep(PyObject *o, PyObject *args) {
         e.shape.push_back(PyLong_AsLongLong(PyTuple_GET_ITEM(shape, i)));
         if (PyErr_Occurred()) return nullptr;
     }
+    THPObjectPtr old;  // released last: that may run other code, which may come back here
     try {
         auto it = self->entries->find(k);
         if (it == self->entries->end() && (Py_ssize_t)self->entries->size() >= self->limit) it = self->entries->find(self->order->front());
         if (it != self->entries->end()) {  // replaced, or the oldest makes room
-            PyObject *old = it->second.owner;
+            old = it->second.owner;
             self->order->erase(it->second.order);
             self->entries->erase(it);
-            Py_DECREF(old);
         }
         e.order = self->order->insert(self->order->end(), k);
         self->entries->emplace(k, e);

@@ -247,6 +247,22 @@ def test_a_failed_allocation_releases_the_owner():
     assert sys.getrefcount(owner) == count - 1
 
 
+@pytest.mark.gpu
+def test_keeping_while_an_owner_is_released_stays_bounded():
+    """Releasing an evicted plan may run other code that keeps a layout: the limit holds, and nothing is lost or doubled."""
+    replays, xs = _hip.native().Replays(1), [torch.randn(m, 16, device=DEV) for m in (4, 5, 6)]
+    inner, outer = _Owner(), _Owner()
+    free = sys.getrefcount(inner), sys.getrefcount(outer)
+    kept = lambda: (sys.getrefcount(inner) - free[0], sys.getrefcount(outer) - free[1])  # noqa: E731
+    _keep(replays, xs[0], _Owner(lambda: _keep(replays, xs[1], inner)))
+    _keep(replays, xs[2], outer)                 # evicts the first, whose release keeps `inner`, which evicts `outer`
+    assert kept() == (1, 0)
+    _keep(replays, xs[2], outer)
+    assert kept() == (0, 1)
+    del replays
+    assert kept() == (0, 0)
+
+
 def test_the_module_is_bound_and_declines_cpu_tensors():
     native = _hip.native()
     x = torch.randn(2, 16)
