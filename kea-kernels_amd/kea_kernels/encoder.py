@@ -489,20 +489,29 @@ def _fragments(planes: list) -> Tensor:
 
 
 class _SplitSubsampling:
-    """The subsampling weights as kea_subsample_stage1 / stage2 read them, laid out once per encoder: the pointwise
+    """The subsampling weights as kea_subsample_stage1 / stage2 / out read them, all of them copies: the pointwise
     convolutions as split FP16 fragments, the first convolution's nine taps as the 27 terms (hi, hi, lo against the
     input's hi, lo, hi) of one 32-deep product with channels 32 w + 2 i + e in fragment 2 w + e, and the output
-    linear's columns in (frequency, channel) order."""
+    linear's columns in (frequency, channel) order. `holds` tells whether they still are what the tensors they were made
+    from hold (by identity and version: an in-place change through `.data` is the one that it does not see)."""
 
     LEAST = -30  # the exponent below which a row of the first convolution is not split (unless it is zero)
 
     def __init__(self, s: dict, gain: float):
         c = 256
-        self.w1, self.b1 = s["conv.0.weight"].reshape(c, 9).t().contiguous(), s["conv.0.bias"].contiguous()
-        self.w2, self.b2 = s["conv.2.weight"].reshape(c, 9).t().contiguous(), s["conv.2.bias"].contiguous()
-        self.w3, self.b3 = s["conv.3.weight"].reshape(c, c).contiguous(), s["conv.3.bias"].contiguous()
-        self.w5, self.b5 = s["conv.5.weight"].reshape(c, 9).t().contiguous(), s["conv.5.bias"].contiguous()
-        self.w6, self.b6 = s["conv.6.weight"].reshape(c, c).contiguous(), s["conv.6.bias"].contiguous()
+        self._source = [(k, v, v._version) for k, v in s.items()]
+
+        def taps(name):
+            return s[name].reshape(c, 9).t().clone(memory_format=torch.contiguous_format)
+
+        def copy(name, *shape):
+            return s[name].reshape(*shape).clone(memory_format=torch.contiguous_format)
+
+        self.w1, self.b1 = taps("conv.0.weight"), copy("conv.0.bias", c)
+        self.w2, self.b2 = taps("conv.2.weight"), copy("conv.2.bias", c)
+        self.w3, self.b3 = copy("conv.3.weight", c, c), copy("conv.3.bias", c)
+        self.w5, self.b5 = taps("conv.5.weight"), copy("conv.5.bias", c)
+        self.w6, self.b6 = copy("conv.6.weight", c, c), copy("conv.6.bias", c)
         hi, lo, self.m1 = _split_f16(s["conv.0.weight"].reshape(c, 9), _SplitSubsampling.LEAST)
         terms = torch.cat([hi, hi, lo, torch.zeros_like(hi[:, :5])], 1)
         self.f1 = terms.view(8, 16, 2, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
@@ -511,21 +520,28 @@ class _SplitSubsampling:
         hi, lo, self.m6 = _split_f16(self.w6)
         self.f6 = _fragments([hi, lo])
         d = s["out.weight"].shape[0]
-        self.out, self.gain, self.bias = s["out.weight"].contiguous(), gain, (s["out.bias"] * gain).contiguous()
+        self.out, self.gain, self.bias = copy("out.weight", d, 16 * c), gain, s["out.bias"] * gain
         hi, lo, self.mo = _split_f16((self.out * gain).view(d, c, 16).transpose(1, 2).reshape(d, 16 * c))
         self.fo = _fragments([hi, lo])
+
+    def holds(self, s: dict) -> bool:
+        return all(s[k] is v and v._version == n for k, v, n in self._source)
 
     @staticmethod
     def prepare(s: dict, cfg: EncoderConfig):
         """The layout, or None where the kernels do not take the model: they are written for 128 mel bins and 256
-        channels (and an output in tiles of 128), a weight that is not finite has no split form, and the first convolution's bias is held in units of
-        its weights (nonzero rows from 2^-30, biases to 2^15, so that it stays finite for any scale of the input)."""
+        channels (and an output in tiles of 128), a weight that is not finite has no split form (2^80 leaves the scaled sums
+        in range), and the first convolution's bias is held in units of its weights (nonzero rows from 2^-30, biases to 2^15,
+        so that it stays finite for any scale of the input). Waits for the GPU once."""
         if cfg.feat_in != 128 or cfg.sub_channels != 256 or s["out.weight"].shape[1] != 16 * 256 or cfg.d_model % 128:
             return None
-        if not all(bool(torch.isfinite(v).all()) for v in s.values()):
+        if any(v.is_inference() for v in s.values()):  # (a tensor that does not count its changes)
             return None
-        top = s["conv.0.weight"].reshape(256, 9).abs().amax(1)
-        if bool(((top > 0) & (top < 2.0**_SplitSubsampling.LEAST)).any()) or bool((s["conv.0.bias"].abs() > 2**15).any()):
+        tops = torch.stack([v.abs().amax() for v in s.values()])          # (NaN compares false)
+        row = s["conv.0.weight"].reshape(256, 9).abs().amax(1)
+        fits = ((tops <= 2.0**80).all() & ((row == 0) | (row >= 2.0**_SplitSubsampling.LEAST)).all()
+                & (s["conv.0.bias"].abs() <= 2**15).all())
+        if not fits.item():
             return None
         return _SplitSubsampling(s, math.sqrt(cfg.d_model) if cfg.xscaling else 1.0)
 
@@ -547,7 +563,9 @@ class FastConformerEncoder:
         self.pre = Preprocessor(cfg, device, fused=fused and not dense)
         dev = lambda t: t.to(device=device, dtype=torch.float32)  # noqa: E731
         p = "encoder.pre_encode."
-        self.sub = {k[len(p):]: dev(v) for k, v in weights.items() if k.startswith(p)}
+        with torch.inference_mode(False):  # (tensors that count their in-place changes; see _SplitSubsampling.holds)
+            self.sub = {k[len(p):]: dev(v) for k, v in weights.items() if k.startswith(p)}
+            self.sub = {k: v.clone() if v.is_inference() else v for k, v in self.sub.items()}
         self._sub_split = _SplitSubsampling.prepare(self.sub, cfg) if self.fused and device.type == "cuda" else None
         self.layers = []
         self._pos_cache: dict = {}
@@ -643,7 +661,8 @@ class FastConformerEncoder:
         """[B, mels, frames] -> [B, T', d] (dw-striding x8, then the output linear).
 
         Fused (quantized) path, 128 mel bins and 256 channels: three kernels (kea_subsample_stage1,
-        kea_subsample_stage2, kea_subsample_out; weights laid out when the encoder is made). Other sizes: the first convolution + ReLU + first depthwise convolution in one kernel
+        kea_subsample_stage2, kea_subsample_out), with weights laid out when the encoder is made and again after a change
+        to `self.sub`. Other sizes: the first convolution + ReLU + first depthwise convolution in one kernel
         (kea_subsample_front), the pointwise convolutions as batched matrix products whose bias + ReLU are applied
         by the next kernel on load, the second depthwise convolution (kea_dwconv2d_s2), the last bias + ReLU with the
         (channel, frequency) flatten (kea_bias_relu_flatten), and the output linear as one matrix product. Otherwise
@@ -667,8 +686,10 @@ class FastConformerEncoder:
         s, c = self.sub, self.cfg.sub_channels
         feats = feats.contiguous()
         b, f, t = feats.shape
-        if self._sub_split is not None and f == 128 and 1 <= t < 1 << 29 and b < 1 << 16 and feats.dtype == torch.float32:
-            return self._subsample_split(feats)
+        if f == 128 and 1 <= t < 1 << 29 and b < 1 << 16 and feats.dtype == torch.float32:
+            split = self._current_split(feats.device)
+            if split is not None:
+                return self._subsample_split(split, feats)
         t1, f1 = (t - 1) // 2 + 1, (f - 1) // 2 + 1
         t2, f2 = (t1 - 1) // 2 + 1, (f1 - 1) // 2 + 1
         t3, f3 = (t2 - 1) // 2 + 1, (f2 - 1) // 2 + 1
@@ -686,13 +707,30 @@ class FastConformerEncoder:
         flat = torch.empty(b, t3, c * f3, device=feats.device, dtype=torch.float32)
         _hip.check(L.kea_bias_relu_flatten(p2.data_ptr(), s["conv.6.bias"].data_ptr(), flat.data_ptr(), b, c, t3,
                                            f3, st), "kea_bias_relu_flatten")
-        if self._sub_out is None:  # the x sqrt(d) scaling folded into the output linear
+        out = self._sub_out
+        if out is None:  # the x sqrt(d) scaling folded into the output linear
             g = math.sqrt(self.cfg.d_model) if self.cfg.xscaling else 1.0
-            self._sub_out = ((s["out.weight"] * g).contiguous(), (s["out.bias"] * g).contiguous())
-        return F.linear(flat, *self._sub_out)
+            out = (s["out.weight"] * g).contiguous(), (s["out.bias"] * g).contiguous()
+            if not torch.cuda.is_current_stream_capturing():  # (a graph's tensors live in its pool)
+                self._sub_out = out
+        return F.linear(flat, *out)
 
-    def _subsample_split(self, feats: Tensor) -> Tensor:
-        w, (b, _, t) = self._sub_split, feats.shape
+    def _current_split(self, device) -> _SplitSubsampling | None:
+        """The laid-out subsampling weights, made again if a tensor of `self.sub` has changed since (not during a graph
+        capture, where the general kernels run instead)."""
+        w = self._sub_split
+        if w is None or w.holds(self.sub):
+            return w
+        self._sub_out = None
+        if torch.cuda.is_current_stream_capturing():
+            return None
+        w = _SplitSubsampling.prepare(self.sub, self.cfg)
+        torch.cuda.current_stream(device).synchronize()  # complete before a call on another stream finds it
+        self._sub_split = w
+        return w
+
+    def _subsample_split(self, w: _SplitSubsampling, feats: Tensor) -> Tensor:
+        b, _, t = feats.shape
         t2 = ((t - 1) // 2) // 2 + 1
         t3 = (t2 - 1) // 2 + 1
         L, st = _hip.lib(), _hip.stream_handle(feats.device)

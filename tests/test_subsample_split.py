@@ -152,6 +152,74 @@ def test_features_of_mixed_sizes():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("key", ["conv.0.weight", "conv.0.bias", "conv.2.weight", "conv.3.weight", "conv.3.bias", "conv.5.weight",
+                                 "conv.6.weight", "out.weight", "out.bias"])
+@pytest.mark.parametrize("how", ["in place", "replaced"])
+@pytest.mark.parametrize("inference", [False, True])
+def test_changed_weights_are_seen(key, how, inference):
+    """The call after a change to a weight uses it in every operand made from it, as a new model does."""
+    with torch.inference_mode(inference):
+        enc, feats = model(), torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(6)).cuda()
+        before = enc.subsample(feats)
+        if how == "in place":
+            enc.sub[key].mul_(1.5)
+        else:
+            enc.sub[key] = enc.sub[key] * 1.5
+        got, want = enc.subsample(feats).double().cpu(), exact(enc, feats)
+        assert not torch.equal(got, before.double().cpu())
+        assert float((got - want).abs().max() / want.abs().max()) < 1e-5
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_weights_changed_into_what_is_not_taken_and_back():
+    enc, feats = model(), torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(7)).cuda()
+    first = enc.subsample(feats)
+    kept = enc.sub["conv.0.weight"].clone()
+    enc.sub["conv.0.weight"][5] = 1e-12
+    want = exact(enc, feats)
+    assert float((enc.subsample(feats).double().cpu() - want).abs().max() / want.abs().max()) < 1e-5
+    enc.sub["conv.0.weight"].copy_(kept)
+    assert float((enc.subsample(feats) - first).abs().max() / first.abs().max()) < 1e-5
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_weights_at_any_address():
+    """Weights that are views into one buffer, off the alignment that the kernels' vector loads need."""
+    cfg = E.EncoderConfig(layers=1)
+    w = E.synthetic_weights(cfg, seed=4)
+    p = "encoder.pre_encode."
+    flat = torch.cat([torch.zeros(1)] + [w[k].flatten().float() for k in w if k.startswith(p)]).cuda()
+    at = 1
+    for k in [k for k in w if k.startswith(p)]:
+        w[k] = flat[at:at + w[k].numel()].view(w[k].shape)
+        at += w[k].numel()
+    feats = torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(8)).cuda()
+    assert torch.equal(E.FastConformerEncoder(w, cfg, "cuda", parts=1).subsample(feats), model().subsample(feats))
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_capture_after_a_change():
+    """A capture cannot lay the weights out: it takes the general kernels, and replays give their results."""
+    enc, feats = model(), torch.randn(2, 128, 64, generator=torch.Generator().manual_seed(9)).cuda()
+    enc.subsample(feats)
+    general(enc, feats)                       # (their libraries are set up before the capture)
+    enc.sub["conv.3.weight"].mul_(0.5)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = enc.subsample(feats)
+    for seed in range(3):
+        feats.copy_(torch.randn(2, 128, 64, generator=torch.Generator().manual_seed(20 + seed)))
+        graph.replay()
+        torch.cuda.synchronize()
+        want = exact(enc, feats)
+        assert float((out.double().cpu() - want).abs().max() / want.abs().max()) < 1e-5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m,n", [(1, 128), (127, 256), (128, 1024), (129, 128), (1000, 1024), (2100, 1024), (4000, 1024),
                                  (17000, 256)])
 @torch.inference_mode()
