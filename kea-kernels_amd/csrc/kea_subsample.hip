@@ -357,11 +357,12 @@ subsample1_kernel(const float *x, int T, int T1, int T2, const _Float16 *w1f, co
             const int p = 16 * mt + i;
             const float pm = plain ? 1.f : 1.0f / pscale[p];  // (powers of two: exact)
             const v4f d = acc[nt][mt];
+            // (the product of both scales may leave the range that the result stays in)
             if (p < rows * kF2)
-                *(float4 *)(yb + p * kC + n) = make_float4(fmaxf(__builtin_fmaf(d[0], wm.x * pm, bias.x), 0.f),
-                                                           fmaxf(__builtin_fmaf(d[1], wm.y * pm, bias.y), 0.f),
-                                                           fmaxf(__builtin_fmaf(d[2], wm.z * pm, bias.z), 0.f),
-                                                           fmaxf(__builtin_fmaf(d[3], wm.w * pm, bias.w), 0.f));
+                *(float4 *)(yb + p * kC + n) = make_float4(fmaxf(__builtin_fmaf(d[0] * wm.x, pm, bias.x), 0.f),
+                                                           fmaxf(__builtin_fmaf(d[1] * wm.y, pm, bias.y), 0.f),
+                                                           fmaxf(__builtin_fmaf(d[2] * wm.z, pm, bias.z), 0.f),
+                                                           fmaxf(__builtin_fmaf(d[3] * wm.w, pm, bias.w), 0.f));
         }
     }
 }
@@ -485,7 +486,7 @@ subsample2_kernel(const float *x, int T2, int T3, const float *w5, const float *
             const int n = 32 * wave + 16 * nt + 4 * g;
             const v4f bs = *(const v4f *)(b6 + n), wm = plain ? (v4f){1.f, 1.f, 1.f, 1.f} : *(const v4f *)(w6m + n);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[nt][mt][r] = fmaxf(__builtin_fmaf(acc[nt][mt][r], wm[r] * pm, bs[r]), 0.f);
+            for (int r = 0; r < 4; ++r) acc[nt][mt][r] = fmaxf(__builtin_fmaf(acc[nt][mt][r] * wm[r], pm, bs[r]), 0.f);
             m = kea::max_abs2(acc[nt][mt][0], acc[nt][mt][1], m);
             m = kea::max_abs2(acc[nt][mt][2], acc[nt][mt][3], m);
         }
@@ -537,7 +538,7 @@ __device__ __forceinline__ void finish(const _Float16 *x, const float *xs, const
         r = v + b;
     } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = __builtin_fmaf(v[e], sc[e] * s, b[e]);
+        for (int e = 0; e < 4; ++e) r[e] = __builtin_fmaf(v[e] * sc[e], s, b[e]);
     }
     *(v4f *)(y + m * N + n) = r;
 }

@@ -531,8 +531,9 @@ class _SplitSubsampling:
     def prepare(s: dict, cfg: EncoderConfig):
         """The layout, or None where the kernels do not take the model: they are written for 128 mel bins and 256
         channels (and an output in tiles of 128), a weight that is not finite has no split form (2^80 leaves the scaled sums
-        in range), and the first convolution's bias is held in units of its weights (nonzero rows from 2^-30, biases to 2^15,
-        so that it stays finite for any scale of the input). Waits for the GPU once."""
+        in range), and the first convolution's sums, its bias among them, are held in units of its weights and of the input
+        (nonzero rows from 2^-30, biases to 2^15, both layers' weights to 2^13, so that these units and what multiplies them
+        stay finite for any scale of the input). Waits for the GPU once."""
         if cfg.feat_in != 128 or cfg.sub_channels != 256 or s["out.weight"].shape[1] != 16 * 256 or cfg.d_model % 128:
             return None
         if any(v.is_inference() for v in s.values()):  # (a tensor that does not count its changes)
@@ -540,7 +541,7 @@ class _SplitSubsampling:
         tops = torch.stack([v.abs().amax() for v in s.values()])          # (NaN compares false)
         row = s["conv.0.weight"].reshape(256, 9).abs().amax(1)
         fits = ((tops <= 2.0**80).all() & ((row == 0) | (row >= 2.0**_SplitSubsampling.LEAST)).all()
-                & (s["conv.0.bias"].abs() <= 2**15).all())
+                & (s["conv.0.bias"].abs() <= 2**15).all() & (row <= 2**13).all() & (s["conv.2.weight"].abs() <= 2**13).all())
         if not fits.item():
             return None
         return _SplitSubsampling(s, math.sqrt(cfg.d_model) if cfg.xscaling else 1.0)

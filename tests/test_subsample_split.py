@@ -52,7 +52,8 @@ def test_split_weights_hold_fp32(n, k):
 
 
 @pytest.mark.parametrize("change,taken", [(None, True), ("inf", False), ("nan", False), ("tiny_row", False), ("zero_row", True),
-                                          ("bias", False), ("channels", False)])
+                                          ("bias", False), ("channels", False), ("huge", False), ("large_first", False),
+                                          ("large_second", False)])
 def test_models_that_are_taken(change, taken):
     """What has no split form, or is of another size, stays on the general kernels."""
     cfg = E.EncoderConfig(layers=1, sub_channels=128 if change == "channels" else 256)
@@ -62,6 +63,10 @@ def test_models_that_are_taken(change, taken):
         s["conv.3.weight"].view(-1)[7] = float(change)
     elif change in ("tiny_row", "zero_row"):
         s["conv.0.weight"][5] = 1e-10 if change == "tiny_row" else 0.0
+    elif change == "huge":
+        s["out.weight"][7, 7] = 2.0**81
+    elif change in ("large_first", "large_second"):
+        s["conv.0.weight" if change == "large_first" else "conv.2.weight"][7] = 1e4
     elif change == "bias":
         s["conv.0.bias"][9] = 1e5
     assert (E._SplitSubsampling.prepare(s, cfg) is not None) == taken
@@ -217,6 +222,21 @@ def test_capture_after_a_change():
         torch.cuda.synchronize()
         want = exact(enc, feats)
         assert float((out.double().cpu() - want).abs().max() / want.abs().max()) < 1e-5
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_scales_whose_product_leaves_the_range():
+    """Small values through small weights, the result still a normal number (and made ordinary by the next layer)."""
+    enc = model()
+    for key, power in [("conv.2.weight", -20), ("conv.3.weight", -54), ("conv.5.weight", 60), ("conv.6.weight", 59)]:
+        enc.sub[key].mul_(2.0**power)
+    for i in (0, 2, 3, 5, 6):
+        enc.sub[f"conv.{i}.bias"].zero_()
+    feats = torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(10)).cuda() * 2.0**-45
+    want, got, old = exact(enc, feats), enc.subsample(feats).double().cpu(), general(enc, feats).double().cpu()
+    print(_row_error(got, want), _row_error(old, want))
+    assert _row_error(got, want) <= 2 * _row_error(old, want)
 
 
 @pytest.mark.gpu
