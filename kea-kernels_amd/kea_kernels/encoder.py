@@ -488,6 +488,14 @@ def _fragments(planes: list) -> Tensor:
                        2).contiguous()
 
 
+def _narrow_rows(w: Tensor) -> Tensor:
+    """Whether the rows of w hold their smaller elements in split form: at most one in 64 nonzero elements of a row (two, of
+    short ones) below 2^-14 of its largest, which is held to 2^-25 of itself there. (A normal row of 4096 has one.)"""
+    size = w.abs()
+    low = ((size > 0) & (size < size.amax(1, keepdim=True) * 2.0**-14)).sum(1)
+    return (low <= max(2, w.shape[1] // 64)).all()
+
+
 class _SplitSubsampling:
     """The subsampling weights as kea_subsample_stage1 / stage2 / out read them, all of them copies: the pointwise
     convolutions as split FP16 fragments, the first convolution's nine taps as the 27 terms (hi, hi, lo against the
@@ -533,7 +541,8 @@ class _SplitSubsampling:
         channels (and an output in tiles of 128), a weight that is not finite has no split form (2^80 leaves the scaled sums
         in range), and the first convolution's sums, its bias among them, are held in units of its weights and of the input
         (nonzero rows from 2^-30, biases to 2^15, both layers' weights to 2^13, so that these units and what multiplies them
-        stay finite for any scale of the input). Waits for the GPU once."""
+        stay finite for any scale of the input). Rows of weights too far apart in size for one scale are left to FP32 as well
+        (_narrow_rows). Waits for the GPU once."""
         if cfg.feat_in != 128 or cfg.sub_channels != 256 or s["out.weight"].shape[1] != 16 * 256 or cfg.d_model % 128:
             return None
         if any(v.is_inference() for v in s.values()):  # (a tensor that does not count its changes)
@@ -542,6 +551,8 @@ class _SplitSubsampling:
         row = s["conv.0.weight"].reshape(256, 9).abs().amax(1)
         fits = ((tops <= 2.0**80).all() & ((row == 0) | (row >= 2.0**_SplitSubsampling.LEAST)).all()
                 & (s["conv.0.bias"].abs() <= 2**15).all() & (row <= 2**13).all() & (s["conv.2.weight"].abs() <= 2**13).all())
+        for name in ("conv.0.weight", "conv.3.weight", "conv.6.weight", "out.weight"):
+            fits &= _narrow_rows(s[name].reshape(s[name].shape[0], -1))
         if not fits.item():
             return None
         return _SplitSubsampling(s, math.sqrt(cfg.d_model) if cfg.xscaling else 1.0)

@@ -53,7 +53,7 @@ def test_split_weights_hold_fp32(n, k):
 
 @pytest.mark.parametrize("change,taken", [(None, True), ("inf", False), ("nan", False), ("tiny_row", False), ("zero_row", True),
                                           ("bias", False), ("channels", False), ("huge", False), ("large_first", False),
-                                          ("large_second", False)])
+                                          ("large_second", False), ("wide_row", False), ("wide_out", False)])
 def test_models_that_are_taken(change, taken):
     """What has no split form, or is of another size, stays on the general kernels."""
     cfg = E.EncoderConfig(layers=1, sub_channels=128 if change == "channels" else 256)
@@ -63,6 +63,8 @@ def test_models_that_are_taken(change, taken):
         s["conv.3.weight"].view(-1)[7] = float(change)
     elif change in ("tiny_row", "zero_row"):
         s["conv.0.weight"][5] = 1e-10 if change == "tiny_row" else 0.0
+    elif change in ("wide_row", "wide_out"):
+        s["conv.3.weight" if change == "wide_row" else "out.weight"][7, 7] = 2.0**18
     elif change == "huge":
         s["out.weight"][7, 7] = 2.0**81
     elif change in ("large_first", "large_second"):
@@ -234,6 +236,20 @@ def test_scales_whose_product_leaves_the_range():
     for i in (0, 2, 3, 5, 6):
         enc.sub[f"conv.{i}.bias"].zero_()
     feats = torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(10)).cuda() * 2.0**-45
+    want, got, old = exact(enc, feats), enc.subsample(feats).double().cpu(), general(enc, feats).double().cpu()
+    print(_row_error(got, want), _row_error(old, want))
+    assert _row_error(got, want) <= 2 * _row_error(old, want)
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_a_large_weight_of_a_dead_channel():
+    """A weight 2^24 times the others of its row for an input that is always zero: what the others give is as accurate as
+    with the general kernels."""
+    enc = model()
+    enc.sub["conv.5.weight"][3], enc.sub["conv.5.bias"][3] = 0.0, 0.0
+    enc.sub["conv.6.weight"][:, 3] *= 2.0**24
+    feats = torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(11)).cuda()
     want, got, old = exact(enc, feats), enc.subsample(feats).double().cpu(), general(enc, feats).double().cpu()
     print(_row_error(got, want), _row_error(old, want))
     assert _row_error(got, want) <= 2 * _row_error(old, want)
