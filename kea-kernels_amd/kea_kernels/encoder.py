@@ -490,10 +490,19 @@ def _fragments(planes: list) -> Tensor:
 
 def _narrow_rows(w: Tensor) -> Tensor:
     """Whether the rows of w hold their smaller elements in split form: at most one in 64 nonzero elements of a row (two, of
-    short ones) below 2^-14 of its largest, which is held to 2^-25 of itself there. (A normal row of 4096 has one.)"""
+    short rows) below 2^-14 of its largest, which is held to 2^-25 of itself there. (A normal row of 4096 has one.)"""
     size = w.abs()
     low = ((size > 0) & (size < size.amax(1, keepdim=True) * 2.0**-14)).sum(1)
     return (low <= max(2, w.shape[1] // 64)).all()
+
+
+def _channel_sizes(s: dict) -> Tensor:
+    """How large the 256 channels are beside each other, by their weights, where a scale is shared: at a position in front
+    of either pointwise convolution and in a row of the output linear's input. [3, 256]."""
+    top = {k: v.reshape(256, -1).abs().amax(1) for k, v in s.items() if k.startswith("conv.")}
+    w, b = (lambda i: top[f"conv.{i}.weight"]), (lambda i: top[f"conv.{i}.bias"])
+    return torch.stack([torch.maximum(torch.maximum(w(0), b(0)) * w(2), b(2)),
+                        torch.maximum(torch.maximum(w(3), b(3)) * w(5), b(5)), torch.maximum(w(6), b(6))])
 
 
 class _SplitSubsampling:
@@ -541,8 +550,8 @@ class _SplitSubsampling:
         channels (and an output in tiles of 128), a weight that is not finite has no split form (2^80 leaves the scaled sums
         in range), and the first convolution's sums, its bias among them, are held in units of its weights and of the input
         (nonzero rows from 2^-30, biases to 2^15, both layers' weights to 2^13, so that these units and what multiplies them
-        stay finite for any scale of the input). Rows of weights too far apart in size for one scale are left to FP32 as well
-        (_narrow_rows). Waits for the GPU once."""
+        stay finite for any scale of the input). Weights, or channels by their weights, too far apart in size for the scale
+        that they share are left to FP32 as well (_narrow_rows). Waits for the GPU once."""
         if cfg.feat_in != 128 or cfg.sub_channels != 256 or s["out.weight"].shape[1] != 16 * 256 or cfg.d_model % 128:
             return None
         if any(v.is_inference() for v in s.values()):  # (a tensor that does not count its changes)
@@ -553,6 +562,7 @@ class _SplitSubsampling:
                 & (s["conv.0.bias"].abs() <= 2**15).all() & (row <= 2**13).all() & (s["conv.2.weight"].abs() <= 2**13).all())
         for name in ("conv.0.weight", "conv.3.weight", "conv.6.weight", "out.weight"):
             fits &= _narrow_rows(s[name].reshape(s[name].shape[0], -1))
+        fits &= _narrow_rows(_channel_sizes(s))
         if not fits.item():
             return None
         return _SplitSubsampling(s, math.sqrt(cfg.d_model) if cfg.xscaling else 1.0)

@@ -53,7 +53,8 @@ def test_split_weights_hold_fp32(n, k):
 
 @pytest.mark.parametrize("change,taken", [(None, True), ("inf", False), ("nan", False), ("tiny_row", False), ("zero_row", True),
                                           ("bias", False), ("channels", False), ("huge", False), ("large_first", False),
-                                          ("large_second", False), ("wide_row", False), ("wide_out", False)])
+                                          ("large_second", False), ("wide_row", False), ("wide_out", False),
+                                          ("wide_channels", False), ("wide_second", False), ("wide_last", False)])
 def test_models_that_are_taken(change, taken):
     """What has no split form, or is of another size, stays on the general kernels."""
     cfg = E.EncoderConfig(layers=1, sub_channels=128 if change == "channels" else 256)
@@ -63,6 +64,11 @@ def test_models_that_are_taken(change, taken):
         s["conv.3.weight"].view(-1)[7] = float(change)
     elif change in ("tiny_row", "zero_row"):
         s["conv.0.weight"][5] = 1e-10 if change == "tiny_row" else 0.0
+    elif change in ("wide_channels", "wide_second", "wide_last"):
+        if change == "wide_channels":                # (each layer within its own range)
+            s["conv.0.weight"][11] *= 2.0**5
+        s[{"wide_channels": "conv.2.weight", "wide_second": "conv.5.weight", "wide_last": "conv.6.weight"}[change]][11] *= (
+            2.0**12 if change == "wide_channels" else 2.0**17)
     elif change in ("wide_row", "wide_out"):
         s["conv.3.weight" if change == "wide_row" else "out.weight"][7, 7] = 2.0**18
     elif change == "huge":
@@ -250,6 +256,20 @@ def test_a_large_weight_of_a_dead_channel():
     enc.sub["conv.5.weight"][3], enc.sub["conv.5.bias"][3] = 0.0, 0.0
     enc.sub["conv.6.weight"][:, 3] *= 2.0**24
     feats = torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(11)).cuda()
+    want, got, old = exact(enc, feats), enc.subsample(feats).double().cpu(), general(enc, feats).double().cpu()
+    print(_row_error(got, want), _row_error(old, want))
+    assert _row_error(got, want) <= 2 * _row_error(old, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("large,reader", [("conv.2", "conv.3"), ("conv.5", "conv.6"), ("conv.6", "out")])
+@torch.inference_mode()
+def test_a_large_channel_that_is_not_read(large, reader):
+    enc = model()
+    enc.sub[large + ".weight"][3] *= 2.0**24
+    w = enc.sub[reader + ".weight"]
+    (w[:, 3] if reader != "out" else w.view(-1, 256, 16)[:, 3]).zero_()
+    feats = torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(12)).cuda()
     want, got, old = exact(enc, feats), enc.subsample(feats).double().cpu(), general(enc, feats).double().cpu()
     print(_row_error(got, want), _row_error(old, want))
     assert _row_error(got, want) <= 2 * _row_error(old, want)
