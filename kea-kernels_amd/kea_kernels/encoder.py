@@ -303,15 +303,24 @@ def relpos_attention(qkv: Tensor, pos: Tensor, bias_u: Tensor, bias_v: Tensor, h
     return out
 
 
+ATTENTION_SCRATCH = 1 << 30  # bytes of workspace that a tiled attention call allocates (or what one clip takes)
+
+
 def _attention_tiled(args: tuple, out: Tensor) -> Tensor:
     """kea_relpos_attention_tiled of checked arguments with a workspace of its own (stream ordered: torch's allocator
-    may hand it out again once the launches are enqueued)."""
+    may hand it out again once the launches are enqueued). Its size grows with the batch, twice the input's, so large
+    batches go in groups of clips that share one."""
     L = _hip.lib()
-    batch, t, heads = args[8], args[9], args[10]
-    need = L.kea_relpos_attention_tiled_workspace(batch, t, heads)
-    ws = torch.empty(need, dtype=torch.uint8, device=out.device)
-    _hip.check(L.kea_relpos_attention_tiled(*args, ws.data_ptr(), need, _hip.stream_handle(out.device)),
-               "kea_relpos_attention_tiled")
+    qkv, ld, pos, ldp, u, v, y, ldo, batch, t, heads, dk, scale = args
+    one = L.kea_relpos_attention_tiled_workspace(1, t, heads)
+    clip = L.kea_relpos_attention_tiled_workspace(2, t, heads) - one
+    group = max(1, min(batch, 1 + (ATTENTION_SCRATCH - one) // max(clip, 1)))
+    need = L.kea_relpos_attention_tiled_workspace(group, t, heads)
+    ws, stream = torch.empty(need, dtype=torch.uint8, device=out.device), _hip.stream_handle(out.device)
+    for i in range(0, max(batch, 1), group):
+        _hip.check(L.kea_relpos_attention_tiled(qkv + 4 * i * t * ld, ld, pos, ldp, u, v, y + 4 * i * t * ldo, ldo,
+                                                min(group, batch - i), t, heads, dk, scale, ws.data_ptr(), need, stream),
+                   "kea_relpos_attention_tiled")
     return out
 
 

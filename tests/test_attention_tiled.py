@@ -260,6 +260,28 @@ def test_layer_attention_routes(monkeypatch):
 
 
 @pytest.mark.gpu
+def test_scratch_is_bounded_whatever_the_batch():
+    """300 clips, 0.94 GB of workspace in one call, with the bound lowered: the scratch stays below it, the bits are a
+    single clip's; an empty batch allocates nothing to speak of."""
+    b, t, bound = 300, 130, 64 << 20
+    qkv = torch.randn(b, t, 3 * D, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    _, pos, u, v = (a.cuda() for a in _inputs(1, t, 17))
+    want = [E.relpos_attention(qkv[i:i + 1], pos, u, v, H) for i in (0, 1, 157, 299)]
+    torch.cuda.synchronize()
+    keep, E.ATTENTION_SCRATCH = getattr(E, "ATTENTION_SCRATCH", None), bound
+    try:
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        got = E.relpos_attention(qkv, pos, u, v, H)
+        peak = torch.cuda.max_memory_allocated() - before - got.numel() * 4
+    finally:
+        E.ATTENTION_SCRATCH = keep
+    assert peak <= bound + 512
+    assert all(torch.equal(got[i], w[0]) for i, w in zip((0, 1, 157, 299), want))
+    assert E.relpos_attention(qkv[:0], pos, u, v, H).shape == (0, t, D)
+
+
+@pytest.mark.gpu
 def test_graph_replays_equal_eager():
     """Captured with its workspace from the graph's pool; every replay equals the eager result on new inputs."""
     qkv, pos, u, v = (a.cuda() for a in _inputs(1, 200, 11))
