@@ -44,6 +44,8 @@ import numpy as np
 import torch
 import torch.nn.functional as F
 from torch import Tensor
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from kea_kernels import _hip, formats, lowbit
 from kea_kernels.binary import bits, layer_parts, provider
@@ -335,7 +337,9 @@ def _plain_f32(t: Tensor, device) -> bool:
 def _traced() -> bool:
     """Whether PyTorch operators called now are recorded or differentiated forward rather than only run."""
     return (torch.autograd.forward_ad._current_level >= 0 or torch.jit.is_tracing() or torch.compiler.is_compiling()
-            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0)
+            or torch._C._len_torch_dispatch_stack() > 0
+            or (torch._C._len_torch_function_stack() > 0 and any(  # (a default device only says where tensors are made)
+                type(mode) is not DeviceContext for mode in _get_current_function_mode_stack())))
 
 
 def _takes_tiled(qkv: Tensor, pos: Tensor, u: Tensor, v_bias: Tensor, heads: int) -> bool:

@@ -252,11 +252,20 @@ def test_layer_attention_routes(monkeypatch):
     assert calls == [1, 1, 1]
     batched = torch.func.vmap(lambda q: model.attention(q, pos, u, v))(torch.stack([qkv, 2 * qkv]))
     _close(batched[0].cpu(), ref, 1e-5)
+    class Watching(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Watching():                                                           # a mode that may rewrite operators
+        _close(model.attention(qkv, pos, u, v).cpu(), ref, 1e-5)
     with pytest.raises((ValueError, RuntimeError)):
         model.attention(qkv.double(), pos, u, v)                               # mixed types: PyTorch refuses
     assert calls == [1, 1, 1]
     with pytest.raises(ValueError, match="256 frames"):
         E.relpos_attention(qkv, pos, u, v, H)
+    with torch.device("cuda"):                                                 # a default device is no such mode
+        _close(model.attention(qkv, pos, u, v).cpu(), ref)
+    assert calls == [1, 1, 1, 1]
 
 
 @pytest.mark.gpu
