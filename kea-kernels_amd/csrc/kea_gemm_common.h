@@ -230,13 +230,8 @@ __device__ __forceinline__ void load_col4(const void *v, int dtype, int nb, int 
     for (int r = 0; r < 4; ++r) out[r] = f[r];
 }
 
-__device__ __forceinline__ void load_col_scales(const Params &p, int nb, EpiOperands &e, bool with_alpha = true) {
-    if (with_alpha) {
-        load_col4(p.ws, p.ws_dtype, nb, p.N, e.alpha);
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) e.alpha[r] = 0.f;
-    }
+__device__ __forceinline__ void load_col_scales(const Params &p, int nb, EpiOperands &e) {
+    load_col4(p.ws, p.ws_dtype, nb, p.N, e.alpha);
     if (p.bias) {
         load_col4(p.bias, p.bias_dtype, nb, p.N, e.bias);
     } else {
@@ -274,21 +269,16 @@ __device__ __forceinline__ void epilogue4(const Params &p, int m, int nb, const 
 }
 
 // The values of 4 consecutive columns from exact accumulators, with the choices known at compile time (a run-time SiLU
-// flag makes the compiler evaluate the SiLU for every output and select). RES: the residual e.res is applied. SILU:
-// 1 / 0 the SiLU is / is not applied, -1: as Params::flags says. SMALL: the residual and the bias as Params say.
-template <int P, bool RES, bool SMALL, int SILU>
+// flag makes the compiler evaluate the SiLU for every output and select). RES: the residual e.res is applied.
+// SILU: the SiLU is applied.
+template <int P, bool RES, bool SILU>
 __device__ __forceinline__ void epilogue4_values(const Params &p, const int (*a)[4], const EpiOperands &e, float (&v)[4]) {
-    const int flags = SILU < 0 ? p.flags : SILU ? (p.flags | KEA_FLAG_SILU) : (p.flags & ~KEA_FLAG_SILU);
+    const int flags = SILU ? (p.flags | KEA_FLAG_SILU) : (p.flags & ~KEA_FLAG_SILU);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         int ar[3] = {a[0][r], P > 1 ? a[1][r] : 0, P > 2 ? a[2][r] : 0};
-        if constexpr (SMALL) {
-            v[r] = finish(combine<P>(ar, e.s, flags), e.alpha[r], p.bias != nullptr, e.bias[r], flags);
-            if (p.res) v[r] = e.res[r] + v[r] * p.res_factor;
-        } else {
-            v[r] = finish(combine<P>(ar, e.s, flags), e.alpha[r], e.bias[r], flags);
-            if constexpr (RES) v[r] = e.res[r] + v[r] * p.res_factor;
-        }
+        v[r] = finish(combine<P>(ar, e.s, flags), e.alpha[r], e.bias[r], flags);
+        if constexpr (RES) v[r] = e.res[r] + v[r] * p.res_factor;
     }
 }
 // Two FP32 values rounded to FP16 / BF16 as one word (see to_f16_bits for the empty asm).
@@ -317,13 +307,13 @@ __device__ __forceinline__ void put4_as(const float (&v)[4], Put put) {
     }
 }
 // epilogue4 for an output without raw accumulators, of compile-time dtype DT, whose 4 columns are all inside N with a
-// vector-aligned y: the same values, one vector store, no per-lane selection.
-template <int P, int DT, bool RES, bool SMALL, int SILU = -1, bool GLU = false>
+// vector-aligned y, without a residual: the same values, one vector store, no per-lane selection.
+template <int P, int DT, bool SILU, bool GLU = false>
 __device__ __forceinline__ void epilogue4_full(const Params &p, void *yrow, int nb, const int (*a)[4],
                                                const EpiOperands &e) {
-    static_assert(!GLU || (!RES && SILU == 0), "the GLU output takes neither a residual nor the SiLU");
+    static_assert(!GLU || !SILU, "the GLU output takes no SiLU");
     float v[4];
-    epilogue4_values<P, RES, SMALL, SILU>(p, a, e, v);
+    epilogue4_values<P, false, SILU>(p, a, e, v);
     char *dst = (char *)yrow + (GLU ? nb / 2 : nb) * (DT == KEA_F32 ? 4 : 2);
     put4_as<DT, GLU>(v, [&](auto bits) { *(decltype(bits) *)dst = bits; });
 }

@@ -523,7 +523,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64, DEEP ? 2 : 1) gemm_kernel
                         e.res[0] = v.x; e.res[1] = v.y; e.res[2] = v.z; e.res[3] = v.w;
                     }
                     float v[4];
-                    epilogue4_values<P, RES, false, SILU ? 1 : 0>(p, a, e, v);
+                    epilogue4_values<P, RES, SILU>(p, a, e, v);
                     put4_as<DT, GLU>(v, [&](auto bits) {
                         const int at = (int)(row_at[i] + col_at);
                         if constexpr (sizeof(bits) == 16) __builtin_amdgcn_raw_buffer_store_b128(bits, view, at, 0, 0);

@@ -205,18 +205,18 @@ __device__ __forceinline__ void wsplit_epilogue(const Params &p, bool plain, int
         uint16_t *y16 = (uint16_t *)p.y + (long long)m * p.ldy;
         float *y32 = (float *)p.y + (long long)m * p.ldy;
         if (p.flags & KEA_FLAG_GLU) {  // the library refuses GLU with the SiLU
-            if (p.y_dtype == KEA_F16) epilogue4_full<P, KEA_F16, false, false, 0, true>(p, y16, nb, a, e);
-            else if (p.y_dtype == KEA_BF16) epilogue4_full<P, KEA_BF16, false, false, 0, true>(p, y16, nb, a, e);
-            else epilogue4_full<P, KEA_F32, false, false, 0, true>(p, y32, nb, a, e);
+            if (p.y_dtype == KEA_F16) epilogue4_full<P, KEA_F16, false, true>(p, y16, nb, a, e);
+            else if (p.y_dtype == KEA_BF16) epilogue4_full<P, KEA_BF16, false, true>(p, y16, nb, a, e);
+            else epilogue4_full<P, KEA_F32, false, true>(p, y32, nb, a, e);
         } else if (p.y_dtype == KEA_F16) {
-            if (silu) epilogue4_full<P, KEA_F16, false, false, 1>(p, y16, nb, a, e);
-            else epilogue4_full<P, KEA_F16, false, false, 0>(p, y16, nb, a, e);
+            if (silu) epilogue4_full<P, KEA_F16, true>(p, y16, nb, a, e);
+            else epilogue4_full<P, KEA_F16, false>(p, y16, nb, a, e);
         } else if (p.y_dtype == KEA_BF16) {
-            if (silu) epilogue4_full<P, KEA_BF16, false, false, 1>(p, y16, nb, a, e);
-            else epilogue4_full<P, KEA_BF16, false, false, 0>(p, y16, nb, a, e);
+            if (silu) epilogue4_full<P, KEA_BF16, true>(p, y16, nb, a, e);
+            else epilogue4_full<P, KEA_BF16, false>(p, y16, nb, a, e);
         } else {
-            if (silu) epilogue4_full<P, KEA_F32, false, false, 1>(p, y32, nb, a, e);
-            else epilogue4_full<P, KEA_F32, false, false, 0>(p, y32, nb, a, e);
+            if (silu) epilogue4_full<P, KEA_F32, true>(p, y32, nb, a, e);
+            else epilogue4_full<P, KEA_F32, false>(p, y32, nb, a, e);
         }
     } else {
         epilogue4<P>(p, m, nb, a, e);
