@@ -65,8 +65,9 @@ static_assert(kKS == 2 && 16 * kQG == kRows && 32 * kKS == kRows, "queries, keys
 constexpr int kPlane = kRows * kDK;             // elements of one plane of a block
 constexpr int kBlockBytes = 2 * kPlane * 2;     // hi and lo planes
 // Rows that the split form would not hold to FP32's accuracy go to the FP32 form. A value row's elements are held to 2^-31 of
-// the row's largest (with their probabilities): a row with kLowPairs or more nonzero pairs of elements 2^10 below it is not
-// split (a normal row's pair is that small once in 10^5, four of 64 at once in 10^14). An element of Q, K or P is held to 2^-39
+// the row's largest (with their probabilities): a wave's 16 rows with nonzero pairs of elements 2^10 below their row's largest
+// in kLowPairs or more of the 64 columns of pairs are not split (a normal pair is that small once in 10^5, four of the 1024
+// once in 10^10). An element of Q, K or P is held to 2^-39
 // of its row's largest (K and P: of four rows'), which costs a score at most 2^-31 of the largest query element times the
 // largest of K and P times the scale, and that if every element of the rows is so small: up to kScores, 2^-25 measured,
 // what FP32 rounds off a score of ordinary rows.
@@ -212,30 +213,35 @@ split_kernel(const float *qkv, long long ld, const float *pos, long long ldp, co
             v[u][e][1] = w.y;
         }
     rows(kbase, ld, j0, T, (_Float16 *)(so.k + (long long)id * kBlockBytes), so.km + (long long)id * 16);
+    // A scale per key: its row may be any size beside the others'. Key index x + 4 y: the exponents are formed in the lanes of
+    // row y and the scales read from there (16 of each in scalar instructions took half a microsecond).
+    float pair[16], most[4], sf[16];
+    int ex[4];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) pair[k] = max_abs<2>(v[k >> 3][k & 7]);
+    kea::wave_max_rows(pair, most);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        ex[x] = exponent_of(__builtin_bit_cast(int, most[x]));
+#pragma unroll
+        for (int y = 0; y < 4; ++y) sf[x + 4 * y] = kea::lane_value(pow2(14 - ex[x]), 16 * y);
+    }
+    if (n == 0) *(int4 *)(so.ve + (long long)id * kRows + 16 * g + 4 * wave) = make_int4(ex[0], ex[1], ex[2], ex[3]);
+    bool low = false;  // (a row's largest is scaled to [2^14, 2^15))
+#pragma unroll
+    for (int k = 0; k < 16; ++k) low = low || (pair[k] != 0.f && pair[k] * sf[k] < 16.f);
+    const bool infinite = fmaxf(fmaxf(most[0], most[1]), fmaxf(most[2], most[3])) >= __builtin_inff();
+    if (__any(infinite) || __popcll(__ballot(low)) >= kLowPairs) seen = kInfBits;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const int grp = 4 * u + wave;
-        int e[8];  // a scale per key: its row may be any size beside the others'
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const float pair = max_abs<2>(v[u][k]);
-            const int bits = wave_max_bits(pair);
-            e[k] = exponent_of(bits);
-            const bool low = pair > 0.f && pair < __builtin_bit_cast(float, bits) * 0x1p-10f;
-            if (bits >= kInfBits || __popcll(__ballot(low)) >= kLowPairs) seen = kInfBits;
-        }
-        if (lane == 0)
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-                *(int4 *)(so.ve + (long long)id * kRows + 32 * u + 16 * t + 4 * wave) =
-                    make_int4(e[4 * t], e[4 * t + 1], e[4 * t + 2], e[4 * t + 3]);
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             v8h hi, lo;
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
                 _Float16 h, l;
-                split1(v[u][k][c], pow2(14 - e[k]), h, l);
+                split1(v[u][k][c], sf[8 * u + k], h, l);
                 hi[k] = h;
                 lo[k] = l;
             }
@@ -545,17 +551,16 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
     const float m1 = mb[32], mm = fmaxf(m_ref, m1);
     const float a0 = __builtin_amdgcn_exp2f(m_ref - mm), a1 = __builtin_amdgcn_exp2f(m1 - mm);
     const float inv = 1.0f / __builtin_fmaf(mb[33], a1, l_run * a0);
-    // each half times 2^(em + m - mm) / l, the exponent last: neither leaves FP32's range before the result does
-    const int e0 = em + (int)fmaxf(m_ref - mm, -1e6f);
-    const int e1 = __builtin_bit_cast(int, mb[34]) + (int)fmaxf(m1 - mm, -1e6f);
+    // each half times 2^(em + m - mm) / l, their common exponent last: nothing leaves FP32's range before the result does
+    const int e0 = em + (int)fmaxf(m_ref - mm, -1e6f), e1 = __builtin_bit_cast(int, mb[34]) + (int)fmaxf(m1 - mm, -1e6f);
+    const int et = max(e0, e1);
+    const float f0 = pow2(max(e0 - et, -127)) * inv, f1 = pow2(max(e1 - et, -127)) * inv;
     if (iq < T) {
         float *dst = out + ((long long)b * T + iq) * ldo + (long long)h * kDK + 4 * g;
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
             const float4 w = *(const float4 *)(mb + 4 * d);
-            auto sum = [&](float x0, float x1) {
-                return __builtin_amdgcn_ldexpf(x0 * inv, e0) + __builtin_amdgcn_ldexpf(x1 * inv, e1);
-            };
+            auto sum = [&](float x0, float x1) { return __builtin_amdgcn_ldexpf(__builtin_fmaf(x1, f1, x0 * f0), et); };
             *(float4 *)(dst + 16 * d) = make_float4(sum(o[d][0], w.x), sum(o[d][1], w.y), sum(o[d][2], w.z), sum(o[d][3], w.w));
         }
     }

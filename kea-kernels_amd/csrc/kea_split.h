@@ -66,6 +66,24 @@ __device__ __forceinline__ int wave_max_bits(float m) {
     return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
                max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
+// The wave's maxima of sixteen non-negative values: top[x] holds that of m[x + 4 y] in the lanes of row y (16 lanes). The halves
+// of two registers trade places, then the rows, so that a step's maximum halves the number of registers: 12 swaps and 4 row
+// maxima where one value after the other takes 16 of them.
+__device__ __forceinline__ void wave_max_rows(const float *m, float *top) {
+    uint32_t r[16];
+#pragma unroll
+    for (int x = 0; x < 16; ++x) r[x] = __builtin_bit_cast(uint32_t, m[x]);
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {  // lanes 0 - 31: value x, 32 - 63: x + 8
+        const auto v = __builtin_amdgcn_permlane32_swap(r[x], r[x + 8], false, false);
+        r[x] = max(v[0], v[1]);
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        const auto v = __builtin_amdgcn_permlane16_swap(r[x], r[x + 4], false, false);
+        top[x] = max16(__builtin_bit_cast(float, max(v[0], v[1])));
+    }
+}
 constexpr int kInfBits = 0x7f800000;
 
 __device__ __forceinline__ v4f mfma_f16(v8h a, v8h b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
