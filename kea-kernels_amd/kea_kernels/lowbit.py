@@ -291,7 +291,7 @@ def _native_quantize(x, rows, m, k, parts, norm, input_activation, qs_dtype, ldq
         xb, xt, xk, t = rows
         nw, nb, eps = (None, None, 0.0) if norm is None else (norm.weight.detach(), norm.bias.detach(), float(norm.eps))
         ldq = round_up(k, 16) if ldq is None else ldq
-        hit = _hip.native().quantize(x, xb, xt, xk, max(t, 1), m, k, parts, nw, nb, eps, input_activation == "silu",
+        hit = _hip.native().quantize(x, xb, xt, xk, t, m, k, parts, nw, nb, eps, input_activation == "silu",
                                      qs_dtype, ldq)
         return hit and (hit[0], hit[1], ldq)
     except (AttributeError, TypeError, ValueError):
@@ -440,7 +440,8 @@ class Launches:
     def remember(self, key, e: _Entry, out_shape: tuple) -> None:
         """Keeps a projection entry under an operator's own key: a tuple of the call's inputs (tensor shapes,
         strides, dtypes, device) from which the operator derives every argument it checks and passes, so that a call
-        with the same key may skip to launch(). Up to `max_entries` keys (the oldest is dropped first)."""
+        with the same key may skip to launch(). Only inputs that replay() declines get here (tensor subclasses, tensors
+        that require grad). Up to `max_entries` keys (the oldest is dropped first)."""
         if len(self._calls) >= self.max_entries:
             self._calls.pop(next(iter(self._calls)), None)
         self._calls[key] = (e, out_shape)

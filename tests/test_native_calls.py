@@ -196,7 +196,7 @@ def test_refused_arguments_raise_as_before():
                          (dict(ws_group=96), ""), (dict(residual=y.half()), "residual must be")]:
         with pytest.raises(ValueError, match=message):
             gemm(**bad)
-    for rows, m in [((0, 272, 1, 9), 9), ((0, 273, 1, 8), 8), ((0, 272, 2, 8), 8), ((0, -1, 1, 8), 8)]:
+    for rows, m in [((0, 272, 1, 9), 9), ((0, 273, 1, 8), 8), ((0, 272, 2, 8), 8), ((0, -1, 1, 8), 8), ((272, 272, 1, 0), 8)]:
         with pytest.raises(ValueError):
             lowbit.quantize(torch.randn(8, 272, device=DEV), rows, m, 272, 2)
 
