@@ -14,8 +14,8 @@
 //
 // Measured on eight 10-second clips (T = 1000): 50 + 26 + 34 us, where five launches and a library GEMM take 53 + 90 +
 // 25 + 27 + 25 + 70 us; one clip 15 + 15 + 17 us.
-// Kernel 1 executes 1850 vector instructions and 232 MFMAs a wave, and the two hardly overlap: about 27 and 12 us of its
-// 50 at the clock it runs at, the rest waits between its phases. Two rows of 32 positions to a workgroup, two workgroups to
+// Kernel 1 executes 1830 vector instructions and 232 MFMAs a wave, which at 2.4 GHz take 24 and 12 us of its 50 and hardly
+// overlap; LDS takes 11, and the waves wait for 38% of their time. Two rows of 32 positions to a workgroup, two workgroups to
 // a CU, is the split that measured best: four rows (one workgroup to a CU, half the weight reads) take 60 and, for one
 // clip, 25 us. Kernel 2 is latency: the weights (256 KB a workgroup) and its input from L2; half the rows to a workgroup
 // take 37 us, as the weights are read twice as often. Kernel 3 is bound by L2: 268 MB of operands in 26 us, then 16 MB of
@@ -24,6 +24,7 @@
 
 #include <cstdint>
 #include <string>
+#include <type_traits>
 
 #include "kea_internal.h"
 #include "kea_split.h"
@@ -466,6 +467,37 @@ subsample2_kernel(const float *x, int T2, int T3, const float *w5, const float *
         for (int w = 0; w < kWaves; ++w) big = max(big, tops[w * kRows3 + r]);
         return big;
     };
+    // A copy for each form: where their sums met in one, the compiler moved them (26.1 against 25.1 us; in kernel 1 the copies
+    // are the slower ones).
+    auto epilogue = [&](auto split_tag, v4f (&acc)[2][kPos2 / 16]) {
+        constexpr bool SPLIT = decltype(split_tag)::value;
+#pragma unroll
+        for (int mt = 0; mt < kPos2 / 16; ++mt) {  // m-tile = output row, m = its column
+            const float pm = SPLIT ? pscale[16 * mt + i] : 1.f;
+            float m = 0.f;
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) {
+                const int n = 32 * wave + 16 * nt + 4 * g;
+                const v4f bs = *(const v4f *)(b6 + n), wm = SPLIT ? *(const v4f *)(w6m + n) : (v4f){1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[nt][mt][r] = fmaxf(__builtin_fmaf(acc[nt][mt][r] * wm[r], pm, bs[r]), 0.f);
+                m = kea::max_abs2(acc[nt][mt][0], acc[nt][mt][1], m);
+                m = kea::max_abs2(acc[nt][mt][2], acc[nt][mt][3], m);
+            }
+            const int t = kea::wave_max_bits(m);
+            if (lane == 0) tops[wave * kRows3 + mt] = t;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int mt = 0; mt < kPos2 / 16; ++mt) {
+            if (mt >= rows) continue;
+            const int big = row_scale(mt), e = exponent_of(big);
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+                store(mt, i * kC + 32 * wave + 16 * nt + 4 * g, acc[nt][mt], pow2(14 - e), big >= kInfBits);
+            if (tid == 0) ys[row0 + mt] = big >= kInfBits ? __builtin_inff() : pow2(e - 14);
+        }
+    };
     v4f acc[2][kPos2 / 16];
     if (plain) {  // an infinity: the same sums in FP32
         float *const h = (float *)lds;  // [kPos2][256]
@@ -474,34 +506,10 @@ subsample2_kernel(const float *x, int T2, int T3, const float *w5, const float *
             *(float4 *)(h + fp32_at(16 * q + f0 + c, 4 * lane)) = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
         __syncthreads();
         pointwise_fp32<kPos2 / 16>(h, w6, wave, lane, acc);
+        epilogue(std::false_type{}, acc);
     } else {
         pointwise<kPos2 / 16>(tile, weights, lane, acc);
-    }
-#pragma unroll
-    for (int mt = 0; mt < kPos2 / 16; ++mt) {  // m-tile = output row, m = its column
-        const float pm = plain ? 1.f : pscale[16 * mt + i];
-        float m = 0.f;
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-            const int n = 32 * wave + 16 * nt + 4 * g;
-            const v4f bs = *(const v4f *)(b6 + n), wm = plain ? (v4f){1.f, 1.f, 1.f, 1.f} : *(const v4f *)(w6m + n);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[nt][mt][r] = fmaxf(__builtin_fmaf(acc[nt][mt][r] * wm[r], pm, bs[r]), 0.f);
-            m = kea::max_abs2(acc[nt][mt][0], acc[nt][mt][1], m);
-            m = kea::max_abs2(acc[nt][mt][2], acc[nt][mt][3], m);
-        }
-        const int t = kea::wave_max_bits(m);
-        if (lane == 0) tops[wave * kRows3 + mt] = t;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int mt = 0; mt < kPos2 / 16; ++mt) {
-        if (mt >= rows) continue;
-        const int big = row_scale(mt), e = exponent_of(big);
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-            store(mt, i * kC + 32 * wave + 16 * nt + 4 * g, acc[nt][mt], pow2(14 - e), big >= kInfBits);
-        if (tid == 0) ys[row0 + mt] = big >= kInfBits ? __builtin_inff() : pow2(e - 14);
+        epilogue(std::true_type{}, acc);
     }
 }
 
