@@ -52,7 +52,7 @@ def main(log_paths: list[str]) -> None:
            "    python3 bench.py --sweep 1,2,3 --sweep-wbits 2 > sweep2.log",
            "    python3 kea-kernels_amd/csrc/gen_tile_table.py sweep1.log sweep2.log", "",
            "Every tile configuration of the library at each (weight bits, parts, N, K, M), fp16 scales and output, "
-           "HIP-graph replay of 100 launches behind a spin, per-launch microseconds. Per row: for each swept M, the "
+           "HIP-graph replay of 100 launches (10 above M = 1000) behind a spin, per-launch microseconds. Per row: for each swept M, the "
            "fastest tile `t<id>` and its time; in brackets the time of the tile that the chooser of the swept build "
            "picked, where that was more than 5% slower. Tile ids: 1-12 and 24 on the LDS-ring tiles, "
            "13-23 the wave-split tiles (`kea_config_name`).", "",

@@ -5,7 +5,7 @@
 // (kk/ternary/fused_kernels.py:163-240) and `_glu_pad` + the depthwise Conv1d of the patched convolution module
 // (kk/ternary/layer_fusions4.py:10-30, :62-72). Arithmetic is IEEE FP32 (fused multiply-adds in the dot products);
 // unlike the reference's online-softmax tiles, a workgroup holds whole score rows (T <= 256), so the softmax is the
-// exact two-pass form. Longer sequences, and callers with a workspace above 128 frames, run kea_attention.hip.
+// exact two-pass form. Longer sequences, and the Python callers above 128 frames, run kea_attention.hip.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -631,7 +631,7 @@ logmel_normalize_kernel(const float2 *spec, int bins, int frames, long long ld_t
 // the same bits. Bands wider than kBand bins are staged kBand bins at a time.
 // Bound by latency: the widest bands (some 8000 bins of 1000 frames) finish last while the rest of the chip waits. A
 // thread loads kLoads bins before it stores their powers (one by one, each load waited for the last), and 512 threads
-// share a band: eight 10-second clips 29.1 -> 27 -> 24.7 us.
+// share a band: eight 10-second clips 29 to 31 -> 27 -> 24.7 us.
 constexpr int kChunk = 512, kBand = 16, kLoads = 8, kFrameThreads = 512;
 __global__ void __launch_bounds__(kFrameThreads)
 logmel_normalize_frames_kernel(const float2 *spec, int bins, int frames, long long ld_f, const float *fb,

@@ -341,7 +341,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64, DEEP ? 2 : 1) gemm_kernel
     // Epilogue operands are fetched before the ring so their latency overlaps the main loads (the copies below are
     // issued after these loads, so the stage waits never depend on them): the raw words, converted after the ring. A
     // conversion here, with its branch on the scale's type, made each of the 4 to 12 loads a memory round trip of its own
-    // before a workgroup's first copy (3200 cycles for a 128x128 tile on 4 waves).
+    // before a workgroup's first copy.
     uint32_t row_raw[RM][P];
     v4u alpha_raw[RN], bias_raw[RN];
     const bool qs_f16 = p.qs_dtype == KEA_F16, ws_f16 = p.ws_dtype == KEA_F16, bias_f16 = p.bias_dtype == KEA_F16;
@@ -487,8 +487,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64, DEEP ? 2 : 1) gemm_kernel
 
     // ---- epilogue: the MFMA result row is the weight row n, the column the activation row m ----
     // The straight epilogue: one copy per output type, residual and SiLU (or GLU), nothing but arithmetic and stores: 5
-    // instructions an output where a block that tests its own bounds and forms 64-bit addresses takes 9. The 16 blocks
-    // of a wave (128x128 tile on 4 waves) took 5800 to 7700 cycles that way, more than its K loop at K = 1024. Epilogue
+    // instructions an output where a block that tests its own bounds and forms 64-bit addresses takes 9. Epilogue
     // and deep tiles together, 16000 x 4096 x 1024 (one part, f16 out): 122 -> 88 us, 16000 x 1024 x 4096 105 -> 66,
     // three parts 5333 x 4096 x 1024 94 -> 77; non-temporal stores made the first 138 us.
     if constexpr (!SLICED && GQ == 0) {

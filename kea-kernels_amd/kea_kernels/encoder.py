@@ -24,8 +24,8 @@ fused HIP kernels of include/kea_encoder.h (the reference's Triton relative_atte
 also applies the SiLU and quantizes for W_pw2 (kea_glu_dwconv_quantize). The four residual projections (W2 of both
 FFs, W_out, W_pw2) add the residual in their GEMM epilogue, in place (the reference's row_fusions,
 kk/ternary/row_fusion.py:121-152); the quantizers run as row kernels between the GEMMs (kea_quantize,
-kea_norm_quantize, kea_attention_merge_quantize), 17 launches a layer. The subsampling convolutions are PyTorch on
-the GPU.
+kea_norm_quantize, kea_attention_merge_quantize), 17 launches a layer. The subsampling is three kernels
+(kea_subsample_stage1, _stage2, _out).
 With fused=False the same model runs with separate quantizers, the residual in the GEMM epilogue
 (kea_lowbit_gemm_residual) and PyTorch attention, GLU and convolution. The quantized linears have no bias
 (Q/K/V must be bias-free to fuse, kk/binary/provider.py:230-244).
