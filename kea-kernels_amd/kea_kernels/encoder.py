@@ -557,6 +557,14 @@ class _SplitSubsampling:
     def holds(self, s: dict) -> bool:
         return all(s[k] is v and v._version == n for k, v, n in self._source)
 
+    def take(self, other: "_SplitSubsampling") -> None:
+        """Becomes `other` in its own buffers, which captured graphs may read."""
+        with torch.inference_mode():  # (either kind of tensor may be written there)
+            for name, v in vars(other).items():
+                if isinstance(v, Tensor):
+                    getattr(self, name).copy_(v)
+        self._source = other._source
+
     @staticmethod
     def prepare(s: dict, cfg: EncoderConfig):
         """The layout, or None where the kernels do not take the model: they are written for 128 mel bins and 256
@@ -722,7 +730,7 @@ class FastConformerEncoder:
         feats = feats.contiguous()
         b, f, t = feats.shape
         if f == 128 and 1 <= t < 1 << 29 and b < 1 << 16 and feats.dtype == torch.float32:
-            split = self._current_split(feats.device)
+            split = self._current_split()
             if split is not None:
                 return self._subsample_split(split, feats)
         t1, f1 = (t - 1) // 2 + 1, (f - 1) // 2 + 1
@@ -750,18 +758,22 @@ class FastConformerEncoder:
                 self._sub_out = out
         return F.linear(flat, *out)
 
-    def _current_split(self, device) -> _SplitSubsampling | None:
-        """The laid-out subsampling weights, made again if a tensor of `self.sub` has changed since (not during a graph
-        capture, where the general kernels run instead)."""
+    def _current_split(self) -> _SplitSubsampling | None:
+        """The laid-out subsampling weights, made again if a tensor of `self.sub` has changed since: in the same buffers,
+        so that captured graphs see them from then on (not during a capture, where the general kernels run instead)."""
         w = self._sub_split
         if w is None or w.holds(self.sub):
             return w
         self._sub_out = None
         if torch.cuda.is_current_stream_capturing():
             return None
-        w = _SplitSubsampling.prepare(self.sub, self.cfg)
-        torch.cuda.current_stream(device).synchronize()  # complete before a call on another stream finds it
-        self._sub_split = w
+        new = _SplitSubsampling.prepare(self.sub, self.cfg)
+        torch.cuda.synchronize(self.device)  # nothing reads the buffers while they change, or before they have changed
+        if new is None:
+            self._sub_split, self._sub_held = None, w  # (graphs captured outside keep reading its buffers)
+            return None
+        w.take(new)
+        torch.cuda.synchronize(self.device)
         return w
 
     def _subsample_split(self, w: _SplitSubsampling, feats: Tensor) -> Tensor:
@@ -938,7 +950,9 @@ class FastConformerEncoder:
 class EncoderGraph:
     """One HIP graph of preprocessing + encoder for a fixed (batch, samples); __call__ copies the audio into the
     graph's input buffer, replays and returns the graph's output buffer (overwritten by the next call). The graph owns
-    its input, its key-split attention workspace (FastConformerEncoder.attention_workspaces) and its output."""
+    its input, its key-split attention workspace (FastConformerEncoder.attention_workspaces) and its output. Changes to
+    the encoder's subsampling weights (encoder.sub) since the last replay are seen, by a new capture (and output buffer)
+    where they move the encoder to its general kernels."""
 
     def __init__(self, encoder: FastConformerEncoder, batch: int, samples: int, *, warmup: int = 2):
         self.encoder = encoder
@@ -946,11 +960,17 @@ class EncoderGraph:
         self.audio = torch.zeros(batch, samples, device=dev)
         self.stream = torch.cuda.Stream(dev)
         self.workspaces: dict = {}
+        self.warmup = warmup
+        self._capture()
+
+    def _capture(self) -> None:
+        encoder, dev = self.encoder, self.audio.device
         with torch.inference_mode(), encoder.attention_workspaces(self.workspaces):
-            encoder.positions(encoded_length(frames_for(encoder.cfg, samples)))
+            encoder.positions(encoded_length(frames_for(encoder.cfg, self.audio.shape[1])))
+            self.split = encoder._current_split()
             self.stream.wait_stream(torch.cuda.current_stream(dev))
             with torch.cuda.stream(self.stream):
-                for _ in range(warmup):
+                for _ in range(self.warmup):
                     encoder(self.audio)
             torch.cuda.synchronize(dev)
             self.graph = torch.cuda.CUDAGraph()
@@ -960,6 +980,8 @@ class EncoderGraph:
 
     def replay(self) -> Tensor:
         """Replays on the graph's stream, ordered after the caller's current stream and before its later work."""
+        if self.encoder._current_split() is not self.split:
+            self._capture()
         caller = torch.cuda.current_stream(self.audio.device)
         self.stream.wait_stream(caller)
         with torch.cuda.stream(self.stream):
@@ -968,6 +990,8 @@ class EncoderGraph:
         return self.out
 
     def __call__(self, audio: Tensor) -> Tensor:
+        if self.encoder._current_split() is not self.split:
+            self._capture()
         caller = torch.cuda.current_stream(self.audio.device)
         self.stream.wait_stream(caller)
         with torch.cuda.stream(self.stream):

@@ -198,6 +198,38 @@ def test_weights_changed_into_what_is_not_taken_and_back():
 
 @pytest.mark.gpu
 @torch.inference_mode()
+def test_graphs_follow_changed_weights():
+    """An EncoderGraph uses the weights of the moment, also where they leave the split kernels; a graph captured by the
+    caller reads the same buffers before and after a change."""
+    enc = model()
+    graph, audio = E.EncoderGraph(enc, 1, 16000), torch.randn(1, 16000, generator=torch.Generator().manual_seed(13)).cuda()
+    feats, own = enc.pre(audio), torch.cuda.CUDAGraph()
+    enc.subsample(feats)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(own):
+        out = enc.subsample(feats)
+    for change in (lambda s: s["conv.3.weight"].mul_(1.5), lambda s: s["out.bias"].add_(1.0),
+                   lambda s: s.update({"conv.6.weight": s["conv.6.weight"].clone().mul_(0.5)})):
+        before = graph(audio).clone()
+        with torch.inference_mode(False):
+            change(enc.sub)
+        after = graph(audio).clone()
+        assert not torch.equal(before, after) and torch.equal(after, enc(audio)) and torch.equal(graph.replay(), after)
+        junk = [torch.full((1 << 20,), 7.0, device="cuda") for _ in range(20)]   # (what was freed meanwhile is overwritten)
+        own.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, enc.subsample(feats))
+        del junk
+    kept = out.clone()
+    enc.sub["conv.0.weight"][5] = 1e-12                                          # the general kernels from here on
+    assert torch.equal(graph(audio), enc(audio)) and enc._sub_split is None
+    own.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, kept)
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
 def test_weights_at_any_address():
     """Weights that are views into one buffer, off the alignment that the kernels' vector loads need."""
     cfg = E.EncoderConfig(layers=1)
