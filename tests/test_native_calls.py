@@ -193,7 +193,7 @@ def test_refused_arguments_raise_as_before():
     for bad, message in [(dict(q=q.float()), "int8"), (dict(qs=qs[:1]), "qs must be"), (dict(words=layer.words[:10]), "native words"),
                          (dict(scale=layer.scale[:9]), "weight scales"), (dict(y=y[:4]), "row-major"), (dict(m=9), "exceeds"),
                          (dict(qs=qs.cpu()), "expected cuda"), (dict(y=None), "nothing to compute"),
-                         (dict(ws_group=96), "ws_group must be"), (dict(residual=y.half()), "residual must be")]:
+                         (dict(ws_group=96, scale=torch.ones(260, 3, device=DEV)), "ws_group must be"), (dict(residual=y.half()), "residual must be")]:
         with pytest.raises(ValueError, match=message):
             gemm(**bad)
     for rows, m in [((0, 272, 1, 9), 9), ((0, 273, 1, 8), 8), ((0, 272, 2, 8), 8), ((0, -1, 1, 8), 8), ((272, 272, 1, 0), 8)]:
