@@ -81,12 +81,12 @@ constexpr int kBandStride = 52;                 // band scores of a query in LDS
 //   planes, in LDS order;  Q: block (b, h, tile): for both biases (u, v) the two planes of four 16-query groups as MFMA
 //   operands [s][lane][8] (lane: query lane % 16, elements 32 s + 8 (lane / 16) .. + 7).
 //   Multipliers 2^(e - 14): km, pm one for four rows, qm [bias][query]; ve: the exponent e of each of the 64 value rows.
-//   top: the bits of the largest magnitude, kt for K, pt for P, qt for Q; kt is an infinity's where the block's value rows
-//   are not to be split.
+//   top: the bits of the largest magnitude, kt for K, pt for P, qt for Q; vt: an infinity's bits where the block's value rows
+//   are not to be split, or zero.
 struct SplitOperands {
     char *q, *k, *v, *p;
     float *qm, *km, *pm;
-    int32_t *ve, *qt, *kt, *pt;
+    int32_t *ve, *qt, *kt, *vt, *pt;
     int tiles, pblocks;  // 64-row tiles of the sequence; blocks of P per head
 };
 constexpr int kQBlockBytes = 2 * kBlockBytes;
@@ -107,14 +107,16 @@ inline long long split_layout(SplitOperands *s, char *ws, long long batch, int h
     take(s->ve, kv * kRows * 4);
     take(s->qt, kv * 4);
     take(s->kt, kv * 4);
+    take(s->vt, kv * 4);
     take(s->pt, np * 4);
     s->tiles = (int)tiles;
     s->pblocks = (int)(2 * tiles);
     return off;
 }
 
-// One workgroup (256 threads) splits one block: blockIdx.x < kv a block of K and V, then kv blocks of Q, then P. Bound by
-// the bytes: 4 read and 4 (Q: 8) written an element.
+// One workgroup (256 threads) splits one block: blockIdx.x < kv a block of V, then kv blocks of Q, kv of K, then P. Bound by
+// the bytes at large sizes (4 read and 4, Q: 8, written an element) and by one block's chain of loads, maxima and stores at
+// small ones: K and V by one workgroup, one after the other, were 0.9 us slower at T = 175, batch 2.
 __global__ void __launch_bounds__(256)
 split_kernel(const float *qkv, long long ld, const float *pos, long long ldp, const float *bias_u, const float *bias_v,
              int T, int H, int kv, SplitOperands so) {
@@ -156,17 +158,22 @@ split_kernel(const float *qkv, long long ld, const float *pos, long long ldp, co
         __syncthreads();
         if (tid == 0) *word = max(max(top[0], top[1]), max(top[2], top[3]));
     };
-    if ((int)blockIdx.x >= 2 * kv) {
-        const int id = blockIdx.x - 2 * kv, h = id / so.pblocks, pb = id - h * so.pblocks;
+    if ((int)blockIdx.x >= 3 * kv) {
+        const int id = blockIdx.x - 3 * kv, h = id / so.pblocks, pb = id - h * so.pblocks;
         rows(pos + (long long)h * kDK, ldp, T - kRows + kRows * (pb + 1 - so.tiles), 2 * T - 1,
              (_Float16 *)(so.p + (long long)id * kBlockBytes), so.pm + (long long)id * 16);
         finish(so.pt + id);
         return;
     }
-    const int id = (int)blockIdx.x < kv ? (int)blockIdx.x : (int)blockIdx.x - kv;
+    const int part = (int)blockIdx.x / kv, id = (int)blockIdx.x - part * kv;
     const int kb = id % so.tiles, bh = id / so.tiles, h = bh % H, b = bh / H, j0 = kb * kRows;
     const float *qbase = qkv + (long long)b * T * ld + (long long)h * kDK;
-    if ((int)blockIdx.x >= kv) {  // queries: wave = 16-query group, a lane per query and quarter of each 32-element step
+    if (part == 2) {
+        rows(qbase + (long long)H * kDK, ld, j0, T, (_Float16 *)(so.k + (long long)id * kBlockBytes), so.km + (long long)id * 16);
+        finish(so.kt + id);
+        return;
+    }
+    if (part == 1) {  // queries: wave = 16-query group, a lane per query and quarter of each 32-element step
         const int i = j0 + 16 * wave + n;
         float x[2][4][8];
         const float *q = qbase + (long long)min(i, T - 1) * ld + 8 * g;
@@ -200,7 +207,7 @@ split_kernel(const float *qkv, long long ld, const float *pos, long long ldp, co
         finish(so.qt + id);
         return;
     }
-    const float *kbase = qbase + (long long)H * kDK, *vbase = kbase + (long long)H * kDK;
+    const float *vbase = qbase + 2LL * H * kDK;
     float v[2][8][2];
 #pragma unroll
     for (int u = 0; u < 2; ++u)
@@ -213,7 +220,6 @@ split_kernel(const float *qkv, long long ld, const float *pos, long long ldp, co
             v[u][e][0] = w.x;
             v[u][e][1] = w.y;
         }
-    rows(kbase, ld, j0, T, (_Float16 *)(so.k + (long long)id * kBlockBytes), so.km + (long long)id * 16);
     // A scale per key: its row may be any size beside the others'. Key index x + 4 y: the exponents are formed in the lanes of
     // row y and the scales read from there (16 of each in scalar instructions took half a microsecond).
     float pair[16], most[4], sf[16];
@@ -251,7 +257,7 @@ split_kernel(const float *qkv, long long ld, const float *pos, long long ldp, co
             *(v8h *)(p + kPlane) = lo;
         }
     }
-    finish(so.kt + id);
+    finish(so.vt + id);
     v8h *dst = (v8h *)(so.v + (long long)id * kBlockBytes);
 #pragma unroll
     for (int u = 0; u < 2 * kPlane / 8 / 256; ++u) dst[u * 256 + tid] = ((const v8h *)vt)[u * 256 + tid];
@@ -318,7 +324,7 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
     const int qtop = so.qt[bh * tiles + iq0];
     int top = 0;
     for (int i = tid; i < tiles; i += kNW * 64)
-        top = max(max(top, so.kt[bh * tiles + i]), max(so.pt[pfirst + i], so.pt[pfirst + i + 1]));
+        top = max(max(max(top, so.kt[bh * tiles + i]), so.vt[bh * tiles + i]), max(so.pt[pfirst + i], so.pt[pfirst + i + 1]));
     const float most = __builtin_bit_cast(float, qtop) * __builtin_bit_cast(float, top) * fabsf(scale * kLog2e);
     const bool wave_plain = __any(max(qtop, top) >= kInfBits || most > kScores) != 0;
     if (lane == 0) plain[wave] = wave_plain;
@@ -357,7 +363,7 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
 #pragma unroll
     for (int w = 0; w < kNW; ++w) any_plain |= plain[w];
     any_plain = __builtin_amdgcn_readfirstlane(any_plain);
-    if (any_plain) {
+    if (__builtin_expect(any_plain, 0)) {
         // The FP32 form, on the FP32 matrix instruction: the same tiles and lanes, operands straight from global memory, the
         // exact two-pass softmax. Element 16 s + 4 g + e of a row is step (s, e) of the contraction.
         const float *qp = qkv + ((long long)b * T + min(iq, T - 1)) * ld + (long long)h * kDK + 4 * g;
@@ -601,7 +607,7 @@ extern "C" int kea_relpos_attention_tiled(const float *qkv, int64_t ld, const fl
     if ((uintptr_t)workspace & 15) return kea::fail(KEA_EALIGN, "attention workspace must be 16-byte aligned");
     SplitOperands so;
     split_layout(&so, (char *)workspace, batch, heads, t);
-    const int64_t kv = batch * heads * so.tiles, blocks = 2 * kv + (int64_t)heads * so.pblocks;
+    const int64_t kv = batch * heads * so.tiles, blocks = 3 * kv + (int64_t)heads * so.pblocks;
     if (!kea::fits_dispatch(blocks, 256)) return kea::fail(KEA_EINVAL, "too large for one launch: split the batch");
     hipError_t e = hipFuncSetAttribute((const void *)relpos_tiled_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kTiledLds);
     if (e != hipSuccess) return kea::fail((int)e, std::string("LDS attribute refused: ") + hipGetErrorString(e));
