@@ -8,7 +8,7 @@
 // row. Against FP64 the result is closer than the FP32 forms (fewer roundings of the accumulator). Where the inputs hold an
 // infinity, or rows whose elements differ so much in size that the pairs would lose what FP32 keeps (kScores, kLowPairs), a
 // workgroup takes an FP32 form on the FP32 matrix instruction instead (NaNs propagate by themselves). That form reads its
-// operands from global memory and computes the scores twice: T = 200 batch 8 130 us, T = 750 batch 2 371.
+// operands from global memory and computes the scores twice: T = 200 batch 8 130 us, T = 750 batch 2 370.
 //
 // Two launches. split_kernel writes K, V and P once as hi / lo planes in the order the LDS of the second kernel holds
 // them, 64 rows to a block; relpos_tiled_kernel then copies blocks straight to LDS (global_load_lds) and spends no
@@ -31,9 +31,9 @@
 // counters) the MFMAs of a SIMD's two waves take 13, their vector instructions 12 and the CU's LDS 12, and the waves wait
 // for 48% of their time. Measured on MI355X, graph-timed, both launches, against what served these
 // lengths before (T <= 256 an FP32 vector kernel, above it PyTorch operators on [T, 2T] score matrices): T = 200 batch 8
-// 31 / 173 us, T = 250 batch 1 25 / 28, T = 375 batch 2 34 / 145, T = 750 batch 2 52 / 284, T = 750 batch 8 153 / 890. Up to
+// 32 / 173 us, T = 250 batch 1 24 / 28, T = 375 batch 2 33 / 146, T = 750 batch 2 52 / 285, T = 750 batch 8 154 / 890. Up to
 // 128 frames the FP32 matrix-core kernels of kea_encoder.hip, one pass without a workspace, are the faster ones: T = 125
-// batch 8 19 against 24 us, batch 1 11 against 18; at T = 129 batch 1 it is 20 against 21.
+// batch 8 19 against 24 us, batch 1 11 against 17; at T = 129 batch 1 it is 20 against 20.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

@@ -294,7 +294,7 @@ def relpos_attention(qkv: Tensor, pos: Tensor, bias_u: Tensor, bias_v: Tensor, h
     args = (qkv.data_ptr(), qkv.stride(1), pos.data_ptr(), pos.stride(0), bias_u.data_ptr(), bias_v.data_ptr(),
             _hip.ptr(out), d, b, t, heads, d // heads, 1.0 / math.sqrt(d // heads))
     if workspace is None and 128 < t <= 256:
-        # the tiled kernel (batch 8, T = 200: 33 us against 181); up to 128 frames the FP32 kernels are faster
+        # the tiled kernel (batch 8, T = 200: 32 us against 173); up to 128 frames the FP32 kernels are faster
         return _attention_tiled(args, out)
     if workspace is None:
         rc = _hip.lib().kea_relpos_attention(*args, _hip.stream_handle(qkv.device))
