@@ -511,11 +511,12 @@ relpos_tiled_kernel(const float *qkv, long long ld, const float *pos, long long 
                 w[e] = __builtin_amdgcn_ldexpf(p[e], ek[e] - em + kProbExp);
             }
             if (__any(max_abs<8>(w) >= (float)(2 << (kLazy + kProbExp)))) {
-                int size = INT32_MIN;  // the largest contribution's exponent
+                // the largest contribution's exponent (a probability of zero has none, however large its value row is)
+                int size = -3000000;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) size = max(size, (int)(__builtin_bit_cast(uint32_t, p[e]) >> 23) + ek[e]);
+                for (int e = 0; e < 8; ++e) size = max(size, p[e] > 0.f ? __builtin_amdgcn_frexp_expf(p[e]) + ek[e] : size);
                 size = max(size, __shfl_xor(size, 16, 64));
-                size = max(size, __shfl_xor(size, 32, 64)) - 127;
+                size = max(size, __shfl_xor(size, 32, 64)) - 1;
                 const int en = size > em + kLazy ? size : em;
                 const float f = pow2(max(em - en, -127));
                 em = en;

@@ -94,6 +94,22 @@ def test_large_values_under_a_suppressed_key(key, power, score):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("key", [0, 69, 199])
+@pytest.mark.parametrize("small,large", [(-60, 90), (-100, 120), (-20, 127)])
+def test_large_values_under_a_key_without_probability(key, small, large):
+    """A key whose probability is zero in FP32 (2^-288) and whose value row is 2^147 to 2^220 times the others': it adds
+    nothing to any output, whatever its exponent, so the bar is that of a suppressed key."""
+    qkv, pos, u, v = _inputs(1, 200, 18)
+    q, k = qkv[..., :D].view(1, 200, H, DK), qkv[..., D:2 * D].view(1, 200, H, DK)
+    q[..., 0], k[..., 0], u[:, 0] = 4.0, 0.0, 0.0
+    k[:, key] = 0.0
+    k[:, key, :, 0] = -200 * math.sqrt(DK) / 4.0
+    qkv[..., 2 * D:] *= 2.0 ** small
+    qkv[:, key, 2 * D:] = torch.sign(qkv[:, key, 2 * D:]) * 2.0 ** large
+    assert _row_error(_tiled(*(a.cuda() for a in (qkv, pos, u, v))), _reference(qkv, pos, u, v)) < 2e-6
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("power", [9, 11, 13, 15, 20, 60])
 @pytest.mark.parametrize("operand", ["k_row", "k_dim", "q_row", "q_dim", "p_row", "p_dim", "v_element", "v_half"])
 def test_rows_and_elements_of_any_size(operand, power):
