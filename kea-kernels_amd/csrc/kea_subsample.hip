@@ -119,6 +119,7 @@ __device__ __forceinline__ void pointwise_fp32(const float *tile, const float *w
 
 // Kernel 1: a workgroup = one clip's output rows t2 = 2 blockIdx.x and + 1, all 32 columns and 256 channels.
 constexpr int kMinExponent = -50, kHalfOne = 0x3c00;  // (FP16 bits of 1, 2^-14 of the scale's lower end)
+constexpr float kLeastTap = 0x1p-102f;               // (2^24 times the smallest normal number)
 constexpr int kRows2 = 2, kPos1 = kRows2 * kF2;              // positions of a tile: 64, m = 32 q + f2
 constexpr int kRows1 = 2 * kRows2 + 1, kPatchR = 2 * kRows1 + 1, kPatchC = kF + 2;
 constexpr int kPatch = kPatchR * kPatchC;                    // input rows 4 t2 - 3 .., columns -1 .. 128
@@ -165,11 +166,11 @@ subsample1_kernel(const float *x, int T, int T1, int T2, const _Float16 *w1f, co
     int bits = top[0];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) bits = max(bits, top[w]);
-    // a tile of zeros has the smallest scale; one of smaller values than that is summed in FP32, as NaNs and infinities are,
-    // and as one is where the scale of its largest value costs others their accuracy: a value that both planes lose (below
-    // 2^-39 of it), or a window of 3x3 inputs without one above 2^-14 of it (held to 2^-25 of the window's largest from there
-    // on). The output rows of a tile do not all see that largest value.
-    const int xe = max(exponent_of(bits), kMinExponent);
+    // a tile of values below the smallest scale is summed in FP32, as NaNs and infinities are, and as one is where the scale
+    // of its largest value costs others their accuracy: a value that both planes lose (below 2^-39 of it), or a window of 3x3
+    // inputs without one above 2^-14 of it (held to 2^-25 of the window's largest from there on). The output rows of a tile do
+    // not all see that largest value.
+    const int xe = bits == 0 ? 0 : max(exponent_of(bits), kMinExponent);
     plain = plain || bits >= kInfBits || (bits != 0 && exponent_of(bits) < kMinExponent);
 #pragma unroll
     for (int u = 0; u < PN; ++u) {
@@ -219,8 +220,16 @@ subsample1_kernel(const float *x, int T, int T1, int T2, const _Float16 *w1f, co
         dw[0][k] = taps[k].x * mul[0];
         dw[1][k] = taps[k].y * mul[1];
     }
+    // (weights that these units make too small for 24 bits: FP32 as well)
+    float tap[2] = {kea::max_abs2(taps[8].x, 0.f, 0.f), kea::max_abs2(taps[8].y, 0.f, 0.f)};
+#pragma unroll
+    for (int k = 0; k < 8; k += 2) {
+        tap[0] = kea::max_abs2(taps[k].x, taps[k + 1].x, tap[0]);
+        tap[1] = kea::max_abs2(taps[k].y, taps[k + 1].y, tap[1]);
+    }
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
+        plain = plain || (tap[e] > 0.f && tap[e] * mul[e] < kLeastTap);
         bias1[e] = (e ? first.y : first.x) * __builtin_amdgcn_rcpf(e ? m1.y : m1.x) * pow2(14 - xe);  // (m1: powers of two)
 #pragma unroll
         for (int q = 0; q < kRows2; ++q)

@@ -280,6 +280,24 @@ def test_scales_whose_product_leaves_the_range():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("size", [0.0, 2.0**-48, 2.0**-20, 1.0])
+@torch.inference_mode()
+def test_small_weights_of_both_first_convolutions(size):
+    """Ordinary biases through a depthwise convolution of small weights, where the first convolution's are small too: the
+    units that the first kernel holds them in leave the product what it is, whatever the features."""
+    enc = model()
+    for key, power in [("conv.0.weight", -26), ("conv.2.weight", -34), ("conv.3.weight", 36)]:
+        enc.sub[key].mul_(2.0**power)
+    enc.sub["conv.2.bias"].zero_()
+    enc.sub["conv.0.bias"].abs_().add_(0.25)
+    assert enc._current_split() is not None
+    feats = torch.randn(2, 128, 40, generator=torch.Generator().manual_seed(14)).cuda() * size
+    want, got, old = exact(enc, feats), enc.subsample(feats).double().cpu(), general(enc, feats).double().cpu()
+    print(size, _row_error(got, want), _row_error(old, want))
+    assert _row_error(got, want) <= 2 * _row_error(old, want)
+
+
+@pytest.mark.gpu
 @torch.inference_mode()
 def test_a_large_weight_of_a_dead_channel():
     """A weight 2^24 times the others of its row for an input that is always zero: what the others give is as accurate as
