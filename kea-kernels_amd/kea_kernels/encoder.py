@@ -569,10 +569,11 @@ class _SplitSubsampling:
     def prepare(s: dict, cfg: EncoderConfig):
         """The layout, or None where the kernels do not take the model: they are written for 128 mel bins and 256
         channels (and an output in tiles of 128), a weight that is not finite has no split form (2^80 leaves the scaled sums
-        in range), and the first convolution's sums, its bias among them, are held in units of its weights and of the input
-        (nonzero rows from 2^-30, biases to 2^15, both layers' weights to 2^13, so that these units and what multiplies them
-        stay finite for any scale of the input). Weights, or channels by their weights, too far apart in size for the scale
-        that they share are left to FP32 as well (_narrow_rows). Waits for the GPU once."""
+        in range; rows are held in full from 2^-90, so a layer's largest is at least 2^-66), and the first convolution's sums,
+        its bias among them, are held in units of its weights and of the input (nonzero rows from 2^-30, biases to 2^15, both
+        layers' weights to 2^13, so that these units and what multiplies them stay finite for any scale of the input).
+        Weights, or channels by their weights, too far apart in size for the scale that they share are left to FP32 as well
+        (_narrow_rows). Waits for the GPU once."""
         if cfg.feat_in != 128 or cfg.sub_channels != 256 or s["out.weight"].shape[1] != 16 * 256 or cfg.d_model % 128:
             return None
         if any(v.is_inference() for v in s.values()):  # (a tensor that does not count its changes)
@@ -583,6 +584,8 @@ class _SplitSubsampling:
                 & (s["conv.0.bias"].abs() <= 2**15).all() & (row <= 2**13).all() & (s["conv.2.weight"].abs() <= 2**13).all())
         for name in ("conv.0.weight", "conv.3.weight", "conv.6.weight", "out.weight"):
             fits &= _narrow_rows(s[name].reshape(s[name].shape[0], -1))
+            top = tops[list(s).index(name)]
+            fits &= (top == 0) | (top >= 2.0**-66)
         fits &= _narrow_rows(_channel_sizes(s))
         if not fits.item():
             return None

@@ -298,6 +298,22 @@ def test_small_weights_of_both_first_convolutions(size):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("small,large", [("conv.3", "conv.5"), ("conv.6", "out")])
+@torch.inference_mode()
+def test_a_layer_of_weights_below_the_split_form(small, large):
+    """Weights that a split row's scale does not reach, made up for by the next layer's."""
+    enc = model()
+    enc.sub[small + ".weight"].mul_(2.0**-108)
+    for layer in (small, "conv.5", "conv.6", "out"):
+        enc.sub[layer + ".bias"].zero_()
+    enc.sub[large + ".weight"].mul_(2.0**76)
+    feats = torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(15)).cuda() * 2.0**12
+    want, got, old = exact(enc, feats), enc.subsample(feats).double().cpu(), general(enc, feats).double().cpu()
+    print(_row_error(got, want), _row_error(old, want))
+    assert _row_error(got, want) <= 2 * _row_error(old, want)
+
+
+@pytest.mark.gpu
 @torch.inference_mode()
 def test_a_large_weight_of_a_dead_channel():
     """A weight 2^24 times the others of its row for an input that is always zero: what the others give is as accurate as
