@@ -523,13 +523,13 @@ class _SplitSubsampling:
     convolutions as split FP16 fragments, the first convolution's nine taps as the 27 terms (hi, hi, lo against the
     input's hi, lo, hi) of one 32-deep product with channels 32 w + 2 i + e in fragment 2 w + e, and the output
     linear's columns in (frequency, channel) order. `holds` tells whether they still are what the tensors they were made
-    from hold (by identity and version: an in-place change through `.data` is the one that it does not see)."""
+    from hold (by identity, version and memory: an in-place change through `.data` is the one that it does not see)."""
 
     LEAST = -30  # the exponent below which a row of the first convolution is not split (unless it is zero)
 
     def __init__(self, s: dict, gain: float):
         c = 256
-        self._source = [(k, v, v._version) for k, v in s.items()]
+        self._source = [(k, v, v._version, v.detach()) for k, v in s.items()]  # (detach(): its memory stays taken)
 
         def taps(name):
             return s[name].reshape(c, 9).t().clone(memory_format=torch.contiguous_format)
@@ -555,7 +555,7 @@ class _SplitSubsampling:
         self.fo = _fragments([hi, lo])
 
     def holds(self, s: dict) -> bool:
-        return all(s[k] is v and v._version == n for k, v, n in self._source)
+        return all(s[k] is v and v._version == n and v.data_ptr() == memory.data_ptr() for k, v, n, memory in self._source)
 
     def take(self, other: "_SplitSubsampling") -> None:
         """Becomes `other` in its own buffers, which captured graphs may read."""

@@ -184,6 +184,18 @@ def test_changed_weights_are_seen(key, how, inference):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("key", ["conv.0.weight", "conv.3.weight", "conv.5.bias", "out.weight"])
+def test_assigned_data_is_seen(key):
+    """`tensor.data = other` leaves the tensor and its count of changes what they were."""
+    enc, feats = model(), torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(16)).cuda()
+    enc.subsample(feats)
+    for factor in (1.5, 0.5):                  # (the second may get the memory of the first)
+        enc.sub[key].data = enc.sub[key].detach() * factor
+        got, want = enc.subsample(feats).double().cpu(), exact(enc, feats)
+        assert float((got - want).abs().max() / want.abs().max()) < 1e-5
+
+
+@pytest.mark.gpu
 @torch.inference_mode()
 def test_weights_changed_into_what_is_not_taken_and_back():
     enc, feats = model(), torch.randn(1, 128, 40, generator=torch.Generator().manual_seed(7)).cuda()
