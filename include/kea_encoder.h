@@ -138,9 +138,9 @@ int kea_bias_relu_flatten(const float *x_dev, const float *bias_dev, float *y_de
  * [16][64][8], fragment 2 w + e, lane 16 g + i, element j = term 8 g + j of channel 32 w + 2 i + e, where terms 0-8 and
  * 9-17 are hi, 18-26 lo, 27-31 zero; w3f, w6f [16][8][2][64][8], n-tile, k-step, plane, lane 16 g + i, element j =
  * row 16 tile + i, column 32 step + 8 g + j. Weights are finite, nonzero rows of
- * w1 at least 2^-30, |w1| and |w2| <= 2^13, the others <= 2^80, |b1| <= 2^15, and m1 no less than 2^-44; inputs may be
- * anything (a NaN is zero after a ReLU; a tile of inputs too far apart in size for one scale is summed in FP32). Every
- * pointer but w1, w3, w6, w, ys, xs and stage 1's x is 16-byte aligned. batch <= 65535. */
+ * w1 at least 2^-30, |w1| and |w2| <= 2^13, the others <= 2^80 (rows are held in full from 2^-90), |b1| <= 2^15, and m1
+ * no less than 2^-44; inputs may be anything (a NaN is zero after a ReLU; a tile of inputs too far apart in size for one
+ * scale is summed in FP32). Every pointer but w1, w3, w6, w, ys, xs and stage 1's x is 16-byte aligned. batch <= 65535. */
 int kea_subsample_stage1(const float *x_dev, int64_t batch, int64_t t, const void *w1f_dev, const float *m1_dev,
                          const float *w1_dev, const float *b1_dev, const float *w2_dev, const float *b2_dev,
                          const void *w3f_dev, const float *m3_dev, const float *w3_dev, const float *b3_dev, float *y_dev,

@@ -31,7 +31,7 @@
 // counters) the MFMAs of a SIMD's two waves take 13, their vector instructions 12 and the CU's LDS 12, and the waves wait
 // for 48% of their time. Measured on MI355X, graph-timed, both launches, against what served these
 // lengths before (T <= 256 an FP32 vector kernel, above it PyTorch operators on [T, 2T] score matrices): T = 200 batch 8
-// 32 / 173 us, T = 250 batch 1 24 / 28, T = 375 batch 2 33 / 146, T = 750 batch 2 52 / 285, T = 750 batch 8 154 / 890. Up to
+// 32 / 173 us, T = 250 batch 1 24 / 28, T = 375 batch 2 33 / 146, T = 750 batch 2 51 / 285, T = 750 batch 8 154 / 890. Up to
 // 128 frames the FP32 matrix-core kernels of kea_encoder.hip, one pass without a workspace, are the faster ones: T = 125
 // batch 8 19 against 24 us, batch 1 11 against 17; at T = 129 batch 1 it is 20 against 20.
 #include <hip/hip_runtime.h>

@@ -14,7 +14,7 @@
 //
 // Measured on eight 10-second clips (T = 1000): 50 + 26 + 34 us, where five launches and a library GEMM take 53 + 90 +
 // 25 + 27 + 25 + 70 us; one clip 15 + 15 + 17 us.
-// Kernel 1 executes 1830 vector instructions and 232 MFMAs a wave, which at 2.4 GHz take 24 and 12 us of its 50 and hardly
+// Kernel 1 executes 1845 vector instructions and 232 MFMAs a wave, which at 2.4 GHz take 25 and 12 us of its 50 and hardly
 // overlap; LDS takes 11, and the waves wait for 38% of their time. Two rows of 32 positions to a workgroup, two workgroups to
 // a CU, is the split that measured best: four rows (one workgroup to a CU, half the weight reads) take 60 and, for one
 // clip, 25 us. Kernel 2 is latency: the weights (256 KB a workgroup) and its input from L2; half the rows to a workgroup

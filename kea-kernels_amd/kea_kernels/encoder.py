@@ -273,7 +273,9 @@ def attention_workspace(batch: int, t: int, heads: int, device) -> Tensor | None
 def relpos_attention(qkv: Tensor, pos: Tensor, bias_u: Tensor, bias_v: Tensor, heads: int, *,
                      workspace: Tensor | None = None, merged: bool = True) -> Tensor | None:
     """qkv [B, T, 3d] (rows contiguous), pos [2T-1, d] (W_pos of the relative encodings), biases [H, dk] ->
-    attention output [B, T, d] (kea_relpos_attention). With `workspace` (from attention_workspace) small grids split
+    attention output [B, T, d] (kea_relpos_attention, and from 129 to 256 frames without a workspace
+    kea_relpos_attention_tiled: operands held as pairs of FP16 values, an output row as accurate for its size as in FP32 on
+    inputs of ordinary sizes, FP32 itself on others). With `workspace` (from attention_workspace) small grids split
     the keys over two workgroups (kea_relpos_attention_ws); merged=False then leaves the two halves in the workspace
     for attention_merge_quantize and returns None."""
     b, t, three_d = qkv.shape
